@@ -278,7 +278,7 @@ struct qcxms_batch {
     std::vector<int> elem;
     std::vector<int2> items;  // shell-pair work items of all systems
     int natoms = 0, nshells = 0, nrefs = 0, nxtot = 0;
-    size_t mat_total = 0, gam_total = 0, d4_total = 0, hist_total = 0, pair_total = 0;
+    size_t mat_total = 0, gam_total = 0, hist_total = 0, pair_total = 0;
     int max_ld = 0, max_m = 0;
     SccOpts opts{1e-9, 1e-8, 0.4, 1e-11, 100, 100, 0, 0, 0, 0};
     int warm_start = 0;
@@ -346,7 +346,7 @@ int layout(qcxms_batch* b, int nsys, const int32_t* offsets, const int32_t* num,
 {
     b->nsys = nsys;
     b->info.resize(nsys);
-    long long mat = 0, gam = 0, d4 = 0, hist = 0, pair = 0;
+    long long mat = 0, gam = 0, hist = 0, pair = 0;
     int at = 0, shl = 0, ref = 0, xo = 0;
     const int mem = b->opts.mem;
     for (int s = 0; s < nsys; ++s) {
@@ -383,7 +383,6 @@ int layout(qcxms_batch* b, int nsys, const int32_t* offsets, const int32_t* num,
         si.x_off = xo;
         si.mat_off = mat;
         si.gam_off = gam;
-        si.d4_off = d4;
         si.hist_off = hist;
         si.pair_off = pair;
         // shell-pair work items: off-atom pairs (atom of ia > atom of ib)
@@ -431,7 +430,6 @@ int layout(qcxms_batch* b, int nsys, const int32_t* offsets, const int32_t* num,
         xo += si.nx;
         mat += (long long)si.ld * si.ld;
         gam += (long long)nsh * nsh;
-        d4 += (long long)nd * nd;
         hist += 2LL * mem * si.nx + 2LL * mem * mem + 2LL * mem + 2LL * si.nx + 8;
         pair += (long long)nat * nat * qx::kPairStride;
         b->max_ld = std::max(b->max_ld, si.ld);
@@ -443,7 +441,6 @@ int layout(qcxms_batch* b, int nsys, const int32_t* offsets, const int32_t* num,
     b->nxtot = xo;
     b->mat_total = mat;
     b->gam_total = gam;
-    b->d4_total = d4;
     b->hist_total = hist;
     b->pair_total = pair;
     return QCXMS_OK;
@@ -487,7 +484,6 @@ int allocate(qcxms_batch* b)
     ALLOC(d.U, mt);
     ALLOC(d.E, mt);
     ALLOC(d.gam, b->gam_total);
-    ALLOC(d.wd4, b->d4_total);
     ALLOC(d.x, b->nxtot);
     ALLOC(d.xo, b->nxtot);
     ALLOC(d.vs, ns);
@@ -498,7 +494,7 @@ int allocate(qcxms_batch* b)
     ALLOC(d.hist, b->hist_total);
     ALLOC(d.pairbuf, b->pair_total);
     ALLOC(d.spbuf, 5 * b->gam_total);
-    ALLOC(d.aesg, b->pair_total / QX_PAIR_STRIDE * QX_AES_COMP);
+    ALLOC(d.pairk, b->pair_total / QX_PAIR_STRIDE * QX_PAIR_KERN);
     ALLOC(d.xprev, b->nxtot);
     ALLOC(d.xprev2, b->nxtot);
     ALLOC(d.xprev3, b->nxtot);
@@ -584,20 +580,36 @@ size_t lds_setup_bytes(const qcxms_batch* b)
     const size_t ls = std::min(b->max_ld, QX_LDS_MAXM);
     return sizeof(double) * (ls * ls + ls * (ls | 1));
 }
-// four m x m working matrices and the AO row sums for the systems that keep
-// them in LDS
+// Dynamic LDS of an SCC launch.  Systems with their matrices in LDS: four
+// m x m working matrices and the AO row sums, a fifth matrix for the MFMA
+// eigen refinement when it is on and the LDS holds it.  The others: the
+// Jacobi blocks where the LDS holds them.  All: the scratch of the potentials
+// (in two of the matrices where they hold it) and the system of the Broyden
+// weights up to kBroydenLds secant pairs.
 size_t lds_scc_bytes_range(const qcxms_batch* b, int s0, int s1, int lds_max_m, int eig)
 {
-    size_t lm = 0;
+    constexpr size_t kBroydenLds = 40;
+    size_t need = 0, lm = 0;
     for (int s = s0; s < s1; ++s) {
-        const size_t m = (size_t)((b->info[s].nao + 1) & ~1);
-        if (m <= (size_t)lds_max_m) lm = std::max(lm, m);
+        const SysInfo& si = b->info[s];
+        const size_t m = (size_t)((si.nao + 1) & ~1);
+        const size_t pot = qx::pot_lds(si.nat, si.ndim), broy = (kBroydenLds + 1) * (kBroydenLds + 1);
+        if (m <= (size_t)lds_max_m) {
+            const size_t mm = m * (m + 1);
+            lm = std::max(lm, m);
+            need = std::max(need, mm + broy);
+            if (pot > 2 * mm) need = std::max(need, 4 * mm + qx::kRs * m + pot);
+        } else {
+            const size_t blk = m * (m + 2) / 2;
+            if (blk * sizeof(double) <= g_scc_dyn_max) need = std::max(need, blk);
+            need = std::max(need, std::max(pot, broy));
+        }
     }
-    const size_t base = sizeof(double) * (4 * lm * (lm + 1) + qx::kRs * lm);
-    // a fifth matrix for the MFMA eigen refinement when it is on and the LDS
-    // holds it
-    const size_t ext = base + sizeof(double) * lm * (lm + 1);
-    return eig && ext <= g_eig_dyn_max ? ext : base;
+    const size_t mm = lm * (lm + 1), base = 4 * mm + qx::kRs * lm;
+    const size_t ext = base + mm;
+    need = std::max(need, base);
+    if (eig && ext * sizeof(double) <= g_eig_dyn_max) need = std::max(need, ext);
+    return sizeof(double) * std::min(need, g_scc_dyn_max / sizeof(double));
 }
 
 size_t lds_scc_bytes(const qcxms_batch* b)
@@ -647,7 +659,7 @@ int enqueue_scc_plan(qcxms_batch* b)
         o.lds_max_m = lmax;
         o.first_sys = r.s0;
         hipLaunchKernelGGL(t.eig ? qx::k_scc<true> : qx::k_scc<false>, dim3(r.s1 - r.s0), dim3(QX_SCC_BLOCK),
-                           lds, st, b->d, o);
+                           lds, st, qx::SccArgs{b->d, o});
         return hipGetLastError();
     };
     if (runs.size() == 1) {
@@ -692,7 +704,7 @@ int enqueue_egrad(qcxms_batch* b, bool with_grad)
              if (!b->tune.empty()) plan_st = enqueue_scc_plan(b);
              else
                  hipLaunchKernelGGL(b->opts.eig_mfma ? qx::k_scc<true> : qx::k_scc<false>, dim3(b->nsys),
-                                    dim3(QX_SCC_BLOCK), l2, b->stream, b->d, launch_opts(b, l2));
+                                    dim3(QX_SCC_BLOCK), l2, b->stream, qx::SccArgs{b->d, launch_opts(b, l2)});
          })))
         return st;
     if (plan_st) return plan_st;
@@ -776,12 +788,14 @@ int enqueue_md_step(qcxms_md* md)
     qcxms_batch* b = md->b;
     int st;
     if ((st = timed(b, b->t_md_pre, [&] {
-             hipLaunchKernelGGL(qx::k_md_pre, dim3(md->ntraj), dim3(64), 0, b->stream, b->d, md->m, md->p);
+             hipLaunchKernelGGL(qx::k_md_pre, dim3(md->ntraj), dim3(64), 0, b->stream,
+                                qx::MdArgs{b->d, md->m, md->p, b->opts, 1});
          })))
         return st;
     if ((st = enqueue_egrad(b, true))) return st;
     return timed(b, b->t_md_post, [&] {
-        hipLaunchKernelGGL(qx::k_md_post, dim3(md->ntraj), dim3(QX_BLOCK), 0, b->stream, b->d, md->m, md->p);
+        hipLaunchKernelGGL(qx::k_md_post, dim3(md->ntraj), dim3(QX_BLOCK), 0, b->stream,
+                           qx::MdArgs{b->d, md->m, md->p, b->opts, 1});
     });
 }
 
@@ -1594,7 +1608,8 @@ int md_enqueue_fused(qcxms_md* md, int nsteps)
     const size_t lds = std::max(lds_setup_bytes(b), lds_scc_bytes(b));
     return timed(b, b->t_fused, [&] {
         hipLaunchKernelGGL(b->opts.eig_mfma ? qx::k_md_fused<true> : qx::k_md_fused<false>, dim3(md->ntraj),
-                           dim3(QX_SCC_BLOCK), lds, b->stream, b->d, md->m, md->p, launch_opts(b, lds), nsteps);
+                           dim3(QX_SCC_BLOCK), lds, b->stream,
+                           qx::MdArgs{b->d, md->m, md->p, launch_opts(b, lds), nsteps});
     });
 }
 

@@ -141,10 +141,10 @@ struct GradLds {
 };
 
 template <bool STORED = false>
-QX_DEV void grad_system(const BatchPtrs& B, int sys, GradLds& Lg)
+QX_DEV void grad_system(BatchRef B, int sys, GradLds& Lg)
 {
-    const SysInfo si = B.info[sys];
-    const int tid = threadIdx.x, nat = si.nat, nsh = si.nsh, ld = si.ld;
+    const SysInfo si = qx_info(B, sys);
+    const int tid = qx_tid(), nat = si.nat, nsh = si.nsh, ld = si.ld;
     SysShared& ss = Lg.ss;
     double* dedcn = Lg.dedcn;
     double* dedcn4 = Lg.dedcn4;
@@ -525,8 +525,8 @@ __global__ __launch_bounds__(QX_BLOCK) void k_grad(BatchPtrs B)
     const int sys = blockIdx.x;
     if (B.active && !B.active[sys]) return;
     __shared__ GradLds Lg;
-    if (B.dblk) grad_system<true>(B, sys, Lg);
-    else grad_system<false>(B, sys, Lg);
+    if (B.dblk) grad_system<true>(qx_args(B), sys, Lg);
+    else grad_system<false>(qx_args(B), sys, Lg);
 }
 
 }  // namespace qx

@@ -63,6 +63,9 @@ struct MdPtrs {
     double* store;   // CID mode: the averaged structure (store_avxyz), 3 per atom
 };
 
+typedef QX_ARG(MdPtrs) MdRef;
+typedef QX_ARG(MdParams) MdParamRef;
+
 constexpr double kMsToAu = 1.0 / 2.18769126364e+06;  // m/s in au (xtb_mctc_convert.f90:63)
 constexpr int kCntSteps = 50;                        // md.f90 cnt_steps
 
@@ -418,10 +421,10 @@ struct MdLds {
 // thread then updates its coordinates of the sums (avxyz2) and the average
 // (store_avxyz).  Called by all threads of the block after the connectivity
 // (list) of this step.
-QX_DEV void md_cid_average(const BatchPtrs& B, const MdPtrs& M, int sys, int nfrag, MdLds& Lm)
+QX_DEV void md_cid_average(BatchRef B, MdRef M, int sys, int nfrag, MdLds& Lm)
 {
     enum { kZero = 1, kAdd = 2, kDrop = 4, kFinal = 8 };
-    const SysInfo si = B.info[sys];
+    const SysInfo si = qx_info(B, sys);
     const int nat = si.nat, off = si.atom_off;
     MdTraj& t = M.traj[sys];
     if (threadIdx.x == 0) {
@@ -491,11 +494,11 @@ QX_DEV void md_cid_average(const BatchPtrs& B, const MdPtrs& M, int sys, int nfr
 // one MD loop iteration up to the force call (md.f90:285-395): time,
 // averages, drift and SCF checks, running sums, leap-frog.  Any block size
 // from 64 threads; lanes from 64 on take no atoms.
-QX_DEV void md_pre_system(const BatchPtrs& B, const MdPtrs& M, const MdParams& p, int sys, MdLds& Lm)
+QX_DEV void md_pre_system(BatchRef B, MdRef M, MdParamRef p, int sys, MdLds& Lm)
 {
-    if (!M.active[sys]) return;
-    const SysInfo si = B.info[sys];
-    const int lane = threadIdx.x, nat = si.nat, off = si.atom_off;
+    if (!qx_uniform(M.active[sys])) return;
+    const SysInfo si = qx_info(B, sys);
+    const int lane = qx_tid(), nat = si.nat, off = si.atom_off;
     MdTraj& t = M.traj[sys];
     double* term = Lm.term;
     int& s_exit = Lm.s_exit;
@@ -534,7 +537,7 @@ QX_DEV void md_pre_system(const BatchPtrs& B, const MdPtrs& M, const MdParams& p
     __syncthreads();
     // the flag is cleared only after every wavefront has passed the entry
     // test above, so that all of them take the same barriers
-    if (s_exit) {
+    if (qx_uniform(s_exit)) {
         if (lane == 0) M.active[sys] = 0;
         return;
     }
@@ -561,11 +564,11 @@ QX_DEV void md_pre_system(const BatchPtrs& B, const MdPtrs& M, const MdParams& p
 // the rest of the iteration after the force call (md.f90:396-682): checkqc,
 // heating, connectivity, fragment temperatures, electronic temperature,
 // exits.  Any block size from 64 threads.
-QX_DEV void md_post_system(const BatchPtrs& B, const MdPtrs& M, const MdParams& p, int sys, MdLds& Lm)
+QX_DEV void md_post_system(BatchRef B, MdRef M, MdParamRef p, int sys, MdLds& Lm)
 {
-    if (!M.active[sys]) return;
-    const SysInfo si = B.info[sys];
-    const int lane = threadIdx.x, nat = si.nat, off = si.atom_off;
+    if (!qx_uniform(M.active[sys])) return;
+    const SysInfo si = qx_info(B, sys);
+    const int lane = qx_tid(), nat = si.nat, off = si.atom_off;
     MdTraj& t = M.traj[sys];
     unsigned long long* adj = Lm.adj;
     int& s_more = Lm.s_more;
@@ -581,7 +584,7 @@ QX_DEV void md_post_system(const BatchPtrs& B, const MdPtrs& M, const MdParams& 
     }
     __syncthreads();
     // heating: impactscale (impact.f90:12-55) with ff = fadd * nstep
-    if (s_more) {
+    if (qx_uniform(s_more)) {
         const int k = dev_impactscale(nat, M.velo + 3 * (size_t)off, M.mass + off, M.velof + off,
                                       t.eimp, t.fadd * t.nstep, t.ekinstart, Lm.atoms);
         if (k >= 20000) {
@@ -598,7 +601,7 @@ QX_DEV void md_post_system(const BatchPtrs& B, const MdPtrs& M, const MdParams& 
     const int nfrag = dev_fragments(nat, M.num + off, B.xyz + 3 * (size_t)off, M.mass + off,
                                     M.list + off, fragm, adj);
     // t.cid does not change during a run: the test is uniform over the block
-    if (t.cid && nfrag <= 6) md_cid_average(B, M, sys, nfrag, Lm);
+    if (qx_uniform(t.cid && nfrag <= 6)) md_cid_average(B, M, sys, nfrag, Lm);
     if (lane != 0) return;
     if (!t.cid) {
         // electronic temperature for the next egrad (md.f90:443-445): setetemp
@@ -684,17 +687,28 @@ QX_DEV void md_post_system(const BatchPtrs& B, const MdPtrs& M, const MdParams& 
     }
 }
 
-__global__ __launch_bounds__(64) void k_md_pre(BatchPtrs B, MdPtrs M, MdParams p)
+// Arguments of the MD step kernels (opt, nsteps: the persistent one)
+struct MdArgs {
+    BatchPtrs B;
+    MdPtrs M;
+    MdParams p;
+    SccOpts opt;
+    int nsteps;
+};
+
+__global__ __launch_bounds__(64) void k_md_pre(MdArgs args)
 {
     __shared__ MdLds Lm;
-    md_pre_system(B, M, p, blockIdx.x, Lm);
+    QX_ARG(MdArgs) a = qx_args(args);
+    md_pre_system(a.B, a.M, a.p, blockIdx.x, Lm);
 }
 
-// 256 threads: the heating search evaluates 256 increments per pass
-__global__ __launch_bounds__(QX_BLOCK) void k_md_post(BatchPtrs B, MdPtrs M, MdParams p)
+// the heating search evaluates as many increments per pass as threads
+__global__ __launch_bounds__(QX_BLOCK) void k_md_post(MdArgs args)
 {
     __shared__ MdLds Lm;
-    md_post_system(B, M, p, blockIdx.x, Lm);
+    QX_ARG(MdArgs) a = qx_args(args);
+    md_post_system(a.B, a.M, a.p, blockIdx.x, Lm);
 }
 
 // Persistent MD: one block of QX_SCC_BLOCK threads per trajectory runs up to
@@ -710,10 +724,10 @@ union FusedLds {
 };
 
 template <bool EIG>
-__global__ __launch_bounds__(QX_SCC_BLOCK) void k_md_fused(BatchPtrs B, MdPtrs M, MdParams p, SccOpts opt,
-                                                           int nsteps)
+__global__ __launch_bounds__(QX_SCC_BLOCK) void k_md_fused(MdArgs args)
 {
     static_assert(QX_SCC_BLOCK == QX_BLOCK, "the fused phases assume one block size");
+    QX_ARG(MdArgs) a0 = qx_args(args);
     const int sys = blockIdx.x;
     __shared__ FusedLds L;
     extern __shared__ double dyn[];
@@ -732,22 +746,35 @@ __global__ __launch_bounds__(QX_SCC_BLOCK) void k_md_fused(BatchPtrs B, MdPtrs M
     do {               \
     } while (0)
 #endif
-    for (int step = 0; step < nsteps; ++step) {
-        if (!M.active[sys]) break;
-        md_pre_system(B, M, p, sys, L.m);
+    auto fresh = [&]() -> QX_ARG(MdArgs) {
+        // the arguments loaded anew for each phase (B is their first member)
+        return (QX_ARG(MdArgs))qx_fresh(a0.B);
+    };
+    for (int step = 0; step < a0.nsteps; ++step) {
+        if (!qx_uniform(fresh().M.active[sys])) break;
+        {
+            QX_ARG(MdArgs) a = fresh();
+            md_pre_system(a.B, a.M, a.p, sys, L.m);
+        }
         __syncthreads();
         QX_FUSED_PH(24);
-        if (!M.active[sys]) break;
-        setup_system(B, sys, 1, L.s, dyn);
+        if (!qx_uniform(fresh().M.active[sys])) break;
+        setup_system(fresh().B, sys, 1, L.s, dyn);
         __syncthreads();
         QX_FUSED_PH(25);
-        scc_system<EIG>(B, opt, sys, L.c, dyn);
+        {
+            QX_ARG(MdArgs) a = fresh();
+            scc_system<EIG>(a.B, a.opt, sys, L.c, dyn);
+        }
         __syncthreads();
         QX_FUSED_PH(26);
-        grad_system(B, sys, L.g);
+        grad_system(fresh().B, sys, L.g);
         __syncthreads();
         QX_FUSED_PH(27);
-        md_post_system(B, M, p, sys, L.m);
+        {
+            QX_ARG(MdArgs) a = fresh();
+            md_post_system(a.B, a.M, a.p, sys, L.m);
+        }
         __syncthreads();
         QX_FUSED_PH(28);
     }

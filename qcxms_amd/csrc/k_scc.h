@@ -81,75 +81,90 @@ __device__ unsigned long long g_phase[kPhaseSys * kPhaseSlots];
 #endif
 
 // C[i][j] = sum_k opA[i][k] * d[k] * opB[k][j] on the FP64 matrix cores
-// (v_mfma_f64_16x16x4f64).  A wavefront computes a strip of two 16 x 16
-// tiles sharing the A operand; operand lanes: A[i0 + l%16][k0 + l/16],
-// B[k0 + l/16][j0 + l%16]; accumulator element r of lane l is
-// C[i0 + 4r + l/16][j0 + l%16].  Out-of-range rows, columns and k are zero.
+// (v_mfma_f64_16x16x4f64).  Operands are given by their element strides:
+// opA[i][k] at A[i * ai + k * ak], opB[k][j] at Bm[k * bk + j * bj].  A
+// wavefront computes a strip of two 16 x 16 tiles sharing the A operand;
+// operand lanes: A[i0 + l%16][k0 + l/16], B[k0 + l/16][j0 + l%16];
+// accumulator element r of lane l is C[i0 + 4r + l/16][j0 + l%16].  Lanes of
+// rows and columns past the edge read the last row or column (their results
+// are not stored); only the last k step is masked.  The operands of the next
+// four k steps are loaded while the matrix cores work on the current four, so
+// a strip waits for memory once.
 typedef double qx_d4 __attribute__((ext_vector_type(4)));
-template <bool TA, bool TB>
-QX_DEV void mfma_gemm(int M, int N, int K, const double* A, int lda, const double* Bm, int ldb,
-                      double* Cm, int ldc, const double* d)
+QX_DEV void mfma_gemm(int M, int N, int K, const double* A, int ai, int ak, const double* Bm, int bk,
+                      int bj, double* Cm, int ldc, const double* d)
 {
-    constexpr int NU = 2;  // 16 x 16 tiles per strip (more tiles cost the SCC body registers)
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    constexpr int NU = 2;  // 16 x 16 tiles per strip
+    constexpr int KS = 4;  // k steps per pass
+    const int tid = qx_tid(), lane = tid & 63, wave = qx_wave(tid);
     const int li = lane & 15, lk = lane >> 4;
     const int tm = (M + 15) >> 4, tc = (N + 16 * NU - 1) / (16 * NU);
+    const int nblk = K / (4 * KS);
     for (int t = wave; t < tm * tc; t += kNT / 64) {
         const int i0 = (t / tc) * 16, jc = (t % tc) * 16 * NU;
-        const int i = i0 + li;
-        const bool iin = i < M;
-        const int ic = iin ? i : M - 1;
-        int jcl[NU];
-        bool jin[NU];
+        const int i = i0 + li < M ? i0 + li : M - 1;
+        const double* pa = A + i * ai + lk * ak;
+        const double* pb[NU];
 #pragma unroll
         for (int u = 0; u < NU; ++u) {
-            const int j = jc + 16 * u + li;
-            jin[u] = j < N;
-            jcl[u] = jin[u] ? j : N - 1;
+            const int j = jc + 16 * u + li < N ? jc + 16 * u + li : N - 1;
+            pb[u] = Bm + lk * bk + j * bj;
         }
         qx_d4 acc[NU];
 #pragma unroll
         for (int u = 0; u < NU; ++u) acc[u] = qx_d4{0.0, 0.0, 0.0, 0.0};
-        // four k-steps per pass: all operand loads first, then the MFMAs
-        // (k-steps past K multiply zeros).  Loads are clamped into the
-        // matrices and out-of-range lanes zeroed afterwards, so no branch
-        // surrounds a load.
-        constexpr int KS = 4;
-        for (int k0 = 0; k0 < K; k0 += 4 * KS) {
-            double a[KS], b[KS][NU];
+        double a[KS], b[KS][NU];
+        auto load = [&](int k0) {
 #pragma unroll
             for (int q = 0; q < KS; ++q) {
-                const int k = k0 + 4 * q + lk;
-                const bool kin = k < K;
-                const int kc = kin ? k : K - 1;
-                double av = TA ? A[(size_t)kc * lda + ic] : A[(size_t)ic * lda + kc];
-                if (d) av *= d[kc];
-                a[q] = (iin && kin) ? av : 0.0;
+                a[q] = pa[(k0 + 4 * q) * ak];
+                if (d) a[q] *= d[k0 + 4 * q + lk];
 #pragma unroll
-                for (int u = 0; u < NU; ++u) {
-                    const double bv = TB ? Bm[(size_t)jcl[u] * ldb + kc] : Bm[(size_t)kc * ldb + jcl[u]];
-                    b[q][u] = (jin[u] && kin) ? bv : 0.0;
-                }
+                for (int u = 0; u < NU; ++u) b[q][u] = pb[u][(k0 + 4 * q) * bk];
             }
+        };
+        if (nblk) load(0);
+        for (int kb = 0; kb < nblk; ++kb) {
+            double ca[KS], cb[KS][NU];
+#pragma unroll
+            for (int q = 0; q < KS; ++q) {
+                ca[q] = a[q];
+#pragma unroll
+                for (int u = 0; u < NU; ++u) cb[q][u] = b[q][u];
+            }
+            if (kb + 1 < nblk) load((kb + 1) * 4 * KS);
 #pragma unroll
             for (int q = 0; q < KS; ++q)
 #pragma unroll
                 for (int u = 0; u < NU; ++u)
-                    acc[u] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[q], b[q][u], acc[u], 0, 0, 0);
+                    acc[u] = __builtin_amdgcn_mfma_f64_16x16x4f64(ca[q], cb[q][u], acc[u], 0, 0, 0);
+        }
+        // the rest, the last k step masked (lanes past K read k0 itself)
+        for (int k0 = nblk * 4 * KS; k0 < K; k0 += 4) {
+            const bool kin = k0 + lk < K;
+            const int k = kin ? k0 : k0 - lk;
+            double ta = pa[k * ak];
+            if (d) ta *= d[k + lk];
+            ta = kin ? ta : 0.0;
+#pragma unroll
+            for (int u = 0; u < NU; ++u) {
+                const double tb = pb[u][k * bk];
+                acc[u] = __builtin_amdgcn_mfma_f64_16x16x4f64(ta, kin ? tb : 0.0, acc[u], 0, 0, 0);
+            }
         }
 #pragma unroll
         for (int u = 0; u < NU; ++u)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const int row = i0 + 4 * r + lk, col = jc + 16 * u + li;
-                if (row < M && col < N) Cm[(size_t)row * ldc + col] = acc[u][r];
+                if (row < M && col < N) Cm[row * ldc + col] = acc[u][r];
             }
     }
 }
 
 QX_DEV double block_max(double v, double* smem)
 {
-    for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o, 64));
+    v = wave_max(v);
     const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
     __syncthreads();
     if (l == 0) smem[w] = v;
@@ -165,8 +180,7 @@ template <int K>
 QX_DEV void block_sums(double* v, double* smem)
 {
 #pragma unroll
-    for (int k = 0; k < K; ++k)
-        for (int o = 32; o > 0; o >>= 1) v[k] += __shfl_xor(v[k], o, 64);
+    for (int k = 0; k < K; ++k) v[k] = wave_sum(v[k]);
     const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
     __syncthreads();
     if (l == 0)
@@ -198,9 +212,10 @@ QX_DEV void rr_pair(int m, int r, int k, int& p, int& q)
 QX_DEV double offdiag_max(const double* A, int m, int lda, double* red)
 {
     double mx = 0.0;
-    for (int i = threadIdx.x >> 6; i < m; i += kNT / 64)
-        for (int j = threadIdx.x & 63; j < m; j += 64)
-            if (i != j) mx = fmax(mx, fabs(A[(size_t)i * lda + j]));
+    const int tid = qx_tid();
+    for (int i = qx_wave(tid); i < m; i += kNT / 64)
+        for (int j = tid & 63; j < m; j += 64)
+            if (i != j) mx = fmax(mx, fabs(A[i * lda + j]));
     return block_max(mx, red);
 }
 
@@ -213,357 +228,642 @@ QX_DEV void tri_index(int b, int& P, int& R)
     R = b - P * (P + 1) / 2;
 }
 
-// Jacobi rotation (c, s) that zeroes a_pq:
-//   r = sqrt(d^2 + 4 a^2), d = a_qq - a_pp, u = r + |d|,
-//   c = sqrt(u / 2r), s = 2 a sign(d) c / u   (c^2 + s^2 = 1 exactly)
+// Jacobi rotation (c, s) that zeroes a_pq: with d = a_qq - a_pp and
+//   1/r = 1 / sqrt(d^2 + 4 a^2),  c^2 = (1 + |d| / r) / 2,
+//   s = a sign(d) / (r c)   (c^2 + s^2 = 1)
 // i.e. t = s / c = 2 a sign(d) / (|d| + r), the smaller root of
-// t^2 + t d / a - 1 = 0.  Three dependent long-latency operations.
+// t^2 + t d / a - 1 = 0.  Two reciprocal roots in a row and no division: the
+// rotation is the critical path of a Jacobi round.
 QX_DEV double2 jacobi_rotation(double app, double aqq, double apq)
 {
-    const double d = aqq - app, ad = fabs(d);
-    const double r = sqrt(d * d + 4.0 * apq * apq);
-    const double u = r + ad;
-    const double ir = 1.0 / r, iu = 1.0 / u;
-    const double c = sqrt(0.5 * u * ir);
-    const double s = 2.0 * (d >= 0.0 ? apq : -apq) * c * iu;
-    return make_double2(c, s);
+    const double d = aqq - app, a2 = 2.0 * apq;
+    const double ir = qx_rsqrt(d * d + a2 * a2);
+    const double w = 0.5 + 0.5 * fabs(d) * ir;
+    const double ic = qx_rsqrt(w);
+    return make_double2(w * ic, (d >= 0.0 ? apq : -apq) * ir * ic);
 }
 
-// Rotated entries of the 2 x 2 blocks (P, R) and (R, P): input b00 = A[p][r],
+// Rotated entries of the 2 x 2 block (P, R): input b00 = A[p][r],
 // b01 = A[p][s], b10 = A[q][r], b11 = A[q][s] with (p, q) the pair of P and
-// (r, s) the pair of R; on the diagonal block (P == R) the off-diagonal
+// (r, s) the pair of R; on a rotated diagonal block (P == R) the off-diagonal
 // entries become exact zeros.
 QX_DEV void rotate_block(double2 rp, double2 rr, bool diag, const double b[4], double n[4])
 {
     const double cp = rp.x, sp = rp.y, cr = rr.x, sr = rr.y;
     const double m00 = b[0] * cr - b[1] * sr, m01 = b[0] * sr + b[1] * cr;
     const double m10 = b[2] * cr - b[3] * sr, m11 = b[2] * sr + b[3] * cr;
+    const bool zero = diag && sp != 0.0;
     n[0] = cp * m00 - sp * m10;
-    n[1] = diag ? 0.0 : cp * m01 - sp * m11;
-    n[2] = diag ? 0.0 : sp * m00 + cp * m10;
+    n[1] = zero ? 0.0 : cp * m01 - sp * m11;
+    n[2] = zero ? 0.0 : sp * m00 + cp * m10;
     n[3] = sp * m01 + cp * m11;
 }
 
-QX_DEV void store_block(double* A, int lda, int2 ip, int2 ir, bool diag, const double n[4])
+// Where the player of seat s (pair slot s / 2, p or q side) sits in the next
+// round: the p players move one slot down, the q players one up, the ends
+// turn round and q of slot 0 stays.
+QX_DEV int rr_move(int half, int s)
 {
-    A[(size_t)ip.x * lda + ir.x] = n[0];
-    A[(size_t)ip.x * lda + ir.y] = n[1];
-    A[(size_t)ip.y * lda + ir.x] = n[2];
-    A[(size_t)ip.y * lda + ir.y] = n[3];
-    if (!diag) {
-        A[(size_t)ir.x * lda + ip.x] = n[0];
-        A[(size_t)ir.y * lda + ip.x] = n[1];
-        A[(size_t)ir.x * lda + ip.y] = n[2];
-        A[(size_t)ir.y * lda + ip.y] = n[3];
+    const int k = s >> 1;
+    if (half == 1) return s;
+    if ((s & 1) == 0) return k == 0 ? 3 : s - 2;
+    if (k == 0) return s;
+    return k == half - 1 ? s - 1 : s + 2;
+}
+
+// The players that meet in pair slot k of the next round: the p side comes
+// from slot K1 (its q player if s1, else its p player), the q side from slot
+// K2 (s2 likewise); K1 > K2 for half > 1.
+QX_DEV void rr_next(int half, int k, int& K1, int& s1, int& K2, int& s2)
+{
+    if (k == 0) {
+        K1 = half > 1 ? 1 : 0;
+        s1 = 0;
+        K2 = 0;
+        s2 = 1;
+    } else {
+        K1 = k == half - 1 ? k : k + 1;
+        s1 = k == half - 1 ? 1 : 0;
+        K2 = k - 1;
+        s2 = k == 1 ? 0 : 1;
     }
 }
 
-QX_DEV void load_block(const double* A, int lda, int2 ip, int2 ir, double b[4])
+// The rotation of one pivot, the identity for pairs left alone
+QX_DEV double2 pivot_rotation(double app, double aqq, double apq, double tol, double min_s)
 {
-    b[0] = A[(size_t)ip.x * lda + ir.x];
-    b[1] = A[(size_t)ip.x * lda + ir.y];
-    b[2] = A[(size_t)ip.y * lda + ir.x];
-    b[3] = A[(size_t)ip.y * lda + ir.y];
+    const double2 cs = jacobi_rotation(app, aqq, apq);
+    const bool turn = !(fabs(apq) < tol) && fabs(cs.y) > min_s;
+    return make_double2(turn ? cs.x : 1.0, turn ? cs.y : 0.0);
+}
+
+// Working storage of the Jacobi sweeps
+struct JacobiBuffers {
+    double* blk;      // A as 2 x 2 blocks by seats: 4 planes of half (half + 1) / 2 doubles (LDS)
+    double* gblk[2];  // two of them in global memory, for systems too large
+    double2* log;     // rotations of a sweep: (m - 1) x m / 2
+    double2* rot;     // rotations of two rounds (LDS)
+    int* any;         // per round of a sweep: whether it rotates anything (LDS, m entries)
+    double* red;
+    bool lds;         // the blocks fit in LDS
+};
+
+// The pivot of a lane in the next round: its two slots and their blocks
+struct JacobiPivot {
+    int K1, K2, i1, i2, i12;
+    bool s1, s2;
+    double d1[3], d2[3], b4[4];
+    double2 r1, r2;
+
+    QX_DEV void place(int half, int k)
+    {
+        int a, b;
+        rr_next(half, k < half ? k : 0, K1, a, K2, b);
+        s1 = a;
+        s2 = b;
+        i1 = K1 * (K1 + 1) / 2 + K1;
+        i2 = K2 * (K2 + 1) / 2 + K2;
+        i12 = K1 * (K1 + 1) / 2 + K2;
+    }
+    QX_DEV void load(const double* blk, int nblk, const double2* rf)
+    {
+        r1 = rf[K1];
+        r2 = rf[K2];
+        d1[0] = blk[i1];
+        d1[1] = blk[nblk + i1];
+        d1[2] = blk[3 * nblk + i1];
+        d2[0] = blk[i2];
+        d2[1] = blk[nblk + i2];
+        d2[2] = blk[3 * nblk + i2];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) b4[e] = blk[e * nblk + i12];
+    }
+    // the rotation, from the pivot's entries after this round (formed as the
+    // threads that store them form them)
+    QX_DEV double2 rotation(int half, double tol, double min_s) const
+    {
+        const double x1 = d1[0] * r1.x - d1[1] * r1.y, y1 = d1[0] * r1.y + d1[1] * r1.x;
+        const double u1 = d1[1] * r1.x - d1[2] * r1.y, v1 = d1[1] * r1.y + d1[2] * r1.x;
+        const double app = s1 ? r1.y * y1 + r1.x * v1 : r1.x * x1 - r1.y * u1;
+        const double x2 = d2[0] * r2.x - d2[1] * r2.y, y2 = d2[0] * r2.y + d2[1] * r2.x;
+        const double u2 = d2[1] * r2.x - d2[2] * r2.y, v2 = d2[1] * r2.y + d2[2] * r2.x;
+        const double aqq = s2 ? r2.y * y2 + r2.x * v2 : r2.x * x2 - r2.y * u2;
+        double nb[4];
+        rotate_block(r1, r2, false, b4, nb);
+        double apq = s1 ? (s2 ? nb[3] : nb[2]) : (s2 ? nb[1] : nb[0]);
+        if (half == 1) apq = r1.y != 0.0 ? 0.0 : d1[1];
+        return pivot_rotation(app, aqq, apq, tol, min_s);
+    }
+};
+
+// Where the four entries of block b go in the next round (indices into the
+// four planes)
+QX_DEV void block_moves(int half, int nblk, int P, int R, int to[4])
+{
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        // (1, 0) of a diagonal block is (0, 1) again
+        const int x = rr_move(half, 2 * P + (P == R && e == 2 ? 0 : e >> 1));
+        const int y = rr_move(half, 2 * R + (P == R && e == 2 ? 1 : e & 1));
+        const int hi = (x >> 1) > (y >> 1) ? x : y, lo = hi == x ? y : x;
+        const int Ph = hi >> 1, Rh = lo >> 1;
+        const int plane = Ph == Rh ? (x == y ? 3 * (x & 1) : 1) : 2 * (hi & 1) + (lo & 1);
+        to[e] = plane * nblk + Ph * (Ph + 1) / 2 + Rh;
+    }
+}
+
+// The rounds of one sweep, blocks in LDS.  NB: blocks per thread of the
+// wavefronts 1 ...; f: half of rot that holds the rotations of round 0.
+// NR > 0 (m <= 64): the rows of Cv as well, x[u] row wave - 1 + u (kNT / 64 -
+// 1) with a lane per column, so a rotation is one exchange between lanes and
+// two multiply-adds per row; they run while wavefront 0 has the pivots.
+// NR = 0: the rotations are logged instead.
+template <int NB, int NR>
+QX_DEV void jacobi_rounds(const JacobiBuffers& jb, int m, int nrow, double tol, double min_s, double* x, int& f)
+{
+    constexpr int kNU = kNT - 64, NW = kNT / 64 - 1, NK = NB > 3 ? 2 : 1;  // NK pivots per lane (half <= 64 NK)
+    const int tid = qx_tid(), lane = tid & 63, wave = qx_wave(tid), ut = tid - 64;
+    const int half = m / 2, nblk = half * (half + 1) / 2;
+    double* blk = jb.blk;
+    JacobiPivot pv[NK];                  // wavefront 0
+    int bPR[NB], to01[NB], to23[NB];     // the others: their blocks and where each entry goes
+    if (wave == 0) {
+#pragma unroll
+        for (int j = 0; j < NK; ++j) pv[j].place(half, lane + 64 * j);
+    } else {
+#pragma unroll
+        for (int j = 0; j < NB; ++j) {
+            int P, R, to[4];
+            tri_index(ut + j * kNU < nblk ? ut + j * kNU : 0, P, R);
+            bPR[j] = P | (R << 16);
+            block_moves(half, nblk, P, R, to);
+            to01[j] = to[0] | (to[1] << 16);
+            to23[j] = to[2] | (to[3] << 16);
+        }
+    }
+    for (int r = 0; r < m - 1; ++r, f ^= 1) {
+        const double2* rf = jb.rot + f * half;
+        double nn[NB][4];
+        int any = 0;
+        if (wave == 0) {
+#pragma unroll
+            for (int j = 0; j < NK; ++j) pv[j].load(blk, nblk, rf);
+        } else {
+            if (NR) any = qx_uniform(jb.any[r]);
+#pragma unroll
+            for (int j = 0; j < NB; ++j) {
+                const int b = ut + j * kNU;
+                if (b >= nblk) continue;
+                const int P = bPR[j] & 0xffff, R = bPR[j] >> 16;
+                double bb[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) bb[e] = blk[e * nblk + b];
+                if (P == R) bb[2] = bb[1];
+                rotate_block(rf[P], rf[R], P == R, bb, nn[j]);
+            }
+        }
+        qx_lds_barrier();
+        if (wave == 0) {
+            bool turn = false;
+#pragma unroll
+            for (int j = 0; j < NK; ++j) {
+                const double2 cs = pv[j].rotation(half, tol, min_s);
+                const int k = lane + 64 * j;
+                if (k < half) {
+                    turn = turn || cs.y != 0.0;
+                    jb.rot[(f ^ 1) * half + k] = cs;
+                    if (!NR && r + 1 < m - 1) jb.log[(r + 1) * half + k] = cs;
+                }
+            }
+            turn = qx_any(turn);
+            if (lane == 0) jb.any[r + 1] = turn;
+        } else {
+#pragma unroll
+            for (int j = 0; j < NB; ++j) {
+                if (ut + j * kNU >= nblk) continue;
+                blk[to01[j] & 0xffff] = nn[j][0];
+                blk[(unsigned)to01[j] >> 16] = nn[j][1];
+                blk[to23[j] & 0xffff] = nn[j][2];
+                blk[(unsigned)to23[j] >> 16] = nn[j][3];
+            }
+            if (NR && any) {
+                // pair slot, side and partner of the lane's player
+                int d = lane - r;
+                if (d < 0) d += m - 1;
+                bool qside = d > half - 1;
+                int k = qside ? m - 1 - d : d;
+                int partner = qside ? r + k : r - k;
+                if (partner < 0) partner += m - 1;
+                if (partner >= m - 1) partner -= m - 1;
+                if (lane == r) partner = m - 1;
+                if (lane >= m - 1) {
+                    qside = true;
+                    k = 0;
+                    partner = lane == m - 1 ? r : lane;
+                }
+                const double2 cs = rf[k];
+                const double s = qside ? cs.y : -cs.y;
+#pragma unroll
+                for (int u = 0; u < NR; ++u)
+                    if (wave - 1 + NW * u < nrow) x[u] = cs.x * x[u] + s * __shfl(x[u], partner, 64);
+            }
+        }
+        qx_lds_barrier();
+    }
+}
+
+// The same with the blocks in global memory (systems too large for LDS): read
+// from one buffer, written to the other.
+QX_DEV void jacobi_rounds_global(const JacobiBuffers& jb, int m, double tol, double min_s, int& f, int& g)
+{
+    constexpr int kNU = kNT - 64;
+    const int tid = qx_tid(), lane = tid & 63, wave = qx_wave(tid), ut = tid - 64;
+    const int half = m / 2, nblk = half * (half + 1) / 2;
+    for (int r = 0; r < m - 1; ++r, f ^= 1, g ^= 1) {
+        const double2* rf = jb.rot + f * half;
+        const double* src = jb.gblk[g];
+        double* dst = jb.gblk[g ^ 1];
+        if (wave == 0) {
+            bool turn = false;
+            for (int k = lane; k < half; k += 64) {
+                JacobiPivot pv;
+                pv.place(half, k);
+                pv.load(src, nblk, rf);
+                const double2 cs = pv.rotation(half, tol, min_s);
+                turn = turn || cs.y != 0.0;
+                jb.rot[(f ^ 1) * half + k] = cs;
+                if (r + 1 < m - 1) jb.log[(r + 1) * half + k] = cs;
+            }
+            turn = qx_any(turn);
+            if (lane == 0) jb.any[r + 1] = turn;
+        } else {
+            for (int b = ut; b < nblk; b += kNU) {
+                int P, R, to[4];
+                tri_index(b, P, R);
+                block_moves(half, nblk, P, R, to);
+                double bb[4], nn[4];
+                for (int e = 0; e < 4; ++e) bb[e] = src[e * nblk + b];
+                if (P == R) bb[2] = bb[1];
+                rotate_block(rf[P], rf[R], P == R, bb, nn);
+                for (int e = 0; e < 4; ++e) dst[to[e]] = nn[e];
+            }
+        }
+        __syncthreads();
+    }
+}
+
+// Columns of the nrow x m matrix Cv rotated by the logged sweep, any m: a
+// lane per pair slot (NS slots per lane) and NR rows per wavefront at a time
+// in registers, the players
+// moved between the lanes after every round, NR rows per wavefront at a time.
+template <int NS, int NR>
+QX_DEV void jacobi_replay_slots(const JacobiBuffers& jb, double* Cv, int m, int nrow, int lda)
+{
+    constexpr int NW = kNT / 64;
+    const int tid = qx_tid(), lane = tid & 63, wave = qx_wave(tid), half = m / 2;
+    for (int i0 = 0; i0 < nrow; i0 += NW * NR) {
+        double p[NR][NS], q[NR][NS];
+#pragma unroll
+        for (int u = 0; u < NR; ++u) {
+            const int i = i0 + wave + NW * u < nrow ? i0 + wave + NW * u : nrow - 1;
+#pragma unroll
+            for (int t = 0; t < NS; ++t) {
+                const int k = lane + 64 * t < half ? lane + 64 * t : half - 1;
+                p[u][t] = Cv[i * lda + k];
+                q[u][t] = Cv[i * lda + m - 1 - k];
+            }
+        }
+        double2 cs[NS];
+        auto fetch = [&](int r) {
+#pragma unroll
+            for (int t = 0; t < NS; ++t) {
+                const int k = lane + 64 * t < half ? lane + 64 * t : half - 1;
+                cs[t] = jb.log[r * half + k];
+            }
+        };
+        fetch(0);
+        for (int r = 0; r < m - 1; ++r) {
+            double2 cr[NS];
+#pragma unroll
+            for (int t = 0; t < NS; ++t) cr[t] = cs[t];
+            if (r + 1 < m - 1) fetch(r + 1);
+            if (qx_uniform(jb.any[r])) {
+#pragma unroll
+                for (int u = 0; u < NR; ++u)
+#pragma unroll
+                    for (int t = 0; t < NS; ++t) {
+                        const double x = p[u][t], y = q[u][t];
+                        p[u][t] = cr[t].x * x - cr[t].y * y;
+                        q[u][t] = cr[t].y * x + cr[t].x * y;
+                    }
+            }
+            // p players one slot down, q players one up (rr_move)
+#pragma unroll
+            for (int u = 0; u < NR; ++u) {
+                double np[NS], nq[NS];
+#pragma unroll
+                for (int t = 0; t < NS; ++t) {
+                    const int k = lane + 64 * t;
+                    const double down = qx_lane_up(p[u][t], t + 1 < NS ? qx_bcast(p[u][t + 1 < NS ? t + 1 : t], 0) : 0.0);
+                    np[t] = k == half - 1 ? q[u][t] : down;
+                    const double y = k == 0 ? p[u][t] : q[u][t];  // p of slot 0 turns round to q of slot 1
+                    nq[t] = qx_lane_down(y, t > 0 ? qx_bcast(q[u][t > 0 ? t - 1 : 0], 63) : q[u][0]);
+                }
+#pragma unroll
+                for (int t = 0; t < NS; ++t) {
+                    p[u][t] = np[t];
+                    q[u][t] = nq[t];
+                }
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < NR; ++u) {
+            const int i = i0 + wave + NW * u;
+#pragma unroll
+            for (int t = 0; t < NS; ++t) {
+                const int k = lane + 64 * t;
+                if (i < nrow && k < half) {
+                    Cv[i * lda + k] = p[u][t];
+                    Cv[i * lda + m - 1 - k] = q[u][t];
+                }
+            }
+        }
+    }
 }
 
 // Parallel cyclic threshold Jacobi on symmetric A (m x m, m even, leading
 // dimension lda).  Pairs with |a_pq| < tol, or whose rotation has |sin| <=
-// min_s, are not rotated; a sweep ends the
-// loop when no off-diagonal element of the result reaches tol.  Each rotation
-// is also applied to columns p, q of the nrow x m matrix Cv (leading
-// dimension lda), so Cv ends as Cv V with A = V^T A_in V diagonal.
-// One round = rotation parameters (one thread per pair) | barrier | block and
-// column updates | barrier; rounds without any rotation skip the updates.
-// A thread's first two blocks (P, R) and its column pair are the same in
-// every round, so their parameters and entries are fetched in two LDS round
-// trips (parameters, then data) before any store.
-QX_DEV int jacobi(double* A, double* Cv, int m, int nrow, int lda, double tol, int maxsweep,
-                  double2* rot, int2* rpq, double* red, int* s_any, double min_s = 0.0)
+// min_s, are not rotated; the sweeps end when no off-diagonal element of the
+// result reaches tol, at the latest after maxsweep.  The rotations are also
+// applied to the columns of the nrow x m matrix Cv (leading dimension lda),
+// so Cv ends as Cv V with A = V^T A_in V diagonal.
+//
+// What bounds a round is the latency of its rotations (two reciprocal roots
+// in a row on one pivot per lane) and the number of instructions that the
+// other wavefronts issue.  So A is kept as 2 x 2 blocks by seats of the
+// round-robin: every address of a thread is the same in every round, a block
+// is four conflict-free reads and four writes to where its players sit next.
+// Wavefront 0 does nothing but the pivots: while the others apply round r it
+// forms the three entries of each pivot of round r + 1 from the blocks they
+// come from and their rotation.  One barrier keeps the reads of a round
+// before its writes, one ends it.  Up to 64 columns the other wavefronts also
+// rotate Cv, held in registers; above that the rotations of a sweep are
+// logged and applied to Cv afterwards, without barriers.
+template <bool FAST, bool LDS>
+QX_DEV int jacobi(double* A, double* Cv, int m, int nrow, int lda, double tol, int maxsweep, double min_s,
+                  const JacobiBuffers& jb)
 {
-    const int half = m / 2;
-    if (offdiag_max(A, m, lda, red) < tol) return 0;
-    if (threadIdx.x == 0) {
-        s_any[0] = 0;
-        s_any[1] = 0;
+    constexpr int NW = kNT / 64 - 1, NR = FAST ? (kFastM + NW - 1) / NW : (64 + NW - 1) / NW;
+    const int half = m / 2, nblk = half * (half + 1) / 2;
+    if (qx_uniform(offdiag_max(A, m, lda, jb.red) < tol)) return 0;
+    const int tid = qx_tid(), lane = tid & 63, wave = qx_wave(tid);
+    const bool rows = FAST || (LDS && m <= 64);
+    int sweep = 0, f = 0, g = 0;
+    double* blk = LDS ? jb.blk : jb.gblk[0];
+    double x[NR];
+    for (int b = tid; b < nblk; b += kNT) {
+        int P, R;
+        int2 p, r;
+        tri_index(b, P, R);
+        rr_pair(m, 0, P, p.x, p.y);
+        rr_pair(m, 0, R, r.x, r.y);
+        blk[b] = A[p.x * lda + r.x];
+        blk[nblk + b] = A[p.x * lda + r.y];
+        blk[2 * nblk + b] = A[p.y * lda + r.x];
+        blk[3 * nblk + b] = A[p.y * lda + r.y];
+    }
+    if (rows) {
+#pragma unroll
+        for (int u = 0; u < NR; ++u) {
+            const int i = wave - 1 + NW * u;
+            x[u] = wave > 0 && i < nrow && lane < m ? Cv[i * lda + lane] : 0.0;
+        }
     }
     __syncthreads();
-    const int nblk = half * (half + 1) / 2;
-    int bP0 = 0, bR0 = 0, bP1 = 0, bR1 = 0;
-    const bool has0 = threadIdx.x < nblk, has1 = threadIdx.x + kNT < nblk;
-    if (has0) tri_index(threadIdx.x, bP0, bR0);
-    if (has1) tri_index(threadIdx.x + kNT, bP1, bR1);
-    // column pair slot from the low 5 thread bits, rows ic + kRG j
-    constexpr int kRG = kNT / 32, kRU = 64 / kRG;  // row groups, rows per thread in the first 64
-    const int kc = threadIdx.x & 31, ic = threadIdx.x >> 5;
-    const bool hasC = kc < half;
-    int sweep = 0;
-    QX_PT_INIT(jt)
+    if (wave == 0) {
+        bool turn = false;
+        for (int k = lane; k < half; k += 64) {
+            const int b = k * (k + 1) / 2 + k;
+            const double2 cs = pivot_rotation(blk[b], blk[3 * nblk + b], blk[nblk + b], tol, min_s);
+            turn = turn || cs.y != 0.0;
+            jb.rot[k] = cs;
+        }
+        turn = qx_any(turn);
+        if (lane == 0) jb.any[m - 1] = turn;
+    }
+    __syncthreads();
     while (sweep < maxsweep) {
         ++sweep;
-        for (int r = 0; r < m - 1; ++r) {
-            const int f = r & 1;
-            QX_PT(20, jt);
-            for (int k = threadIdx.x; k < half; k += kNT) {
-                int p, q;
-                rr_pair(m, r, k, p, q);
-                const double apq = A[(size_t)p * lda + q];
-                const double app = A[(size_t)p * lda + p], aqq = A[(size_t)q * lda + q];
-                double2 cs = make_double2(1.0, 0.0);
-                if (fabs(apq) >= tol) {
-                    cs = jacobi_rotation(app, aqq, apq);
-                    if (fabs(cs.y) > min_s) s_any[f] = 1;
-                    else cs = make_double2(1.0, 0.0);
-                }
-                rot[k] = cs;
-                rpq[k] = make_int2(p, q);
-            }
+        // round 0 of this sweep (its rotations come from the sweep before)
+        if (!rows)
+            for (int k = tid; k < half; k += kNT) jb.log[k] = jb.rot[f * half + k];
+        if (tid == 0) jb.any[0] = jb.any[m - 1];
+        __syncthreads();
+        if (FAST) jacobi_rounds<1, NR>(jb, m, nrow, tol, min_s, x, f);
+        else if (!LDS) jacobi_rounds_global(jb, m, tol, min_s, f, g);
+        else if (m <= 64) jacobi_rounds<2, NR>(jb, m, nrow, tol, min_s, x, f);
+        else if (nblk <= 3 * (kNT - 64)) jacobi_rounds<3, 0>(jb, m, nrow, tol, min_s, x, f);
+        else jacobi_rounds<6, 0>(jb, m, nrow, tol, min_s, x, f);
+        if (!LDS) blk = jb.gblk[g];
+        if (!rows) {
             __syncthreads();
-            QX_PT(16, jt);
-            QX_PT_COUNT(jt, 3);
-#ifdef QX_PHASE_TIMING
-            if (threadIdx.x == 0)
-                for (int k = 0; k < half; ++k) jt_acc[5] += rot[k].y != 0.0 ? 1 : 0;
-#endif
-            if (s_any[f]) {
-                QX_PT_COUNT(jt, 2);
-                // parameters
-                const double2 rp0 = rot[bP0], rr0 = rot[bR0], rp1 = rot[bP1], rr1 = rot[bR1];
-                const int2 ip0 = rpq[bP0], ir0 = rpq[bR0], ip1 = rpq[bP1], ir1 = rpq[bR1];
-                const double2 rc = rot[hasC ? kc : 0];
-                const int2 pc = rpq[hasC ? kc : 0];
-                const bool do0 = has0 && (rp0.y != 0.0 || rr0.y != 0.0);
-                const bool do1 = has1 && (rp1.y != 0.0 || rr1.y != 0.0);
-                const bool doC = hasC && rc.y != 0.0;
-                // data
-                double b0[4] = {0, 0, 0, 0}, b1[4] = {0, 0, 0, 0}, vp[kRU], vq[kRU];
-                if (do0) load_block(A, lda, ip0, ir0, b0);
-                if (do1) load_block(A, lda, ip1, ir1, b1);
-#pragma unroll
-                for (int u = 0; u < kRU; ++u) {
-                    const int i = ic + kRG * u;
-                    const bool ok = doC && i < nrow;
-                    vp[u] = ok ? Cv[(size_t)i * lda + pc.x] : 0.0;
-                    vq[u] = ok ? Cv[(size_t)i * lda + pc.y] : 0.0;
-                }
-                // rotate and store
-                if (do0) {
-                    double n0[4];
-                    const bool dg = bP0 == bR0;
-                    rotate_block(rp0, rr0, dg, b0, n0);
-                    store_block(A, lda, ip0, ir0, dg, n0);
-                }
-                if (do1) {
-                    double n1[4];
-                    const bool dg = bP1 == bR1;
-                    rotate_block(rp1, rr1, dg, b1, n1);
-                    store_block(A, lda, ip1, ir1, dg, n1);
-                }
-                if (doC) {
-                    const double c = rc.x, s = rc.y;
-#pragma unroll
-                    for (int u = 0; u < kRU; ++u) {
-                        const int i = ic + kRG * u;
-                        if (i < nrow) {
-                            Cv[(size_t)i * lda + pc.x] = c * vp[u] - s * vq[u];
-                            Cv[(size_t)i * lda + pc.y] = s * vp[u] + c * vq[u];
-                        }
-                    }
-                }
-                // larger systems: remaining blocks, rows and column pairs
-                for (int b = threadIdx.x + 2 * kNT; b < nblk; b += kNT) {
-                    int P, R;
-                    tri_index(b, P, R);
-                    const double2 xp = rot[P], xr = rot[R];
-                    if (xp.y == 0.0 && xr.y == 0.0) continue;
-                    const int2 jp = rpq[P], jr = rpq[R];
-                    double bb[4], nn[4];
-                    load_block(A, lda, jp, jr, bb);
-                    rotate_block(xp, xr, P == R, bb, nn);
-                    store_block(A, lda, jp, jr, P == R, nn);
-                }
-                for (int k = kc; k < half; k += 32) {
-                    const double2 cs = rot[k];
-                    if (cs.y == 0.0) continue;
-                    const int2 pq = rpq[k];
-                    for (int i = (k == kc ? ic + 64 : ic); i < nrow; i += kRG) {
-                        const double xv = Cv[(size_t)i * lda + pq.x], yv = Cv[(size_t)i * lda + pq.y];
-                        Cv[(size_t)i * lda + pq.x] = cs.x * xv - cs.y * yv;
-                        Cv[(size_t)i * lda + pq.y] = cs.y * xv + cs.x * yv;
-                    }
-                }
-            }
-            if (threadIdx.x == 0) s_any[f ^ 1] = 0;
-            __syncthreads();
-            QX_PT(17, jt);
+            if (m <= 128) jacobi_replay_slots<1, 6>(jb, Cv, m, nrow, lda);
+            else jacobi_replay_slots<2, 6>(jb, Cv, m, nrow, lda);
         }
-        if (threadIdx.x == 0) s_any[0] = 0;  // set by the sweep's last round
-        if (offdiag_max(A, m, lda, red) < tol) break;
+        if (sweep < maxsweep) {
+            double mx = 0.0;
+            for (int b = tid; b < nblk; b += kNT) {
+                int P, R;
+                tri_index(b, P, R);
+                mx = fmax(mx, fabs(blk[nblk + b]));
+                if (P != R) mx = fmax(fmax(mx, fabs(blk[b])), fmax(fabs(blk[2 * nblk + b]), fabs(blk[3 * nblk + b])));
+            }
+            if (qx_uniform(block_max(mx, jb.red) < tol)) break;
+        }
     }
-    QX_PT_FLUSH(jt);
+    __syncthreads();
+    for (int b = tid; b < nblk; b += kNT) {
+        int P, R;
+        int2 p, r;
+        tri_index(b, P, R);
+        rr_pair(m, 0, P, p.x, p.y);
+        rr_pair(m, 0, R, r.x, r.y);
+        const double n[4] = {blk[b], blk[nblk + b], blk[P == R ? nblk + b : 2 * nblk + b], blk[3 * nblk + b]};
+        A[p.x * lda + r.x] = n[0];
+        A[p.x * lda + r.y] = n[1];
+        A[p.y * lda + r.x] = n[2];
+        A[p.y * lda + r.y] = n[3];
+        if (P == R) continue;
+        A[r.x * lda + p.x] = n[0];
+        A[r.y * lda + p.x] = n[1];
+        A[r.x * lda + p.y] = n[2];
+        A[r.y * lda + p.y] = n[3];
+    }
+    if (rows) {
+#pragma unroll
+        for (int u = 0; u < NR; ++u) {
+            const int i = wave - 1 + NW * u;
+            if (wave > 0 && i < nrow && lane < m) Cv[i * lda + lane] = x[u];
+        }
+    }
+    __syncthreads();
     return sweep;
 }
 
 constexpr double kCoarseSin = 0.02;  // |sin| of the rotations a coarse sweep applies
 constexpr int kCoarseSweeps = 3;      // coarse sweeps before the refinement gives up
 
-// Simultaneous-rotation refinement of a nearly diagonal symmetric A (m x m,
-// leading dimension lda) by FP64 MFMA products.  Every pair (i, j) gets the
-// angle of the Jacobi rotation that would zero a_ij alone; with K the
-// antisymmetric matrix of the angles, Y = I + K (+ K^2 / 2 when max |K| >
-// 1e-4 or <= 1e-5) is orthogonal up to O(K^2) (O(K^4)), and none, one or two
-// Newton-Schulz steps R <- R (3 I - R^T R) / 2 make it orthogonal to
-// rounding.  Then A <- R^T A R and Cv <- Cv R (nrow x m).  The off-diagonal
-// decreases quadratically (errors of the simultaneous angles are second
-// order in the off-diagonal over the eigenvalue gaps).  An angle above 0.1
-// (near-degenerate pairs with a relatively large coupling, typically at the
-// first SCC iteration after the geometry moved: the series would need more
-// terms) calls for a coarse Jacobi sweep that rotates only the pairs whose
-// rotation has |sin| > kCoarseSin, up to kCoarseSweeps times; from the first
-// one on, pairs with a coupling below tol are left alone, as Jacobi leaves
-// them.  Returns true when the largest off-diagonal magnitude is below tol
-// after at most maxit rounds (besides the coarse sweeps); false, possibly
-// after some rounds, when the angles stay above 0.1 or the rounds did not
-// suffice, and the caller finishes with Jacobi.  Y, Z, T: m x m scratch
-// (leading dimension lda); rot, rpq, s_any: the Jacobi buffers.  Called by
-// all threads.
-QX_DEV bool eig_rotate(double* A, double* Cv, int m, int nrow, int lda, double tol, int maxit, double* Y,
-                       double* Z, double* T, double* red, double2* rot, int2* rpq, int* s_any)
+// Eigenvectors of a symmetric A (m x m, leading dimension lda) to
+// off-diagonals below tol, Cv <- Cv V (nrow x m).
+//
+// With T (a fifth matrix), simultaneous rotations by FP64 MFMA products come
+// first.  Every pair (i, j) gets the angle of the Jacobi rotation that would
+// zero a_ij alone; with K the antisymmetric matrix of the angles,
+// Y = I + K (+ K^2 / 2 when max |K| > 1e-4 or <= 1e-5) is orthogonal up to
+// O(K^2) (O(K^4)), and none, one or two Newton-Schulz steps
+// R <- R (3 I - R^T R) / 2 make it orthogonal to rounding.  Then
+// A <- R^T A R and Cv <- Cv R.  The off-diagonal decreases quadratically
+// (errors of the simultaneous angles are second order in the off-diagonal
+// over the eigenvalue gaps).  An angle above 0.1 (near-degenerate pairs with
+// a relatively large coupling, typically at the first SCC iteration after
+// the geometry moved: the series would need more terms) calls for a coarse
+// Jacobi sweep that rotates only the pairs whose rotation has |sin| >
+// kCoarseSin, up to kCoarseSweeps times; from the first one on, pairs with a
+// coupling below tol are left alone, as Jacobi leaves them.  When the angles
+// stay above 0.1, kRounds rounds did not suffice or there is no T, full
+// Jacobi sweeps finish (or do it all).
+// Y, Z, T: m x m scratch (leading dimension lda; T may be null).  Called by
+// all threads.  Returns the number of full Jacobi sweeps.
+constexpr int kRounds = 3;
+template <bool EIG, bool FAST>
+QX_DEV int eig_solve(double* A, double* Cv, int m, int nrow, int lda, double tol, double* Y, double* Z,
+                     double* T, const JacobiBuffers& jb)
 {
-    const int tid = threadIdx.x;
-    if (offdiag_max(A, m, lda, red) < tol) return true;
-    int coarse = 0;
-    for (int it = 0; it < maxit + coarse; ++it) {
-        // one angle per pair i < j (K_ji = -K_ij): rows r and m - 1 - r of
-        // the upper triangle together hold m - 1 pairs, so pair b maps to
-        // (r, c) = (b / (m - 1), b % (m - 1)) without a square root (m even)
-        double kmax = 0.0;
-        for (int b = tid; b < (m / 2) * (m - 1); b += kNT) {
-            const int r = b / (m - 1), c = b - r * (m - 1);
-            const bool first = c < m - 1 - r;
-            const int i = first ? r : m - 1 - r;
-            const int j = first ? r + 1 + c : m - r + (c - (m - 1 - r));
-            const double a = A[(size_t)i * lda + j];
-            const double d = A[(size_t)j * lda + j] - A[(size_t)i * lda + i];
-            const double rr = sqrt(d * d + 4.0 * a * a);
-            const double t = rr > 0.0 ? 2.0 * (d >= 0.0 ? a : -a) / (fabs(d) + rr) : 0.0;
-            // after a coarse sweep, pairs below tol are left alone as Jacobi leaves them
-            const double th = (coarse && fabs(a) < tol) ? 0.0 : atan(t);
-            Y[(size_t)i * lda + j] = th;
-            Y[(size_t)j * lda + i] = -th;
-            kmax = fmax(kmax, fabs(th));
-        }
-        for (int i = tid; i < m; i += kNT) Y[(size_t)i * lda + i] = 0.0;
-        kmax = block_max(kmax, red);
-        if (kmax > 0.1) {
+    double* red = jb.red;
+    int coarse = 0, rounds = 0;
+    bool refine = EIG && T;
+    if (refine && qx_uniform(offdiag_max(A, m, lda, red) < tol)) return 0;
+    for (;;) {
+        const int tid = qx_tid();
+        int sweeps = 50;
+        double min_s = 0.0;
+        if (refine && rounds < kRounds) {
+            // one angle per pair i < j (K_ji = -K_ij): rows r and m - 1 - r of
+            // the upper triangle together hold m - 1 pairs, so pair b maps to
+            // (r, c) = (b / (m - 1), b % (m - 1)) without a square root (m even)
+            double kmax = 0.0;
+            for (int b = tid; b < (m / 2) * (m - 1); b += kNT) {
+                const int r = b / (m - 1), c = b - r * (m - 1);
+                const bool first = c < m - 1 - r;
+                const int i = first ? r : m - 1 - r;
+                const int j = first ? r + 1 + c : m - r + (c - (m - 1 - r));
+                const double a = A[i * lda + j];
+                const double d = A[j * lda + j] - A[i * lda + i];
+                const double rr = sqrt(d * d + 4.0 * a * a);
+                const double t = rr > 0.0 ? 2.0 * (d >= 0.0 ? a : -a) / (fabs(d) + rr) : 0.0;
+                // after a coarse sweep, pairs below tol are left alone as Jacobi leaves them
+                const double th = (coarse && fabs(a) < tol) ? 0.0 : atan(t);
+                Y[i * lda + j] = th;
+                Y[j * lda + i] = -th;
+                kmax = fmax(kmax, fabs(th));
+            }
+            for (int i = tid; i < m; i += kNT) Y[i * lda + i] = 0.0;
+            kmax = block_max(kmax, red);
+            if (qx_uniform(kmax <= 0.1)) {
+                // Y = I + K + K^2/2 has Y^T Y = I + K^4/4: with max |K| <= 1e-5
+                // that is below rounding and no Newton-Schulz step is needed
+                const bool quad = qx_uniform(kmax > 1e-4 || kmax <= 1e-5);
+                const int nns = qx_uniform(kmax > 0.005 ? 2 : (kmax > 1e-5 ? 1 : 0));
+                // the products one after the other (one copy of the product's
+                // code): K K, then per Newton-Schulz step R^T R and R Z, then
+                // A R, R^T (A R) and Cv R
+                double* R = Y;
+                double* W = T;
+                const int last = 1 + 2 * nns + 3;
+                for (int s = quad ? 0 : 1; s < last; ++s) {
+                    const int k = s == 0 ? 0 : s < 1 + 2 * nns ? 1 + ((s - 1) & 1) : 3 + (s - 1 - 2 * nns);
+                    if (s == 1) {
+                        for (int p = tid; p < m * m; p += kNT) {
+                            const int i = p / m, j = p - i * m, o = i * lda + j;
+                            Y[o] = (i == j ? 1.0 : 0.0) + Y[o] + (quad ? 0.5 * Z[o] : 0.0);
+                        }
+                        __syncthreads();
+                    }
+                    const double* pa = k == 3 ? A : k == 5 ? Cv : R;
+                    const bool ta = k == 1 || k == 4;
+                    const double* pb = k == 2 ? Z : k == 4 ? W : R;
+                    double* pc = k == 2 ? W : k == 3 ? W : k == 4 ? A : Z;
+                    mfma_gemm(k == 5 ? nrow : m, m, m, pa, ta ? 1 : lda, ta ? lda : 1, pb, lda, 1, pc, lda, nullptr);
+                    if (k != 4) __syncthreads();  // Cv R reads nothing that R^T W writes
+                    if (k == 1) {
+                        for (int p = tid; p < m * m; p += kNT) {
+                            const int i = p / m, j = p - i * m, o = i * lda + j;
+                            Z[o] = (i == j ? 1.5 : 0.0) - 0.5 * Z[o];
+                        }
+                        __syncthreads();
+                    } else if (k == 2) {
+                        double* t = R;
+                        R = W;
+                        W = t;
+                    }
+                }
+                for (int p = tid; p < nrow * m; p += kNT) {
+                    const int i = p / m, j = p - i * m;
+                    Cv[i * lda + j] = Z[i * lda + j];
+                }
+                __syncthreads();
+                ++rounds;
+                if (qx_uniform(offdiag_max(A, m, lda, red) < tol)) return 0;
+                continue;
+            }
             // strongly coupled pairs (near-degenerate orbitals after the
             // geometry moved): one Jacobi sweep over the pairs whose rotation
-            // exceeds kCoarseSin, up to kCoarseSweeps times, then the
-            // simultaneous rotations again
-            if (coarse == kCoarseSweeps) return false;
-            ++coarse;
-            jacobi(A, Cv, m, nrow, lda, tol, 1, rot, rpq, red, s_any, kCoarseSin);
-            QX_PH_ADD(29, 1);
-            continue;
-        }
-        // Y = I + K + K^2/2 has Y^T Y = I + K^4/4: with max |K| <= 1e-5 that
-        // is below rounding and no Newton-Schulz step is needed
-        const bool quad = kmax > 1e-4 || kmax <= 1e-5;
-        if (quad) {
-            mfma_gemm<false, false>(m, m, m, Y, lda, Y, lda, Z, lda, nullptr);
-            __syncthreads();
-        }
-        for (int p = tid; p < m * m; p += kNT) {
-            const int i = p / m, j = p - i * m;
-            const size_t o = (size_t)i * lda + j;
-            Y[o] = (i == j ? 1.0 : 0.0) + Y[o] + (quad ? 0.5 * Z[o] : 0.0);
-        }
-        __syncthreads();
-        double* R = Y;
-        const int nns = kmax > 0.005 ? 2 : (kmax > 1e-5 ? 1 : 0);
-        for (int s = 0; s < nns; ++s) {
-            mfma_gemm<true, false>(m, m, m, R, lda, R, lda, Z, lda, nullptr);
-            __syncthreads();
-            for (int p = tid; p < m * m; p += kNT) {
-                const int i = p / m, j = p - i * m;
-                const size_t o = (size_t)i * lda + j;
-                Z[o] = (i == j ? 1.5 : 0.0) - 0.5 * Z[o];
+            // exceeds kCoarseSin, then the simultaneous rotations again
+            if (coarse < kCoarseSweeps) {
+                ++coarse;
+                sweeps = 1;
+                min_s = kCoarseSin;
             }
-            __syncthreads();
-            double* out = R == Y ? T : Y;
-            mfma_gemm<false, false>(m, m, m, R, lda, Z, lda, out, lda, nullptr);
-            __syncthreads();
-            R = out;
         }
-        double* W = R == Y ? T : Y;
-        mfma_gemm<false, false>(m, m, m, A, lda, R, lda, W, lda, nullptr);
-        __syncthreads();
-        mfma_gemm<true, false>(m, m, m, R, lda, W, lda, A, lda, nullptr);
-        mfma_gemm<false, false>(nrow, m, m, Cv, lda, R, lda, Z, lda, nullptr);
-        __syncthreads();
-        for (int p = tid; p < nrow * m; p += kNT) {
-            const int i = p / m, j = p - i * m;
-            Cv[(size_t)i * lda + j] = Z[(size_t)i * lda + j];
-        }
-        __syncthreads();
-        if (offdiag_max(A, m, lda, red) < tol) return true;
+        const int done = FAST || jb.lds ? jacobi<FAST, true>(A, Cv, m, nrow, lda, tol, sweeps, min_s, jb)
+                                        : jacobi<FAST, false>(A, Cv, m, nrow, lda, tol, sweeps, min_s, jb);
+        if (sweeps != 1) return done;
+        QX_PH_ADD(29, 1);
     }
-    return false;
 }
 
-// The Broyden weights of up to kWaveSolve secant pairs on wavefront 0: solve
-// (B) x = diag(om) gm for the n x n symmetric positive definite B (leading
-// dimension lb) and return gm <- diag(om) x.  Lane i keeps row i of B in
-// registers; a right-looking Cholesky factor B = L L^T (column j: lane j's
-// pivot, the other lanes' multipliers, rank-1 update of the trailing rows by
-// lane broadcasts), then L y = diag(om) gm forward and L^T x = y backward.
-// Called by the 64 threads of wavefront 0.
-constexpr int kWaveSolve = 16;
-QX_DEV void broyden_solve_wave(const double* B, int lb, double* gm, const double* om, int n)
+// The Broyden weights of n secant pairs by the whole block: solves (B) x = g
+// for the n x n symmetric positive definite B in rows 0 .. n - 1 of bt (lower
+// triangle, leading dimension st) with g as row n, and returns x in gm.
+// B = U D^-1 U^T column by column without roots (column j of U is the column
+// as the elimination reaches it), one barrier per column; g eliminated along
+// with it is the forward substitution.  The backward substitution is on
+// wavefront 0, a lane per column (two for n > 64).  n <= 128.
+QX_DEV void broyden_solve(double* bt, int st, double* gm, int n)
 {
-    const int i = threadIdx.x & 63;
-    double r[kWaveSolve];
-#pragma unroll
-    for (int k = 0; k < kWaveSolve; ++k)
-        r[k] = (i < n && k < n) ? B[(size_t)i * lb + k] : (i == k ? 1.0 : 0.0);
-    double g = i < n ? gm[i] * om[i] : 0.0;
-#pragma unroll
-    for (int j = 0; j < kWaveSolve; ++j) {
-        if (j < n) {
-            const double d = sqrt(__shfl(r[j], j, 64));
-            if (i == j) r[j] = d;
-            else if (i > j) r[j] = r[j] / d;
-#pragma unroll
-            for (int k = j + 1; k < kWaveSolve; ++k) {
-                const double lkj = __shfl(r[j], k, 64);
-                if (i >= k) r[k] = r[k] - r[j] * lkj;
-            }
+    const int tid = qx_tid(), lane = tid & 63;
+    const int ti = tid >> 4, tk = tid & 15;
+    for (int j = 0; j < n; ++j) {
+        const double inv = 1.0 / bt[j * st + j];
+        for (int i = j + 1 + ti; i <= n; i += kNT / 16) {
+            const double l = bt[i * st + j] * inv;
+            for (int k = j + 1 + tk; k <= i && k < n; k += 16) bt[i * st + k] -= l * bt[k * st + j];
+        }
+        __syncthreads();
+    }
+    if (tid < 64) {
+        const int j0 = lane < n ? lane : n - 1, j1 = lane + 64 < n ? lane + 64 : n - 1;
+        double y0 = bt[n * st + j0], y1 = bt[n * st + j1];
+        const double d0 = 1.0 / bt[j0 * st + j0], d1 = 1.0 / bt[j1 * st + j1];
+        for (int i = n - 1; i >= 0; --i) {
+            const double x = i < 64 ? qx_bcast(y0 * d0, i) : qx_bcast(y1 * d1, i - 64);
+            const double* u = bt + i * st;
+            if (lane == 0) gm[i] = x;
+            if (j0 < i) y0 -= u[j0] * x;
+            if (j1 < i) y1 -= u[j1] * x;
         }
     }
-    // forward: L y = g
-#pragma unroll
-    for (int k = 0; k < kWaveSolve; ++k) {
-        if (k < n) {
-            const double yk = __shfl(g, k, 64) / __shfl(r[k], k, 64);
-            if (i == k) g = yk;
-            else if (i > k) g = g - r[k] * yk;
-        }
-    }
-    // backward: L^T x = y (lane i takes L[k][i] from lane k)
-#pragma unroll
-    for (int k = kWaveSolve - 1; k >= 0; --k) {
-        if (k < n) {
-            const double xk = __shfl(g, k, 64) / __shfl(r[k], k, 64);
-            double lki = 0.0;
-#pragma unroll
-            for (int c = 0; c < kWaveSolve; ++c) {
-                const double v = __shfl(r[c], k, 64);
-                if (c == i) lki = v;
-            }
-            if (i == k) g = xk;
-            else if (i < k) g = g - lki * xk;
-        }
-    }
-    if (i < n) gm[i] = g * om[i];
+    __syncthreads();
 }
 
 // Fermi occupations per spin on wavefront 0 for nalpha electrons; returns -TS.
@@ -625,104 +925,192 @@ struct SysShared {
     int ao_at[QX_MAX_NAO], ao_sh[QX_MAX_NAO];
     int shoff[QX_MAX_NAT + 1], aooff[QX_MAX_NAT + 1];  // shells/AOs of atom a: [off[a], off[a+1])
     int sel[QX_MAX_NAT], refoff[QX_MAX_NAT + 1];
+    unsigned char refat[kMaxRef];          // atom of a D4 reference
+    int eroff[gfn2::kElem + 1];            // D4 references of the elements present: [off[e], off[e+1])
     double sx[3 * QX_MAX_NAT];
     double mrad[QX_MAX_NAT];
     double qat[QX_MAX_NAT], vat[QX_MAX_NAT];
-    double zr[kMaxRef], dzr[kMaxRef], yr[kMaxRef];
+    // D4 references inside potentials(); between its calls the same LDS holds
+    // the Jacobi rotations, its round flags and the Broyden weights
+    union {
+        struct {
+            double zr[kMaxRef], dzr[kMaxRef], yr[kMaxRef];
+        };
+        struct {
+            alignas(16) double rot[2 * QX_MAX_NAO];  // (c, s) pairs of two rounds
+            int any[QX_MAX_NAO];
+            double gm[128];  // at most `mem` <= 100 pairs
+        };
+    };
     double red[8 * (kNT / 64)];
     double eparts[6];  // es2, es3, aes, axc, d4, unused
 };
 
+// LDS doubles potentials() works in: inner D4 sums, multipole shares, outer
+// D4 sums
+inline __host__ __device__ int pot_lds(int nat, int ndim)
+{
+    const int nu = kNT - 64, nseg = ndim * 4 <= nu ? 4 : ndim * 2 <= nu ? 2 : 1;
+    return gfn2::kElem * QX_MAX_REF * nat + (nat <= 32 ? 20 : 40) * nat + nseg * ndim;
+}
+
 // Potentials vs (per shell), vd (3 per atom), vq (6 per atom) and interaction
 // energies (ES2, ES3, AES, AXC, D4 two-body) at moments x = [qsh, dp, qp].
-// Wavefront 0 evaluates the multipole terms (lane = atom, loop over partners
-// through the precomputed kernel planes); wavefronts 1-3 evaluate the D4
-// response y = W z and the shell Coulomb potential gamma q as column sweeps
-// of the symmetric matrices.  The AES energy is x . v_aes / 2 (the
-// multipole energy is a symmetric bilinear form of the moments).
-QX_DEV void potentials(const SysInfo& si, const BatchPtrs& B, SysShared& ss, const double* x,
-                       double* vs, double* vd, double* vq)
+// The D4 response of reference k of atom i is
+//   y_k = gw_k sum_j disp_ij sum_(l of j) C6ref_kl gw_l z_l,
+// whose inner sum depends on i through its element and reference number only:
+// it is formed once per (element, reference, atom j), which leaves nat
+// terms per reference instead of ndim, and nat^2 values to read instead of
+// ndim^2.  The multipole terms read two damped kernels per atom pair (1/r^3
+// and 1/r^5) and take the directions from the coordinates.  First the
+// wavefronts 0 .. na - 1 sum the multipole terms of a share of the partners
+// each while the others form the inner D4 sums and the shell Coulomb
+// potential gamma q; then wavefront 0 adds the shares up (lane = atom) while
+// the others take the outer D4 sums, several threads per reference.  The AES
+// energy is x . v_aes / 2 (the multipole energy is a symmetric bilinear form
+// of the moments).  scr: LDS, pot_lds(nat, ndim) doubles.
+// (26-atom C8H18+, 50 basis functions: 20-30 k cycles a call with one
+// multipole wavefront, ten kernel planes and the ndim^2 response matrix.)
+QX_DEV void potentials(const SysInfo& si, BatchRef B, SysShared& ss, const double* x, double* vs, double* vd,
+                       double* vq, double* scr)
 {
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int nat = si.nat, nsh = si.nsh, nd = si.ndim;
+    const int tid = qx_tid(), lane = tid & 63, wave = qx_wave(tid);
+    const int nat = si.nat, nsh = si.nsh, nd = si.ndim, nn = nat * nat;
     const double* qsh = x;
     const double* dp = x + nsh;
     const double* qp = x + nsh + 3 * nat;
-    QX_PT_INIT(pt)
+    const bool split = nat <= 32;  // two half-wavefronts of atoms
+    const int na = split ? 2 : 4;
+    const int ner = qx_uniform(ss.eroff[gfn2::kElem]);
+    double* tt = scr;                  // ner x nat inner D4 sums
+    double* pa = tt + ner * nat;       // na x 10 x nat multipole shares
+    double* py = pa + na * 10 * nat;   // outer D4 sums of the threads of a reference
+    const double* pk = B.pairk + (size_t)si.pair_off / QX_PAIR_STRIDE * QX_PAIR_KERN;
     for (int a = tid; a < nat; a += kNT) {
         double q = 0.0;
         for (int s = ss.shoff[a]; s < ss.shoff[a + 1]; ++s) q += qsh[s];
         ss.qat[a] = q;
     }
     __syncthreads();
+    const double* gw = B.gw + si.ref_off;
     for (int k = tid; k < nd; k += kNT) {
-        int a = 0;
-        while (ss.refoff[a + 1] <= k) ++a;
+        const int a = ss.refat[k];
         const ElemParams& e = g_tab.e[ss.sel[a]];
         const int r = k - ss.refoff[a];
-        const double c = e.gam * gfn2::kD4Gc;
-        ss.zr[k] = d4_zeta(gfn2::kD4Ga, c, e.refq[r] + e.zeff, ss.qat[a] + e.zeff);
-        ss.dzr[k] = d4_dzeta(gfn2::kD4Ga, c, e.refq[r] + e.zeff, ss.qat[a] + e.zeff);
+        double z, dz;
+        d4_zeta_both(gfn2::kD4Ga, e.gam * gfn2::kD4Gc, e.refq[r] + e.zeff, ss.qat[a] + e.zeff, z, dz);
+        const double g = gw[k];
+        ss.zr[k] = z * g;
+        ss.dzr[k] = dz * g;
     }
     __syncthreads();
-    QX_PT(22, pt);
     double eaes = 0.0, eaxc = 0.0, es2 = 0.0, es3 = 0.0, ed4 = 0.0;
-    if (wave == 0) {
-        // up to 32 atoms: lanes i and i + 32 take the two halves of the
-        // partners of atom i and add their sums; more atoms: one lane per atom
-        const bool split = nat <= 32;
-        const int i = split ? (lane & 31) : lane, h = split ? (lane >> 5) : 0;
-        const int jm = split ? (nat + 1) / 2 : nat;
-        const int j0 = h ? jm : 0, j1 = (split && !h) ? jm : nat;
+    if (wave < na) {
+        const int i = split ? (lane & 31) : lane;
+        const int part = split ? 2 * wave + (lane >> 5) : wave;  // of four
+        const int len = (nat + 3) / 4, j0 = part * len, j1 = j0 + len < nat ? j0 + len : nat;
         double v0 = 0.0, d0 = 0.0, d1 = 0.0, d2 = 0.0;
         double w0 = 0.0, w1 = 0.0, w2 = 0.0, w3 = 0.0, w4 = 0.0, w5 = 0.0;
         if (i < nat) {
-            const int nn = nat * nat;
-            const double* ag = B.aesg + (size_t)si.pair_off / QX_PAIR_STRIDE * QX_AES_COMP + i;
-#pragma unroll 4
-            for (int j = j0; j < j1; ++j) {
-                const double* g = ag + (size_t)j * nat;
-                const double g0 = g[0], g1 = g[nn], g2 = g[2 * nn], g3 = g[3 * nn], g4 = g[4 * nn],
-                             g5 = g[5 * nn], g6 = g[6 * nn], g7 = g[7 * nn], g8 = g[8 * nn],
-                             g9 = g[9 * nn];
-                const double qj = ss.qat[j];
-                const double m0 = dp[3 * j], m1 = dp[3 * j + 1], m2 = dp[3 * j + 2];
-                const double* t = qp + 6 * j;
-                v0 += m0 * g0 + m1 * g1 + m2 * g2 + t[0] * g3 + 2.0 * t[1] * g4 + t[2] * g5 +
-                      2.0 * t[3] * g6 + 2.0 * t[4] * g7 + t[5] * g8;
-                d0 += -qj * g0 + g9 * m0 - 3.0 * (g3 * m0 + g4 * m1 + g6 * m2);
-                d1 += -qj * g1 + g9 * m1 - 3.0 * (g4 * m0 + g5 * m1 + g7 * m2);
-                d2 += -qj * g2 + g9 * m2 - 3.0 * (g6 * m0 + g7 * m1 + g8 * m2);
-                w0 += qj * g3;
-                w1 += qj * g4;
-                w2 += qj * g5;
-                w3 += qj * g6;
-                w4 += qj * g7;
-                w5 += qj * g8;
+            const double x0 = ss.sx[3 * i], x1 = ss.sx[3 * i + 1], x2 = ss.sx[3 * i + 2];
+            constexpr int NJ = 8;
+            for (int jb = j0; jb < j1; jb += NJ) {
+                double h3[NJ], h5[NJ];
+#pragma unroll
+                for (int u = 0; u < NJ; ++u) {
+                    const int j = jb + u < j1 ? jb + u : i;  // (i, i) is zero
+                    h3[u] = pk[j * nat + i];
+                    h5[u] = pk[nn + j * nat + i];
+                }
+                qx_sched_fence();
+#pragma unroll
+                for (int u = 0; u < NJ; ++u) {
+                    const int j = jb + u < j1 ? jb + u : i;
+                    const double rv0 = x0 - ss.sx[3 * j], rv1 = x1 - ss.sx[3 * j + 1], rv2 = x2 - ss.sx[3 * j + 2];
+                    const double r2 = rv0 * rv0 + rv1 * rv1 + rv2 * rv2;
+                    const double g0 = h3[u] * rv0, g1 = h3[u] * rv1, g2 = h3[u] * rv2;
+                    const double t0 = h5[u] * rv0, t1 = h5[u] * rv1;
+                    const double g3 = t0 * rv0, g4 = t0 * rv1, g5 = t1 * rv1, g6 = t0 * rv2, g7 = t1 * rv2,
+                                 g8 = h5[u] * rv2 * rv2, g9 = r2 * h5[u];
+                    const double qj = ss.qat[j];
+                    const double m0 = dp[3 * j], m1 = dp[3 * j + 1], m2 = dp[3 * j + 2];
+                    const double* t = qp + 6 * j;
+                    v0 += m0 * g0 + m1 * g1 + m2 * g2 + t[0] * g3 + 2.0 * t[1] * g4 + t[2] * g5 +
+                          2.0 * t[3] * g6 + 2.0 * t[4] * g7 + t[5] * g8;
+                    d0 += -qj * g0 + g9 * m0 - 3.0 * (g3 * m0 + g4 * m1 + g6 * m2);
+                    d1 += -qj * g1 + g9 * m1 - 3.0 * (g4 * m0 + g5 * m1 + g7 * m2);
+                    d2 += -qj * g2 + g9 * m2 - 3.0 * (g6 * m0 + g7 * m1 + g8 * m2);
+                    w0 += qj * g3;
+                    w1 += qj * g4;
+                    w2 += qj * g5;
+                    w3 += qj * g6;
+                    w4 += qj * g7;
+                    w5 += qj * g8;
+                }
             }
         }
-        if (split) {
-            v0 += __shfl_xor(v0, 32, 64);
-            d0 += __shfl_xor(d0, 32, 64);
-            d1 += __shfl_xor(d1, 32, 64);
-            d2 += __shfl_xor(d2, 32, 64);
-            w0 += __shfl_xor(w0, 32, 64);
-            w1 += __shfl_xor(w1, 32, 64);
-            w2 += __shfl_xor(w2, 32, 64);
-            w3 += __shfl_xor(w3, 32, 64);
-            w4 += __shfl_xor(w4, 32, 64);
-            w5 += __shfl_xor(w5, 32, 64);
+        double pv[10] = {v0, d0, d1, d2, w0, w1, w2, w3, w4, w5};
+#pragma unroll
+        for (int k = 0; k < 10; ++k) {
+            if (split) pv[k] += __shfl_xor(pv[k], 32, 64);
+            if (i < nat && lane < (split ? 32 : 64)) pa[(wave * 10 + k) * nat + i] = pv[k];
         }
-        if (i < nat && h == 0) {
-            w1 *= 2.0;
-            w3 *= 2.0;
-            w4 *= 2.0;
+    } else {
+        const int t0 = tid - 64 * na, nt = kNT - 64 * na;
+        for (int p = t0; p < ner * nat; p += nt) {
+            const int er = p / nat, j = p - er * nat, ej = ss.sel[j];
+            int e = 0;
+            while (ss.eroff[e + 1] <= er) ++e;
+            const double* c6 = g_tab.c6ref[e][er - ss.eroff[e]][ej];
+            const int l0 = ss.refoff[j], nl = ss.refoff[j + 1] - l0;
+            double c[QX_MAX_REF], s = 0.0;
+#pragma unroll
+            for (int l = 0; l < QX_MAX_REF; ++l) c[l] = c6[l];
+#pragma unroll
+            for (int l = 0; l < QX_MAX_REF; ++l)
+                if (l < nl) s += c[l] * ss.zr[l0 + l];
+            tt[p] = s;
+        }
+        // shell Coulomb rows, from the threads at the other end
+        const double* G = B.gam + si.gam_off;
+        for (int a = nt - 1 - t0; a < nsh; a += nt) {
+            double v = 0.0;
+            constexpr int NB = 12;
+            for (int b0 = 0; b0 < nsh; b0 += NB) {
+                double g[NB];
+#pragma unroll
+                for (int u = 0; u < NB; ++u) g[u] = G[(b0 + u < nsh ? b0 + u : b0) * nsh + a];
+                qx_sched_fence();
+#pragma unroll
+                for (int u = 0; u < NB; ++u)
+                    if (b0 + u < nsh) v += g[u] * qsh[b0 + u];
+            }
+            const double q = qsh[a];
+            const double g3 = g_tab.e[ss.sh[a].el].third[ss.sh[a].k];
+            es2 += 0.5 * q * v;
+            es3 += g3 * q * q * q / 3.0;
+            vs[a] = v + g3 * q * q;
+        }
+    }
+    __syncthreads();
+    const int nu = kNT - 64, nseg = nd * 4 <= nu ? 4 : nd * 2 <= nu ? 2 : 1;
+    if (wave == 0) {
+        const int i = lane;
+        if (i < nat) {
+            double pv[10];
+#pragma unroll
+            for (int k = 0; k < 10; ++k) {
+                pv[k] = 0.0;
+                for (int w = 0; w < na; ++w) pv[k] += pa[(w * 10 + k) * nat + i];
+            }
+            const double v0 = pv[0], d0 = pv[1], d1 = pv[2], d2 = pv[3];
+            const double w0 = pv[4], w1 = 2.0 * pv[5], w2 = pv[6], w3 = 2.0 * pv[7], w4 = 2.0 * pv[8], w5 = pv[9];
             const ElemParams& ei = g_tab.e[ss.sel[i]];
             const double qi = ss.qat[i];
             const double mi0 = dp[3 * i], mi1 = dp[3 * i + 1], mi2 = dp[3 * i + 2];
             const double* ti = qp + 6 * i;
-            eaes = 0.5 * (qi * v0 + mi0 * d0 + mi1 * d1 + mi2 * d2 + ti[0] * w0 + ti[1] * w1 +
-                          ti[2] * w2 + ti[3] * w3 + ti[4] * w4 + ti[5] * w5);
+            eaes = 0.5 * (qi * v0 + mi0 * d0 + mi1 * d1 + mi2 * d2 + ti[0] * w0 + ti[1] * w1 + ti[2] * w2 +
+                          ti[3] * w3 + ti[4] * w4 + ti[5] * w5);
             const double dk = ei.dkernel, qk = ei.qkernel;
             eaxc = dk * (mi0 * mi0 + mi1 * mi1 + mi2 * mi2) +
                    qk * (ti[0] * ti[0] + ti[2] * ti[2] + ti[5] * ti[5] +
@@ -739,36 +1127,37 @@ QX_DEV void potentials(const SysInfo& si, const BatchPtrs& B, SysShared& ss, con
             ss.vat[i] = v0;
         }
     } else {
-        const int t0 = tid - 64, nt = kNT - 64;
-        const double* WD = B.wd4 + si.d4_off;
-        for (int k = t0; k < nd; k += nt) {
+        const int len = (nat + nseg - 1) / nseg;
+        for (int p = tid - 64; p < nseg * nd; p += nu) {
+            const int seg = p / nd, k = p - seg * nd;
+            const int i = ss.refat[k];
+            const double* t = tt + (ss.eroff[ss.sel[i]] + k - ss.refoff[i]) * nat;
+            const double* dsp = pk + 2 * nn + i;
+            const int j1 = (seg + 1) * len < nat ? (seg + 1) * len : nat;
             double y = 0.0;
-#pragma unroll 16
-            for (int l = 0; l < nd; ++l) y += WD[(size_t)l * nd + k] * ss.zr[l];
-            ss.yr[k] = y;
+            constexpr int NJ = 8;
+            for (int j0 = seg * len; j0 < j1; j0 += NJ) {
+                double ds[NJ];
+#pragma unroll
+                for (int u = 0; u < NJ; ++u) ds[u] = dsp[(j0 + u < j1 ? j0 + u : j0) * nat];
+                qx_sched_fence();
+#pragma unroll
+                for (int u = 0; u < NJ; ++u)
+                    if (j0 + u < j1) y += ds[u] * t[j0 + u];
+            }
+            py[p] = y;
             ed4 += -0.5 * ss.zr[k] * y;
-        }
-        // the shell Coulomb rows on the threads the D4 rows leave free
-        const double* G = B.gam + si.gam_off;
-        const int ga = nd + nsh <= nt ? nd : 0;
-        for (int a = t0 - ga; a < nsh; a += nt) {
-            if (a < 0) break;
-            double v = 0.0;
-#pragma unroll 8
-            for (int b = 0; b < nsh; ++b) v += G[(size_t)b * nsh + a] * qsh[b];
-            const double q = qsh[a];
-            const double g3 = g_tab.e[ss.sh[a].el].third[ss.sh[a].k];
-            es2 += 0.5 * q * v;
-            es3 += g3 * q * q * q / 3.0;
-            vs[a] = v + g3 * q * q;
         }
     }
     __syncthreads();
-    QX_PT(22, pt);
     for (int a = tid; a < nsh; a += kNT) {
         const int at = ss.sh[a].at;
         double vdisp = 0.0;
-        for (int k = ss.refoff[at]; k < ss.refoff[at + 1]; ++k) vdisp += -ss.dzr[k] * ss.yr[k];
+        for (int k = ss.refoff[at]; k < ss.refoff[at + 1]; ++k) {
+            double y = py[k];
+            for (int s = 1; s < nseg; ++s) y += py[s * nd + k];
+            vdisp += -ss.dzr[k] * y;
+        }
         vs[a] += ss.vat[at] + vdisp;
     }
     double e5[5] = {es2, es3, eaes, eaxc, ed4};
@@ -776,13 +1165,11 @@ QX_DEV void potentials(const SysInfo& si, const BatchPtrs& B, SysShared& ss, con
     if (tid == 0)
         for (int k = 0; k < 5; ++k) ss.eparts[k] = e5[k];
     __syncthreads();
-    QX_PT(23, pt);
-    QX_PT_FLUSH(pt);
 }
 
-QX_DEV void load_system(const SysInfo& si, const BatchPtrs& B, SysShared& ss)
+QX_DEV void load_system(const SysInfo& si, BatchRef B, SysShared& ss)
 {
-    const int tid = threadIdx.x, nt = blockDim.x, nat = si.nat;
+    const int tid = qx_tid(), nt = blockDim.x, nat = si.nat;
     for (int i = tid; i < 3 * nat; i += nt) ss.sx[i] = B.xyz[3 * (size_t)si.atom_off + i];
     for (int i = tid; i < nat; i += nt) {
         ss.sel[i] = B.elem[si.atom_off + i];
@@ -791,11 +1178,14 @@ QX_DEV void load_system(const SysInfo& si, const BatchPtrs& B, SysShared& ss)
     build_shell_tables(si, B.elem, ss.sh, ss.ao_at, ss.ao_sh);
     if (tid == 0) {
         int o = 0, so = 0, ao = 0;
+        unsigned present = 0;
         for (int a = 0; a < nat; ++a) {
             const ElemParams& e = g_tab.e[ss.sel[a]];
+            present |= 1u << ss.sel[a];
             ss.refoff[a] = o;
             ss.shoff[a] = so;
             ss.aooff[a] = ao;
+            for (int r = 0; r < e.nref; ++r) ss.refat[o + r] = (unsigned char)a;
             o += e.nref;
             so += e.nsh;
             ao += (e.nsh == 2) ? 4 : 1;
@@ -803,6 +1193,12 @@ QX_DEV void load_system(const SysInfo& si, const BatchPtrs& B, SysShared& ss)
         ss.refoff[nat] = o;
         ss.shoff[nat] = so;
         ss.aooff[nat] = ao;
+        o = 0;
+        for (int e = 0; e < gfn2::kElem; ++e) {
+            ss.eroff[e] = o;
+            if (present >> e & 1) o += g_tab.e[e].nref;
+        }
+        ss.eroff[gfn2::kElem] = o;
     }
     __syncthreads();
 }
@@ -811,222 +1207,362 @@ struct SccBuffers {
     double *A, *C, *F, *P;  // m x m working matrices (LDS or global), leading dimension ld
     double* rs;             // kRs row sums per AO
     int ld;
-    double* E;              // fifth m x m matrix for the MFMA eigen refinement, or null
+    double* E;              // fifth m x m matrix (with LDS matrices: or null)
+    double* lds;            // LDS that is free while xin is updated (with LDS matrices from A on)
+    int nlds;               // its size in doubles
+    double* pot;            // LDS that is free while the potentials are taken (pot_lds doubles)
 };
 
-template <bool FAST, bool EIG>
-QX_DEV void scc_body(int sys, const SysInfo& si, const BatchPtrs& B, const SccOpts& opt, SysShared& ss,
-                     SccBuffers bf, double* xin, double* xout, double* vs, double* vd, double* vq,
-                     double* eps, double* focc, double* f2, double2* rot, int2* rpq, double* s_e,
-                     int* s_any)
+// LDS of one system's SCC
+struct SccLds {
+    SysShared ss;
+    double xin[kMaxNx], xout[kMaxNx], vs[QX_MAX_NSH], vd[3 * QX_MAX_NAT], vq[6 * QX_MAX_NAT];
+    double eps[QX_MAX_NAO], focc[QX_MAX_NAO], f2[QX_MAX_NAO];
+    double s_e[4];
+};
+
+// Modified Broyden update (Johnson) of xin from dq = xout - xin, which is left
+// in xout; it: SCC iteration, hcount: secant pairs seen so far.
+QX_DEV void broyden_step(const SysInfo& si, double* hist, OptRef opt, const SccBuffers& bf, double* xin,
+                         double* xout, double* gm, double* red, int it, int& hcount)
 {
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = qx_tid(), lane = tid & 63, wave = qx_wave(tid);
+    const int nx = si.nx, mem = opt.mem;
+    double* hdf = hist;
+    double* hu = hist + (size_t)mem * nx;
+    double* ha = hist + 2 * (size_t)mem * nx;
+    double* hom = ha + mem * mem;
+    double* hql = hom + mem;
+    double* hdql = hql + nx;
+    double* hbeta = hdql + nx;
+    // secant pairs form a ring of `ring` slots; with opt.keep > 0 a warm
+    // start continues from the pairs of the previous call
+    const int ring = (opt.keep > 0 && opt.keep < mem) ? opt.keep : mem;
+    if (it == 1 && hcount == 0) {
+        for (int i = tid; i < nx; i += kNT) {
+            const double dq = xout[i] - xin[i];
+            hdql[i] = dq;
+            hql[i] = xin[i];
+            xin[i] = xin[i] + opt.damp * dq;
+        }
+        __syncthreads();
+        return;
+    }
+    // a new secant pair from this call's previous iterate (it >= 2) into
+    // ring slot k1; on the first iteration of a continued call only the
+    // kept pairs enter
+    const bool add = it >= 2;
+    const int k1 = hcount % ring;
+    if (add) {
+        double nr[2] = {0.0, 0.0};
+        for (int i = tid; i < nx; i += kNT) {
+            const double dq = xout[i] - xin[i];
+            xout[i] = dq;
+            const double d = dq - hdql[i];
+            hdf[k1 * nx + i] = d;
+            nr[0] += d * d;
+            nr[1] += dq * dq;
+        }
+        block_sums<2>(nr, red);
+        const double inv = nr[0] > 0.0 ? 1.0 / sqrt(nr[0]) : 0.0;
+        for (int i = tid; i < nx; i += kNT) {
+            const double d = hdf[k1 * nx + i] * inv;
+            hdf[k1 * nx + i] = d;
+            hu[k1 * nx + i] = opt.damp * d + inv * (xin[i] - hql[i]);
+        }
+        if (tid == 0) {
+            double w = sqrt(nr[1]);
+            w = (w > 0.01 / 100000.0) ? 0.01 / w : 100000.0;
+            if (w < 1.0) w = 1.0;
+            hom[k1] = w;
+        }
+        ++hcount;
+    } else {
+        for (int i = tid; i < nx; i += kNT) xout[i] = xout[i] - xin[i];
+    }
+    const int it1 = hcount < ring ? hcount : ring;  // live pairs
+    __syncthreads();
+    // dot products df_i . df_k1 and df_i . dq: wavefront per i
+    for (int i = wave; i < it1; i += kNT / 64) {
+        double s = 0.0, c = 0.0;
+        for (int j = lane; j < nx; j += 64) {
+            const double di = hdf[i * nx + j];
+            if (add) s += di * hdf[k1 * nx + j];
+            c += di * xout[j];
+        }
+        s = wave_sum(s);
+        c = wave_sum(c);
+        if (lane == 0) {
+            if (add) {
+                ha[i * mem + k1] = s;
+                ha[k1 * mem + i] = s;
+            }
+            gm[i] = c;
+        }
+    }
+    __syncthreads();
+    // (w0^2 I + diag(om) a diag(om)) x = diag(om) c and the weights
+    // diag(om) x, in LDS when the matrix and the right-hand side below it
+    // fit, else in global memory
+    auto solve = [&](double* bt, int st) {
+        for (int p = tid; p < (it1 + 1) * it1; p += kNT) {
+            const int i = p / it1, j = p - i * it1;
+            bt[i * st + j] = i == it1 ? hom[j] * gm[j] : hom[i] * hom[j] * ha[i * mem + j] + (i == j ? 1e-4 : 0.0);
+        }
+        __syncthreads();
+        broyden_solve(bt, st, gm, it1);
+    };
+    if ((it1 + 1) * (it1 | 1) <= bf.nlds) solve(bf.lds, it1 | 1);
+    else solve(hbeta, mem);
+    for (int j = tid; j < nx; j += kNT) {
+        const double dq = xout[j];
+        double q = xin[j];
+        hdql[j] = dq;
+        hql[j] = q;
+        q += opt.damp * dq;
+        for (int i0 = 0; i0 < it1; i0 += 8) {
+            double u[8], w[8];
+#pragma unroll
+            for (int v = 0; v < 8; ++v) {
+                const int i = i0 + v < it1 ? i0 + v : i0;
+                u[v] = hu[i * nx + j];
+                w[v] = hom[i];
+            }
+            qx_sched_fence();
+#pragma unroll
+            for (int v = 0; v < 8; ++v)
+                if (i0 + v < it1) q -= gm[i0 + v] * w[v] * u[v];
+        }
+        xin[j] = q;
+    }
+    __syncthreads();
+}
+
+template <bool FAST, bool EIG>
+QX_DEV void scc_body(int sys, const SysInfo& si, BatchRef B0, OptRef opt, SysShared& ss, SccBuffers bf,
+                     SccLds& L)
+{
     const int nat = si.nat, nsh = si.nsh, n = si.nao, ld = si.ld, nx = si.nx;
     const int m = (n + 1) & ~1;
     const int lb = bf.ld;
-    const size_t ms = (size_t)ld * ld;
-    const double* S = B.S + si.mat_off;
-    const double* H = B.H0 + si.mat_off;
-    const double* Dm = B.D + 3 * si.mat_off;  // transposed: (mu, nu) at nu * ld + mu
-    const double* Qm = B.Q + 6 * si.mat_off;
-    double* xg = B.x + si.x_off;
-    double* xp = B.xprev + si.x_off;    // converged moments of the step before
-    double* xpp = B.xprev2 + si.x_off;  // and of the one before that
-    double* xp3 = B.xprev3 + si.x_off;  // and of the one before that
-    double* xp4 = B.xprev4 + si.x_off;  // and of the one before that
-    const int warm = B.warm[sys];
+    const int ms = ld * ld;
+    const int warm = qx_uniform(B0.warm[sys]);
     double* A = bf.A;
     double* Cc = bf.C;
     double* Ft = bf.F;
     double* P = bf.P;
     double* rs = bf.rs;
+    double* xin = L.xin;
+    double* xout = L.xout;
+    double *vs = L.vs, *vd = L.vd, *vq = L.vq;
+    double* eps = L.eps;
+    double* f2 = L.f2;
 
     QX_PH_INIT
-    // initial moments (polynomial extrapolation of order 1-4 over the
-    // previous steps' converged moments in MD) and basis C = X U (padding
-    // column zero)
-    for (int i = tid; i < nx; i += kNT) {
-        double v = 0.0;
-        if (warm >= 5 && opt.extrapolate >= 4)
-            v = 5.0 * (xg[i] - xp3[i]) - 10.0 * (xp[i] - xpp[i]) + xp4[i];
-        else if (warm >= 4 && opt.extrapolate >= 3) v = 4.0 * (xg[i] + xpp[i]) - 6.0 * xp[i] - xp3[i];
-        else if (warm >= 3 && opt.extrapolate >= 2) v = 3.0 * (xg[i] - xp[i]) + xpp[i];
-        else if (warm >= 2 && opt.extrapolate >= 1) v = 2.0 * xg[i] - xp[i];
-        else if (warm >= 1) v = xg[i];
-        xin[i] = v;
-        if (warm >= 4) xp4[i] = xp3[i];
-        if (warm >= 3) xp3[i] = xpp[i];
-        if (warm >= 2) xpp[i] = xp[i];
-        if (warm >= 1) xp[i] = xg[i];
-    }
-    if (warm) {
-        mfma_gemm<false, false>(n, n, n, B.X + si.mat_off, ld, B.U + si.mat_off, ld, Cc, lb, nullptr);
-    } else {
+    {
+        // initial moments (polynomial extrapolation of order 1-4 over the
+        // previous steps' converged moments in MD) and basis C = X U (padding
+        // column zero)
+        BatchRef B = qx_fresh(B0);
+        const int tid = qx_tid();
+        double* xg = B.x + si.x_off;
+        double* xp = B.xprev + si.x_off;    // converged moments of the step before
+        double* xpp = B.xprev2 + si.x_off;  // and of the one before that
+        double* xp3 = B.xprev3 + si.x_off;  // and of the one before that
+        double* xp4 = B.xprev4 + si.x_off;  // and of the one before that
+        for (int i = tid; i < nx; i += kNT) {
+            double v = 0.0;
+            if (warm >= 5 && opt.extrapolate >= 4)
+                v = 5.0 * (xg[i] - xp3[i]) - 10.0 * (xp[i] - xpp[i]) + xp4[i];
+            else if (warm >= 4 && opt.extrapolate >= 3) v = 4.0 * (xg[i] + xpp[i]) - 6.0 * xp[i] - xp3[i];
+            else if (warm >= 3 && opt.extrapolate >= 2) v = 3.0 * (xg[i] - xp[i]) + xpp[i];
+            else if (warm >= 2 && opt.extrapolate >= 1) v = 2.0 * xg[i] - xp[i];
+            else if (warm >= 1) v = xg[i];
+            xin[i] = v;
+            if (warm >= 4) xp4[i] = xp3[i];
+            if (warm >= 3) xp3[i] = xpp[i];
+            if (warm >= 2) xpp[i] = xp[i];
+            if (warm >= 1) xp[i] = xg[i];
+        }
         const double* X = B.X + si.mat_off;
-        for (int p = tid; p < n * n; p += kNT) Cc[(size_t)(p / n) * lb + p % n] = X[(size_t)(p / n) * ld + p % n];
+        if (warm) {
+            mfma_gemm(n, n, n, X, ld, 1, B.U + si.mat_off, ld, 1, Cc, lb, nullptr);
+        } else {
+            for (int p = tid; p < n * n; p += kNT) Cc[(p / n) * lb + p % n] = X[(p / n) * ld + p % n];
+        }
+        if (m > n)
+            for (int i = tid; i < n; i += kNT) Cc[i * lb + n] = 0.0;
+        if (tid == 0) L.s_e[1] = -1e300;
     }
-    if (m > n)
-        for (int i = tid; i < n; i += kNT) Cc[(size_t)i * lb + n] = 0.0;
-    if (tid == 0) s_e[1] = -1e300;
     __syncthreads();
     QX_PH(11);
 
-    double* hist = B.hist + si.hist_off;
-    const int mem = opt.mem;
-    double* hdf = hist;
-    double* hu = hist + (size_t)mem * nx;
-    double* ha = hist + 2 * (size_t)mem * nx;
-    double* hom = ha + (size_t)mem * mem;
-    double* hql = hom + mem;
-    double* hdql = hql + nx;
-    double* hbeta = hdql + nx;
-    double* hgam = hbeta + (size_t)mem * mem;
-    // secant pairs form a ring of `ring` slots; with opt.keep > 0 a warm
-    // start continues from the pairs of the previous call (count in hcnt)
-    const int ring = (opt.keep > 0 && opt.keep < mem) ? opt.keep : mem;
-    double* hcnt = hgam + mem;
-    int hcount = (opt.keep > 0 && warm >= 1) ? (int)hcnt[0] : 0;
-
+    int hcount = 0;
+    if (opt.keep > 0 && warm >= 1) {
+        const double* hcnt = B0.hist + si.hist_off + 2 * (size_t)opt.mem * nx + 2 * (size_t)opt.mem * opt.mem +
+                             2 * (size_t)opt.mem + 2 * (size_t)nx;
+        hcount = qx_uniform((int)hcnt[0]);
+    }
     const double nalpha = 0.5 * si.nel;
     double eold = 0.0, etot = 0.0, ts = 0.0, eband = 0.0, errp = 1e-3;
     int it = 1, conv = 0;
-    for (; it <= opt.maxiter; ++it) {
-        potentials(si, B, ss, xin, vs, vd, vq);
-        QX_PH(0);
-        // G^T (row nu holds G_{mu nu} over mu), then F = H0 - (G + G^T) / 2
-        for (int mu = lane; mu < n; mu += 64) {
-            const int am = ss.ao_at[mu];
-            const double w0 = vs[ss.ao_sh[mu]], w1 = vd[3 * am], w2 = vd[3 * am + 1],
-                         w3 = vd[3 * am + 2];
-            const double* q = vq + 6 * am;
-            const double w4 = q[0], w5 = q[1], w6 = q[2], w7 = q[3], w8 = q[4], w9 = q[5];
-            for (int nu0 = wave; nu0 < n; nu0 += 4 * (kNT / 64)) {
-                double g[4];
+    // each iteration takes the potentials twice, at the input and at the
+    // output moments (one copy of their code)
+    for (bool out = false;; out = !out) {
+        potentials(si, qx_fresh(B0), ss, out ? xout : xin, vs, vd, vq, bf.pot);
+        if (!out) {
+            QX_PH(0);
+            {
+                // G^T (row nu holds G_{mu nu} over mu), then F = H0 - (G + G^T) / 2
+                BatchRef B = qx_fresh(B0);
+                const double* S = B.S + si.mat_off;
+                const double* H = B.H0 + si.mat_off;
+                const double* Dm = B.D + 3 * si.mat_off;  // transposed: (mu, nu) at nu * ld + mu
+                const double* Qm = B.Q + 6 * si.mat_off;
+                const int tid = qx_tid(), wave = qx_wave(tid);
+                constexpr int NU = 3;  // rows per batch of loads
+                for (int mu = tid & 63; mu < n; mu += 64) {
+                    const int am = ss.ao_at[mu];
+                    const double w0 = vs[ss.ao_sh[mu]], w1 = vd[3 * am], w2 = vd[3 * am + 1], w3 = vd[3 * am + 2];
+                    const double* q = vq + 6 * am;
+                    const double w4 = q[0], w5 = q[1], w6 = q[2], w7 = q[3], w8 = q[4], w9 = q[5];
+                    for (int nu0 = wave; nu0 < n; nu0 += NU * (kNT / 64)) {
+                        double g[NU][10];
 #pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    const int nu = nu0 + u * (kNT / 64);
-                    const size_t o = (size_t)(nu < n ? nu : 0) * ld + mu;
-                    g[u] = S[o] * w0 + Dm[o] * w1 + Dm[ms + o] * w2 + Dm[2 * ms + o] * w3 +
-                           Qm[o] * w4 + Qm[ms + o] * w5 + Qm[2 * ms + o] * w6 +
-                           Qm[3 * ms + o] * w7 + Qm[4 * ms + o] * w8 + Qm[5 * ms + o] * w9;
-                }
+                        for (int u = 0; u < NU; ++u) {
+                            const int nu = nu0 + u * (kNT / 64);
+                            const int o = (nu < n ? nu : nu0) * ld + mu;
+                            g[u][0] = S[o];
 #pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    const int nu = nu0 + u * (kNT / 64);
-                    if (nu < n) Ft[(size_t)nu * lb + mu] = g[u];
-                }
-            }
-        }
-        __syncthreads();
-        for (int p = tid; p < n * n; p += kNT) {
-            const int mu = p / n, nu = p % n;
-            if (nu < mu) continue;
-            const double gmn = Ft[(size_t)mu * lb + nu], gnm = Ft[(size_t)nu * lb + mu];
-            const double f = H[(size_t)mu * ld + nu] - 0.5 * (gmn + gnm);
-            Ft[(size_t)mu * lb + nu] = f;
-            Ft[(size_t)nu * lb + mu] = f;
-        }
-        __syncthreads();
-        QX_PH(1);
-        // A = C^T F C (F C staged in the density buffer)
-        mfma_gemm<false, false>(n, n, n, Ft, lb, Cc, lb, P, lb, nullptr);
-        __syncthreads();
-        mfma_gemm<true, false>(n, n, n, Cc, lb, P, lb, A, lb, nullptr);
-        if (m > n)
-            for (int j = tid; j < m; j += kNT) {
-                A[(size_t)n * lb + j] = 0.0;
-                A[(size_t)j * lb + n] = 0.0;
-            }
-        __syncthreads();
-        QX_PH(2);
-        double jtol = fmin(1e-6, 1e-3 * errp);
-        if (jtol < opt.jacobi_tol) jtol = opt.jacobi_tol;
-        int nsweep = 0;
-        if (EIG && bf.E && eig_rotate(A, Cc, m, n, lb, jtol, 3, Ft, P, bf.E, ss.red, rot, rpq, s_any)) {
-            QX_PH_ADD(15, 1);
-        } else {
-            nsweep = jacobi(A, Cc, m, n, lb, jtol, 50, rot, rpq, ss.red, s_any);
-        }
-        QX_PH(3);
-        QX_PH_ADD(12, nsweep);
-        (void)nsweep;
-        for (int i = tid; i < n; i += kNT) eps[i] = A[(size_t)i * lb + i];
-        __syncthreads();
-        if (tid < 64) {
-            double mu = s_e[1];
-            int fit = 0;
-            const double t = fermi_wave(n, eps, si.kt, nalpha, focc, mu, fit);
-            if (tid == 0) {
-                s_e[0] = t;
-                s_e[1] = mu;
-            }
-            QX_PH_ADD(14, fit);
-            (void)fit;
-            for (int i = tid; i < n; i += 64) f2[i] = 2.0 * focc[i];
-        }
-        __syncthreads();
-        ts = s_e[0];
-        QX_PH(4);
-        mfma_gemm<false, true>(n, n, n, Cc, lb, Cc, lb, P, lb, f2);
-        __syncthreads();
-        QX_PH(5);
-        // row sums of P o M for M = S, D (3), Q (6), H0 as coalesced column
-        // sweeps: wavefront w takes the matrices w, w + 4, w + 8 for all AOs,
-        // so every lane keeps three independent sums (in nu order) and three
-        // times the loads in flight of one sum per thread
-        {
-            static_assert(kNT == 256 && kRs <= 12, "three row-sum matrices per wavefront");
-            const int c0 = wave, c1 = wave + 4, c2 = wave + 8;
-            const bool has2 = c2 < kRs;
-            const double* M0 = c0 == 0 ? S : Dm + (size_t)(c0 - 1) * ms;
-            const double* M1 = Qm + (size_t)(c1 - 4) * ms;
-            const double* M2 = !has2 ? M1 : c2 < 10 ? Qm + (size_t)(c2 - 4) * ms : H;
-            for (int mu = lane; mu < n; mu += 64) {
-                double a0 = 0.0, a1 = 0.0, a2 = 0.0;
-                if (has2) {
-#pragma unroll 8
-                    for (int nu = 0; nu < n; ++nu) {
-                        const double p = P[(size_t)nu * lb + mu];
-                        const size_t o = (size_t)nu * ld + mu;
-                        a0 += p * M0[o];
-                        a1 += p * M1[o];
-                        a2 += p * M2[o];
-                    }
-                } else {
-#pragma unroll 8
-                    for (int nu = 0; nu < n; ++nu) {
-                        const double p = P[(size_t)nu * lb + mu];
-                        const size_t o = (size_t)nu * ld + mu;
-                        a0 += p * M0[o];
-                        a1 += p * M1[o];
+                            for (int c = 0; c < 3; ++c) g[u][1 + c] = Dm[c * ms + o];
+#pragma unroll
+                            for (int c = 0; c < 6; ++c) g[u][4 + c] = Qm[c * ms + o];
+                        }
+                        qx_sched_fence();
+#pragma unroll
+                        for (int u = 0; u < NU; ++u) {
+                            const int nu = nu0 + u * (kNT / 64);
+                            if (nu < n)
+                                Ft[nu * lb + mu] = g[u][0] * w0 + g[u][1] * w1 + g[u][2] * w2 + g[u][3] * w3 +
+                                                   g[u][4] * w4 + g[u][5] * w5 + g[u][6] * w6 + g[u][7] * w7 +
+                                                   g[u][8] * w8 + g[u][9] * w9;
+                        }
                     }
                 }
-                rs[(size_t)mu * kRs + c0] = a0;
-                rs[(size_t)mu * kRs + c1] = a1;
-                if (has2) rs[(size_t)mu * kRs + c2] = a2;
+                __syncthreads();
+                for (int p = tid; p < n * n; p += kNT) {
+                    const int mu = p / n, nu = p - mu * n;
+                    if (nu < mu) continue;
+                    const double gmn = Ft[mu * lb + nu], gnm = Ft[nu * lb + mu];
+                    const double f = H[mu * ld + nu] - 0.5 * (gmn + gnm);
+                    Ft[mu * lb + nu] = f;
+                    Ft[nu * lb + mu] = f;
+                }
+                __syncthreads();
             }
+            QX_PH(1);
+            // A = C^T F C (F C staged in the density buffer)
+            for (int s = 0; s < 2; ++s) {
+                mfma_gemm(n, n, n, s ? Cc : Ft, s ? 1 : lb, s ? lb : 1, s ? P : Cc, lb, 1, s ? A : P, lb, nullptr);
+                if (s && m > n)
+                    for (int j = qx_tid(); j < m; j += kNT) {
+                        A[n * lb + j] = 0.0;
+                        A[j * lb + n] = 0.0;
+                    }
+                __syncthreads();
+            }
+            QX_PH(2);
+            double jtol = fmin(1e-6, 1e-3 * errp);
+            if (jtol < opt.jacobi_tol) jtol = opt.jacobi_tol;
+            const int nblk = (m / 2) * (m / 2 + 1) / 2;
+            const bool blk_lds = FAST || (4 * nblk <= bf.nlds && nblk <= 6 * (kNT - 64));
+            const JacobiBuffers jb{FAST ? Ft : bf.lds, {Ft, bf.E}, (double2*)P, (double2*)ss.rot, ss.any, ss.red, blk_lds};
+            const int nsweep = eig_solve<EIG, FAST>(A, Cc, m, n, lb, jtol, Ft, P, bf.E, jb);
+            QX_PH(3);
+            QX_PH_ADD(12, nsweep);
+            QX_PH_ADD(15, nsweep == 0);
+            (void)nsweep;
+            const int tid = qx_tid();
+            for (int i = tid; i < n; i += kNT) eps[i] = A[i * lb + i];
+            __syncthreads();
+            if (tid < 64) {
+                double mu = L.s_e[1];
+                int fit = 0;
+                const double t = fermi_wave(n, eps, si.kt, nalpha, L.focc, mu, fit);
+                if (tid == 0) {
+                    L.s_e[0] = t;
+                    L.s_e[1] = mu;
+                }
+                QX_PH_ADD(14, fit);
+                (void)fit;
+                for (int i = tid; i < n; i += 64) f2[i] = 2.0 * L.focc[i];
+            }
+            __syncthreads();
+            ts = L.s_e[0];
+            QX_PH(4);
+            mfma_gemm(n, n, n, Cc, lb, 1, Cc, 1, lb, P, lb, f2);
+            __syncthreads();
+            QX_PH(5);
+            // row sums of P o M for M = S, D (3), Q (6), H0 as coalesced column
+            // sweeps over all AOs (lanes), the matrices dealt over the wavefronts
+            {
+                static_assert(kNT / 64 >= (kRs + 1) / 2, "at most two row-sum matrices per wavefront");
+                BatchRef B = qx_fresh(B0);
+                const int tid = qx_tid(), lane = tid & 63, c0 = qx_wave(tid), c1 = c0 + kNT / 64;
+                auto mat = [&](int c) {
+                    return c == 0 ? B.S + si.mat_off
+                           : c < 4 ? B.D + 3 * si.mat_off + (c - 1) * ms
+                           : c < 10 ? B.Q + 6 * si.mat_off + (c - 4) * ms
+                                    : B.H0 + si.mat_off;
+                };
+                const double* M0 = mat(c0);
+                const double* M1 = mat(c1 < kRs ? c1 : c0);
+                constexpr int NU = 10;  // rows per batch of loads
+                for (int mu = lane; mu < n; mu += 64) {
+                    double a0 = 0.0, a1 = 0.0;
+                    for (int nu0 = 0; nu0 < n; nu0 += NU) {
+                        double x0[NU], x1[NU];
+#pragma unroll
+                        for (int u = 0; u < NU; ++u) {
+                            const int o = (nu0 + u < n ? nu0 + u : nu0) * ld + mu;
+                            x0[u] = M0[o];
+                            if (c1 < kRs) x1[u] = M1[o];
+                        }
+                        qx_sched_fence();
+#pragma unroll
+                        for (int u = 0; u < NU; ++u)
+                            if (nu0 + u < n) {
+                                const double p = P[(nu0 + u) * lb + mu];
+                                a0 += p * x0[u];
+                                if (c1 < kRs) a1 += p * x1[u];
+                            }
+                    }
+                    rs[mu * kRs + c0] = a0;
+                    if (c1 < kRs) rs[mu * kRs + c1] = a1;
+                }
+            }
+            __syncthreads();
+            for (int s = tid; s < nsh; s += kNT) {
+                const ShellDesc d = ss.sh[s];
+                double pop = 0.0;
+                for (int a = 0; a < d.nao; ++a) pop += rs[(d.ao0 + a) * kRs];
+                xout[s] = g_tab.e[d.el].refocc[d.k] - pop;
+            }
+            for (int t = tid; t < 9 * nat; t += kNT) {
+                const int a = t / 9, c = t % 9;
+                double v = 0.0;
+                for (int mu = ss.aooff[a]; mu < ss.aooff[a + 1]; ++mu) v += rs[mu * kRs + 1 + c];
+                if (c < 3) xout[nsh + 3 * a + c] = -v;
+                else xout[nsh + 3 * nat + 6 * a + (c - 3)] = -v;
+            }
+            __syncthreads();
+            QX_PH(6);
+            continue;
         }
-        __syncthreads();
-        for (int s = tid; s < nsh; s += kNT) {
-            const ShellDesc d = ss.sh[s];
-            double pop = 0.0;
-            for (int a = 0; a < d.nao; ++a) pop += rs[(size_t)(d.ao0 + a) * kRs];
-            xout[s] = g_tab.e[d.el].refocc[d.k] - pop;
-        }
-        for (int t = tid; t < 9 * nat; t += kNT) {
-            const int a = t / 9, c = t % 9;
-            double v = 0.0;
-            for (int mu = ss.aooff[a]; mu < ss.aooff[a + 1]; ++mu) v += rs[(size_t)mu * kRs + 1 + c];
-            if (c < 3) xout[nsh + 3 * a + c] = -v;
-            else xout[nsh + 3 * nat + 6 * a + (c - 3)] = -v;
-        }
-        double red2[2] = {0.0, 0.0};
-        for (int mu = tid; mu < n; mu += kNT) red2[0] += rs[(size_t)mu * kRs + 10];
-        __syncthreads();
-        QX_PH(6);
-        potentials(si, B, ss, xout, vs, vd, vq);
         QX_PH(7);
-        for (int i = tid; i < nx; i += kNT) {
+        double red2[2] = {0.0, 0.0};
+        for (int mu = qx_tid(); mu < n; mu += kNT) red2[0] += rs[mu * kRs + 10];
+        for (int i = qx_tid(); i < nx; i += kNT) {
             const double dd = xout[i] - xin[i];
             red2[1] += dd * dd;
         }
@@ -1037,141 +1573,27 @@ QX_DEV void scc_body(int sys, const SysInfo& si, const BatchPtrs& B, const SccOp
         errp = err;
         const double de = etot - eold;
         eold = etot;
-        if (it > 1 && fabs(de) < opt.econv && err < opt.pconv) {
+        if (qx_uniform(it > 1 && fabs(de) < opt.econv && err < opt.pconv)) {
             conv = 1;
             break;
         }
         if (it == opt.maxiter) break;
         QX_PH(8);
-        // modified Broyden update of xin with dq = xout - xin (stored into xout)
-        if (it == 1 && hcount == 0) {
-            for (int i = tid; i < nx; i += kNT) {
-                const double dq = xout[i] - xin[i];
-                hdql[i] = dq;
-                hql[i] = xin[i];
-                xin[i] = xin[i] + opt.damp * dq;
-            }
-            __syncthreads();
-            QX_PH(9);
-            continue;
-        }
-        // a new secant pair from this call's previous iterate (it >= 2) into
-        // ring slot k1; on the first iteration of a continued call only the
-        // kept pairs enter
-        const bool add = it >= 2;
-        const int k1 = hcount % ring;
-        if (add) {
-            double nr[2] = {0.0, 0.0};
-            for (int i = tid; i < nx; i += kNT) {
-                const double dq = xout[i] - xin[i];
-                xout[i] = dq;
-                const double d = dq - hdql[i];
-                hdf[(size_t)k1 * nx + i] = d;
-                nr[0] += d * d;
-                nr[1] += dq * dq;
-            }
-            block_sums<2>(nr, ss.red);
-            const double inv = nr[0] > 0.0 ? 1.0 / sqrt(nr[0]) : 0.0;
-            for (int i = tid; i < nx; i += kNT) {
-                const double d = hdf[(size_t)k1 * nx + i] * inv;
-                hdf[(size_t)k1 * nx + i] = d;
-                hu[(size_t)k1 * nx + i] = opt.damp * d + inv * (xin[i] - hql[i]);
-            }
-            if (tid == 0) {
-                double w = sqrt(nr[1]);
-                w = (w > 0.01 / 100000.0) ? 0.01 / w : 100000.0;
-                if (w < 1.0) w = 1.0;
-                hom[k1] = w;
-            }
-            ++hcount;
-        } else {
-            for (int i = tid; i < nx; i += kNT) xout[i] = xout[i] - xin[i];
-        }
-        const int it1 = hcount < ring ? hcount : ring;  // live pairs
-        __syncthreads();
-        // dot products df_i . df_k1 and df_i . dq: wavefront per i
-        for (int i = wave; i < it1; i += kNT / 64) {
-            double s = 0.0, c = 0.0;
-            for (int j = lane; j < nx; j += 64) {
-                const double di = hdf[(size_t)i * nx + j];
-                if (add) s += di * hdf[(size_t)k1 * nx + j];
-                c += di * xout[j];
-            }
-            s = wave_sum(s);
-            c = wave_sum(c);
-            if (lane == 0) {
-                if (add) {
-                    ha[(size_t)i * mem + k1] = s;
-                    ha[(size_t)k1 * mem + i] = s;
-                }
-                hgam[i] = c;
-            }
-        }
-        __syncthreads();
-        // (w0^2 I + diag(om) a diag(om)) gamma = diag(om) c, Cholesky in LDS
-        // (the Fock buffer is free here) when it fits, else in global memory
-        const bool lds_solve = it1 * (it1 + 2) <= m * m;
-        double* bt = lds_solve ? Ft : hbeta;
-        const int lbt = lds_solve ? it1 : mem;
-        double* gm = lds_solve ? Ft + (size_t)it1 * it1 : hgam;
-        double* om = lds_solve ? gm + it1 : hom;
-        if (lds_solve) {
-            for (int i = tid; i < it1; i += kNT) {
-                om[i] = hom[i];
-                gm[i] = hgam[i];
-            }
-            __syncthreads();
-        }
-        for (int p = tid; p < it1 * it1; p += kNT) {
-            const int i = p / it1, j = p % it1;
-            bt[(size_t)i * lbt + j] = om[i] * om[j] * ha[(size_t)i * mem + j] + (i == j ? 1e-4 : 0.0);
-        }
-        __syncthreads();
-        if (it1 <= kWaveSolve) {
-            if (tid < 64) broyden_solve_wave(bt, lbt, gm, om, it1);
-        } else if (tid == 0) {
-            for (int i = 0; i < it1; ++i) gm[i] *= om[i];
-            for (int j = 0; j < it1; ++j) {
-                double d = bt[(size_t)j * lbt + j];
-                for (int k = 0; k < j; ++k) d -= bt[(size_t)j * lbt + k] * bt[(size_t)j * lbt + k];
-                d = sqrt(d);
-                bt[(size_t)j * lbt + j] = d;
-                for (int i = j + 1; i < it1; ++i) {
-                    double v = bt[(size_t)i * lbt + j];
-                    for (int k = 0; k < j; ++k) v -= bt[(size_t)i * lbt + k] * bt[(size_t)j * lbt + k];
-                    bt[(size_t)i * lbt + j] = v / d;
-                }
-            }
-            for (int i = 0; i < it1; ++i) {
-                double v = gm[i];
-                for (int k = 0; k < i; ++k) v -= bt[(size_t)i * lbt + k] * gm[k];
-                gm[i] = v / bt[(size_t)i * lbt + i];
-            }
-            for (int i = it1 - 1; i >= 0; --i) {
-                double v = gm[i];
-                for (int k = i + 1; k < it1; ++k) v -= bt[(size_t)k * lbt + i] * gm[k];
-                gm[i] = v / bt[(size_t)i * lbt + i];
-            }
-            for (int i = 0; i < it1; ++i) gm[i] *= om[i];
-        }
-        __syncthreads();
-        for (int j = tid; j < nx; j += kNT) {
-            const double dq = xout[j];
-            double q = xin[j];
-            hdql[j] = dq;
-            hql[j] = q;
-            q += opt.damp * dq;
-            for (int i = 0; i < it1; ++i) q -= gm[i] * hu[(size_t)i * nx + j];
-            xin[j] = q;
-        }
-        __syncthreads();
+        broyden_step(si, qx_fresh(B0).hist + si.hist_off, opt, bf, xin, xout, ss.gm, ss.red, it, hcount);
         QX_PH(9);
+        ++it;
     }
-    QX_PH_ADD(13, it > opt.maxiter ? opt.maxiter : it);
-    if (opt.keep > 0 && tid == 0) hcnt[0] = (double)hcount;
+    QX_PH_ADD(13, it);
+    BatchRef B = qx_fresh(B0);
+    const int tid = qx_tid();
+    if (opt.keep > 0 && tid == 0) {
+        double* hcnt = B.hist + si.hist_off + 2 * (size_t)opt.mem * nx + 2 * (size_t)opt.mem * opt.mem +
+                       2 * (size_t)opt.mem + 2 * (size_t)nx;
+        hcnt[0] = (double)hcount;
+    }
     // results: moments, charges, potentials at the output moments
     for (int i = tid; i < nx; i += kNT) {
-        xg[i] = xout[i];
+        B.x[si.x_off + i] = xout[i];
         B.xo[si.x_off + i] = xout[i];
     }
     for (int a = tid; a < nat; a += kNT) B.qat[si.atom_off + a] = ss.qat[a];
@@ -1180,16 +1602,17 @@ QX_DEV void scc_body(int sys, const SysInfo& si, const BatchPtrs& B, const SccOp
     for (int i = tid; i < 6 * nat; i += kNT) B.vq[6 * (size_t)si.atom_off + i] = vq[i];
     for (int i = tid; i < n; i += kNT) {
         B.eps[(size_t)sys * QX_MAX_NAO + i] = eps[i];
-        B.focc[(size_t)sys * QX_MAX_NAO + i] = focc[i];
-        f2[i] = 2.0 * focc[i] * eps[i];
+        B.focc[(size_t)sys * QX_MAX_NAO + i] = L.focc[i];
+        f2[i] = 2.0 * L.focc[i] * eps[i];
     }
-    double* Pg = B.P + si.mat_off;
-    if (P != Pg)
-        for (int p = tid; p < n * n; p += kNT) Pg[(size_t)(p / n) * ld + p % n] = P[(size_t)(p / n) * lb + p % n];
+    if (FAST) {
+        double* Pg = B.P + si.mat_off;
+        for (int p = tid; p < n * n; p += kNT) Pg[(p / n) * ld + p % n] = P[(p / n) * lb + p % n];
+    }
     __syncthreads();
     // W = C diag(2 f e) C^T ; U = L^T C for the next warm start
-    mfma_gemm<false, true>(n, n, n, Cc, lb, Cc, lb, B.W + si.mat_off, ld, f2);
-    mfma_gemm<true, false>(n, n, n, B.L + si.mat_off, ld, Cc, lb, B.U + si.mat_off, ld, nullptr);
+    mfma_gemm(n, n, n, Cc, lb, 1, Cc, 1, lb, B.W + si.mat_off, ld, f2);
+    mfma_gemm(n, n, n, B.L + si.mat_off, 1, ld, Cc, lb, 1, B.U + si.mat_off, ld, nullptr);
     QX_PH(10);
     if (tid == 0) {
         double* ep = B.eparts + 10 * sys;
@@ -1202,62 +1625,53 @@ QX_DEV void scc_body(int sys, const SysInfo& si, const BatchPtrs& B, const SccOp
         ep[8] = ts;
         ep[9] = etot;
         B.energy[sys] = etot + ep[6] + ep[7];
-        const int itn = it > opt.maxiter ? opt.maxiter : it;
-        B.iters[sys] = itn;
-        B.iters_total[sys] += (unsigned long long)itn;
+        B.iters[sys] = it;
+        B.iters_total[sys] += (unsigned long long)it;
         B.status[sys] = conv ? 0 : -1;
         B.warm[sys] = warm >= 5 ? 5 : warm + 1;
     }
 }
 
-// LDS of one system's SCC
-struct SccLds {
-    SysShared ss;
-    double xin[kMaxNx], xout[kMaxNx], vs[QX_MAX_NSH], vd[3 * QX_MAX_NAT], vq[6 * QX_MAX_NAT];
-    double eps[QX_MAX_NAO], focc[QX_MAX_NAO], f2[QX_MAX_NAO];
-    double2 rot[QX_MAX_NAO / 2];
-    int2 rpq[QX_MAX_NAO / 2];
-    double s_e[4];
-    int s_any[2];
-};
-
 // the whole SCC of system sys by the block (dyn: the launch's dynamic LDS)
-//   EIG: with the MFMA eigen refinement (a separate instantiation: the code
-//   alone, even when not taken, costs the Jacobi-only kernel a quarter of
-//   its speed through the scheduling of the shared SCC body)
+//   EIG: with the MFMA eigen refinement
 template <bool EIG>
-QX_DEV void scc_system(const BatchPtrs& B, const SccOpts& opt, int sys, SccLds& L, double* dyn)
+QX_DEV void scc_system(BatchRef B, OptRef opt, int sys, SccLds& L, double* dyn)
 {
-    const SysInfo si = B.info[sys];
+    const SysInfo si = qx_info(B, sys);
     load_system(si, B, L.ss);
     const int m = (si.nao + 1) & ~1;
     if (m <= opt.lds_max_m) {
         // odd leading dimension: column-wise LDS accesses hit distinct banks
-        const size_t mm = (size_t)m * (m + 1);
+        const int mm = m * (m + 1);
         // a fifth matrix after the row sums when the launch's LDS holds it
-        double* E = EIG && 5 * mm + kRs * (size_t)m <= (size_t)opt.lds_doubles ? dyn + 4 * mm + kRs * m
-                                                                            : nullptr;
-        SccBuffers bf{dyn, dyn + mm, dyn + 2 * mm, dyn + 3 * mm, dyn + 4 * mm, m + 1, E};
-        scc_body<true, EIG>(sys, si, B, opt, L.ss, bf, L.xin, L.xout, L.vs, L.vd, L.vq, L.eps, L.focc, L.f2,
-                       L.rot, L.rpq, L.s_e, L.s_any);
+        double* E = EIG && 5 * mm + kRs * m <= opt.lds_doubles ? dyn + 4 * mm + kRs * m : nullptr;
+        // A and F are free at the potentials, P and the row sums are not
+        double* pot = dyn + (pot_lds(si.nat, si.ndim) <= 2 * mm ? mm : 4 * mm + kRs * m);
+        SccBuffers bf{dyn + mm, dyn, dyn + 2 * mm, dyn + 3 * mm, dyn + 4 * mm, m + 1, E, dyn + mm,
+                      opt.lds_doubles - mm, pot};
+        scc_body<true, EIG>(sys, si, B, opt, L.ss, bf, L);
     } else {
-        // the energy-weighted density slot doubles as the row-sum scratch;
-        // the MFMA eigen refinement's fifth matrix is the batch's E slot
-        SccBuffers bf{B.T + si.mat_off, B.C + si.mat_off, B.U + si.mat_off, B.P + si.mat_off,
-                      B.W + si.mat_off, si.ld, EIG ? B.E + si.mat_off : nullptr};
-        scc_body<false, EIG>(sys, si, B, opt, L.ss, bf, L.xin, L.xout, L.vs, L.vd, L.vq, L.eps, L.focc,
-                        L.f2, L.rot, L.rpq, L.s_e, L.s_any);
+        // the energy-weighted density slot doubles as the row-sum scratch
+        SccBuffers bf{B.T + si.mat_off, B.C + si.mat_off, B.U + si.mat_off, B.P + si.mat_off, B.W + si.mat_off,
+                      si.ld, B.E + si.mat_off, dyn, opt.lds_doubles, dyn};
+        scc_body<false, EIG>(sys, si, B, opt, L.ss, bf, L);
     }
 }
 
+struct SccArgs {
+    BatchPtrs B;
+    SccOpts opt;
+};
+
 template <bool EIG>
-__global__ __launch_bounds__(kNT) void k_scc(BatchPtrs B, SccOpts opt)
+__global__ __launch_bounds__(kNT) void k_scc(SccArgs args)
 {
-    const int sys = opt.first_sys + blockIdx.x;
-    if (B.active && !B.active[sys]) return;
+    QX_ARG(SccArgs) a = qx_args(args);
+    const int sys = a.opt.first_sys + blockIdx.x;
+    if (a.B.active && !a.B.active[sys]) return;
     __shared__ SccLds L;
     extern __shared__ double dyn[];
-    scc_system<EIG>(B, opt, sys, L, dyn);
+    scc_system<EIG>(a.B, a.opt, sys, L, dyn);
 }
 
 }  // namespace qx

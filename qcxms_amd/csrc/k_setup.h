@@ -19,6 +19,19 @@ QX_DEV double d4_dzeta(double a, double c, double qref, double qmod)
     return -a * c * e * exp(a * (1.0 - e)) * qref / (qmod * qmod);
 }
 
+// both at once
+QX_DEV void d4_zeta_both(double a, double c, double qref, double qmod, double& z, double& dz)
+{
+    if (qmod < 0.0) {
+        z = exp(a);
+        dz = 0.0;
+        return;
+    }
+    const double e = exp(c * (1.0 - qref / qmod));
+    z = exp(a * (1.0 - e));
+    dz = -a * c * e * z * qref / (qmod * qmod);
+}
+
 // GFN2 coordination-number count and its derivative d(count)/dr
 QX_DEV void gfn_count(double rc, double r, double& f, double& df)
 {
@@ -139,15 +152,14 @@ struct SetupLds {
     double scn[QX_MAX_NAT], scnd4[QX_MAX_NAT];
     int refoff[QX_MAX_NAT + 1];
     double red[QX_BLOCK / 64];
-    // per D4 reference: atom, index within the atom, zeta(q = 0) * gw
-    int refat[QX_MAX_REF * QX_MAX_NAT], refii[QX_MAX_REF * QX_MAX_NAT];
+    // per D4 reference: zeta(q = 0) * gw
     double zg[QX_MAX_REF * QX_MAX_NAT];
 };
 
-QX_DEV void setup_system(const BatchPtrs& B, int sys, int with_chol, SetupLds& Ls, double* dyn)
+QX_DEV void setup_system(BatchRef B, int sys, int with_chol, SetupLds& Ls, double* dyn)
 {
-    const SysInfo si = B.info[sys];
-    const int tid = threadIdx.x;
+    const SysInfo si = qx_info(B, sys);
+    const int tid = qx_tid();
     const int nat = si.nat, nsh = si.nsh, n = si.nao, ld = si.ld;
     ShellDesc* sh = Ls.sh;
     int* ao_at = Ls.ao_at;
@@ -304,72 +316,40 @@ QX_DEV void setup_system(const BatchPtrs& B, int sys, int with_chol, SetupLds& L
         const double eta = 0.5 * (g_tab.e[sh[a].el].hard[sh[a].k] + g_tab.e[sh[b].el].hard[sh[b].k]);
         G[p] = 1.0 / sqrt(dx * dx + dy * dy + dz * dz + 1.0 / (eta * eta));
     }
-    // 6. D4 charge-response matrix wd4[k][l] = gw_k gw_l C6ref_kl disp_ij (i != j):
-    //    the pair damping disp_ij into LDS (the Cholesky slot is free here),
-    //    then one element per thread, coalesced along l
-    const int nd = si.ndim;
-    double* WD = B.wd4 + si.d4_off;
+    // 6. per D4 reference zeta(q = 0) gw, and the kernels of an ordered atom
+    //    pair (i, j) at planes c * nat^2 + j * nat + i: the damped multipole
+    //    kernels 1/r^3 and 1/r^5 and the D4 pair damping, zero for i = j
     const double* gw = B.gw + si.ref_off;
-    double* disp = dyn;  // nat x nat
-    int* refat = Ls.refat;
-    int* refii = Ls.refii;
     double* zg = Ls.zg;
     __syncthreads();
-    for (int k = tid; k < nd; k += QX_BLOCK) {
-        int a = 0;
-        while (refoff[a + 1] <= k) ++a;
+    for (int a = tid; a < nat; a += QX_BLOCK) {
         const ElemParams& e = g_tab.e[sel[a]];
-        const int r = k - refoff[a];
-        refat[k] = a;
-        refii[k] = r;
-        zg[k] = d4_zeta(gfn2::kD4Ga, e.gam * gfn2::kD4Gc, e.refq[r] + e.zeff, e.zeff) * gw[k];
+        for (int r = 0; r < e.nref; ++r) {
+            const int k = refoff[a] + r;
+            zg[k] = d4_zeta(gfn2::kD4Ga, e.gam * gfn2::kD4Gc, e.refq[r] + e.zeff, e.zeff) * gw[k];
+        }
     }
-    for (int p = tid; p < nat * nat; p += QX_BLOCK) {
-        const int i = p / nat, j = p % nat;
-        const ElemParams& ei = g_tab.e[sel[i]];
-        const ElemParams& ej = g_tab.e[sel[j]];
-        const double dx = sx[3 * i] - sx[3 * j], dy = sx[3 * i + 1] - sx[3 * j + 1],
-                     dz = sx[3 * i + 2] - sx[3 * j + 2];
-        const double r2 = dx * dx + dy * dy + dz * dz;
-        disp[p] = (i != j && r2 <= gfn2::kD4RThr) ? d4_disp(ei, ej, r2, nullptr) : 0.0;
-    }
-    __syncthreads();
-    for (int p = tid; p < nd * nd; p += QX_BLOCK) {
-        const int k = p / nd, l = p - k * nd;
-        const int i = refat[k], j = refat[l];
-        WD[p] = disp[i * nat + j] * gw[k] * gw[l] * g_tab.c6ref[sel[i]][refii[k]][sel[j]][refii[l]];
-    }
-    // 6b. damped multipole kernels (AES2) per ordered pair (i, j), rv = R_i - R_j,
-    //     stored as planes c * nat^2 + j * nat + i:
-    //     h3 rv (3), h5 rv_a rv_b (xx, xy, yy, xz, yz, zz), r^2 h5
-    double* ag = B.aesg + (size_t)si.pair_off / QX_PAIR_STRIDE * QX_AES_COMP;
+    double* pk = B.pairk + (size_t)si.pair_off / QX_PAIR_STRIDE * QX_PAIR_KERN;
     const int nn = nat * nat;
     for (int p = tid; p < nn; p += QX_BLOCK) {
-        const int j = p / nat, i = p % nat;
-        double o[QX_AES_COMP];
-        for (int k = 0; k < QX_AES_COMP; ++k) o[k] = 0.0;
+        const int j = p / nat, i = p - j * nat;
+        double h3 = 0.0, h5 = 0.0, disp = 0.0;
         if (i != j) {
-            const double rv0 = sx[3 * i] - sx[3 * j], rv1 = sx[3 * i + 1] - sx[3 * j + 1],
-                         rv2 = sx[3 * i + 2] - sx[3 * j + 2];
-            const double r2 = rv0 * rv0 + rv1 * rv1 + rv2 * rv2;
+            const double dx = sx[3 * i] - sx[3 * j], dy = sx[3 * i + 1] - sx[3 * j + 1],
+                         dz = sx[3 * i + 2] - sx[3 * j + 2];
+            const double r2 = dx * dx + dy * dy + dz * dz;
             const double r = sqrt(r2);
             const double r0 = 0.5 * (B.mrad[si.atom_off + i] + B.mrad[si.atom_off + j]);
             const double r03 = r0 * r0 * r0;
-            const double h3 = 1.0 / (r2 * r + 6.0 * r03);
-            const double h5 = 1.0 / (r * (r2 * r2 + 6.0 * r03 * r0));
-            o[0] = h3 * rv0;
-            o[1] = h3 * rv1;
-            o[2] = h3 * rv2;
-            o[3] = h5 * rv0 * rv0;
-            o[4] = h5 * rv0 * rv1;
-            o[5] = h5 * rv1 * rv1;
-            o[6] = h5 * rv0 * rv2;
-            o[7] = h5 * rv1 * rv2;
-            o[8] = h5 * rv2 * rv2;
-            o[9] = r2 * h5;
+            h3 = 1.0 / (r2 * r + 6.0 * r03);
+            h5 = 1.0 / (r * (r2 * r2 + 6.0 * r03 * r0));
+            if (r2 <= gfn2::kD4RThr) disp = d4_disp(g_tab.e[sel[i]], g_tab.e[sel[j]], r2, nullptr);
         }
-        for (int k = 0; k < QX_AES_COMP; ++k) ag[(size_t)k * nn + p] = o[k];
+        pk[p] = h3;
+        pk[nn + p] = h5;
+        pk[2 * nn + p] = disp;
     }
+    __syncthreads();
     // 7. repulsion energy
     double erep = 0.0;
     for (int p = tid; p < nat * nat; p += QX_BLOCK) {
@@ -524,7 +504,7 @@ __global__ __launch_bounds__(QX_BLOCK) void k_setup(BatchPtrs B, int with_chol)
     if (B.active && !B.active[sys]) return;
     __shared__ SetupLds Ls;
     extern __shared__ double dyn[];
-    setup_system(B, sys, with_chol, Ls, dyn);
+    setup_system(qx_args(B), sys, with_chol, Ls, dyn);
 }
 
 }  // namespace qx
