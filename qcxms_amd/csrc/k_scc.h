@@ -80,28 +80,41 @@ __device__ unsigned long long g_phase[kPhaseSys * kPhaseSlots];
     } while (0)
 #endif
 
+typedef double qx_d4 __attribute__((ext_vector_type(4)));
+
 // C[i][j] = sum_k opA[i][k] * d[k] * opB[k][j] on the FP64 matrix cores
 // (v_mfma_f64_16x16x4f64).  Operands are given by their element strides:
 // opA[i][k] at A[i * ai + k * ak], opB[k][j] at Bm[k * bk + j * bj].  A
 // wavefront computes a strip of two 16 x 16 tiles sharing the A operand;
 // operand lanes: A[i0 + l%16][k0 + l/16], B[k0 + l/16][j0 + l%16];
-// accumulator element r of lane l is C[i0 + 4r + l/16][j0 + l%16].  Lanes of
-// rows and columns past the edge read the last row or column (their results
-// are not stored); only the last k step is masked.  The operands of the next
-// four k steps are loaded while the matrix cores work on the current four, so
-// a strip waits for memory once.
-typedef double qx_d4 __attribute__((ext_vector_type(4)));
+// accumulator element r of lane l is C[i0 + 4r + l/16][j0 + l%16].
+// sym: the result is symmetric (M = N); only strips that reach the diagonal
+// or lie above it are formed, and mirrored.  Lanes of rows and columns past
+// the edge read the last row or column (their results are not stored); only
+// the last k step is masked.  The operands of the next four k steps are
+// loaded while the matrix cores work on the current four, so a strip waits
+// for memory once.
 QX_DEV void mfma_gemm(int M, int N, int K, const double* A, int ai, int ak, const double* Bm, int bk,
-                      int bj, double* Cm, int ldc, const double* d)
+                      int bj, double* Cm, int ldc, const double* d, bool sym)
 {
     constexpr int NU = 2;  // 16 x 16 tiles per strip
     constexpr int KS = 4;  // k steps per pass
+    constexpr int NW = kNT / 64;
     const int tid = qx_tid(), lane = tid & 63, wave = qx_wave(tid);
     const int li = lane & 15, lk = lane >> 4;
     const int tm = (M + 15) >> 4, tc = (N + 16 * NU - 1) / (16 * NU);
     const int nblk = K / (4 * KS);
-    for (int t = wave; t < tm * tc; t += kNT / 64) {
-        const int i0 = (t / tc) * 16, jc = (t % tc) * 16 * NU;
+    int ti = 0, ts = wave;  // tile row, strip in the row counted from its first one
+    auto row_strips = [&](int t) { return sym ? tc - t / NU : tc; };
+    while (ti < tm) {
+        const int ns = row_strips(ti);
+        if (ts >= ns) {
+            ts -= ns;
+            ++ti;
+            continue;
+        }
+        const int i0 = ti * 16, jc = (ts + tc - ns) * 16 * NU;
+        ts += NW;
         const int i = i0 + li < M ? i0 + li : M - 1;
         const double* pa = A + i * ai + lk * ak;
         const double* pb[NU];
@@ -157,7 +170,10 @@ QX_DEV void mfma_gemm(int M, int N, int K, const double* A, int ai, int ak, cons
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const int row = i0 + 4 * r + lk, col = jc + 16 * u + li;
-                if (row < M && col < N) Cm[row * ldc + col] = acc[u][r];
+                if (row < M && col < N && (!sym || (col >> 4) >= ti)) {
+                    Cm[row * ldc + col] = acc[u][r];
+                    if (sym && (col >> 4) > ti) Cm[col * ldc + row] = acc[u][r];
+                }
             }
     }
 }
@@ -793,7 +809,8 @@ QX_DEV int eig_solve(double* A, double* Cv, int m, int nrow, int lda, double tol
                     const bool ta = k == 1 || k == 4;
                     const double* pb = k == 2 ? Z : k == 4 ? W : R;
                     double* pc = k == 2 ? W : k == 3 ? W : k == 4 ? A : Z;
-                    mfma_gemm(k == 5 ? nrow : m, m, m, pa, ta ? 1 : lda, ta ? lda : 1, pb, lda, 1, pc, lda, nullptr);
+                    mfma_gemm(k == 5 ? nrow : m, m, m, pa, ta ? 1 : lda, ta ? lda : 1, pb, lda, 1, pc, lda, nullptr,
+                                   k == 0 || k == 1 || k == 4);
                     if (k != 4) __syncthreads();  // Cv R reads nothing that R^T W writes
                     if (k == 1) {
                         for (int p = tid; p < m * m; p += kNT) {
@@ -1386,7 +1403,7 @@ QX_DEV void scc_body(int sys, const SysInfo& si, BatchRef B0, OptRef opt, SysSha
         }
         const double* X = B.X + si.mat_off;
         if (warm) {
-            mfma_gemm(n, n, n, X, ld, 1, B.U + si.mat_off, ld, 1, Cc, lb, nullptr);
+            mfma_gemm(n, n, n, X, ld, 1, B.U + si.mat_off, ld, 1, Cc, lb, nullptr, false);
         } else {
             for (int p = tid; p < n * n; p += kNT) Cc[(p / n) * lb + p % n] = X[(p / n) * ld + p % n];
         }
@@ -1463,7 +1480,8 @@ QX_DEV void scc_body(int sys, const SysInfo& si, BatchRef B0, OptRef opt, SysSha
             QX_PH(1);
             // A = C^T F C (F C staged in the density buffer)
             for (int s = 0; s < 2; ++s) {
-                mfma_gemm(n, n, n, s ? Cc : Ft, s ? 1 : lb, s ? lb : 1, s ? P : Cc, lb, 1, s ? A : P, lb, nullptr);
+                mfma_gemm(n, n, n, s ? Cc : Ft, s ? 1 : lb, s ? lb : 1, s ? P : Cc, lb, 1, s ? A : P, lb, nullptr,
+                          s != 0);
                 if (s && m > n)
                     for (int j = qx_tid(); j < m; j += kNT) {
                         A[n * lb + j] = 0.0;
@@ -1500,7 +1518,7 @@ QX_DEV void scc_body(int sys, const SysInfo& si, BatchRef B0, OptRef opt, SysSha
             __syncthreads();
             ts = L.s_e[0];
             QX_PH(4);
-            mfma_gemm(n, n, n, Cc, lb, 1, Cc, 1, lb, P, lb, f2);
+            mfma_gemm(n, n, n, Cc, lb, 1, Cc, 1, lb, P, lb, f2, true);
             __syncthreads();
             QX_PH(5);
             // row sums of P o M for M = S, D (3), Q (6), H0 as coalesced column
@@ -1611,8 +1629,8 @@ QX_DEV void scc_body(int sys, const SysInfo& si, BatchRef B0, OptRef opt, SysSha
     }
     __syncthreads();
     // W = C diag(2 f e) C^T ; U = L^T C for the next warm start
-    mfma_gemm(n, n, n, Cc, lb, 1, Cc, 1, lb, B.W + si.mat_off, ld, f2);
-    mfma_gemm(n, n, n, B.L + si.mat_off, 1, ld, Cc, lb, 1, B.U + si.mat_off, ld, nullptr);
+    mfma_gemm(n, n, n, Cc, lb, 1, Cc, 1, lb, B.W + si.mat_off, ld, f2, true);
+    mfma_gemm(n, n, n, B.L + si.mat_off, 1, ld, Cc, lb, 1, B.U + si.mat_off, ld, nullptr, false);
     QX_PH(10);
     if (tid == 0) {
         double* ep = B.eparts + 10 * sys;
