@@ -601,7 +601,9 @@ size_t lds_scc_bytes_range(const qcxms_batch* b, int s0, int s1, int lds_max_m, 
             if (pot > 2 * mm) need = std::max(need, 4 * mm + qx::kRs * m + pot);
         } else {
             const size_t blk = m * (m + 2) / 2;
-            if (blk * sizeof(double) <= g_scc_dyn_max) need = std::max(need, blk);
+            const size_t nblk = (m / 2) * (m / 2 + 1) / 2;
+            if (blk * sizeof(double) <= g_scc_dyn_max && nblk <= (size_t)qx::kMaxNB * (QX_SCC_BLOCK - 64))
+                need = std::max(need, blk);
             need = std::max(need, std::max(pot, broy));
         }
     }

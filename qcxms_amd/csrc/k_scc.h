@@ -313,6 +313,8 @@ QX_DEV double2 pivot_rotation(double app, double aqq, double apq, double tol, do
     return make_double2(turn ? cs.x : 1.0, turn ? cs.y : 0.0);
 }
 
+constexpr int kMaxNB = 5;  // blocks per thread the rounds take (132 basis functions)
+
 // Working storage of the Jacobi sweeps
 struct JacobiBuffers {
     double* blk;      // A as 2 x 2 blocks by seats: 4 planes of half (half + 1) / 2 doubles (LDS)
@@ -390,17 +392,21 @@ QX_DEV void block_moves(int half, int nblk, int P, int R, int to[4])
 
 // The rounds of one sweep, blocks in LDS.  NB: blocks per thread of the
 // wavefronts 1 ...; f: half of rot that holds the rotations of round 0.
-// NR > 0 (m <= 64): the rows of Cv as well, x[u] row wave - 1 + u (kNT / 64 -
-// 1) with a lane per column, so a rotation is one exchange between lanes and
-// two multiply-adds per row; they run while wavefront 0 has the pivots.
-// NR = 0: the rotations are logged instead.
+// NR > 0 (m <= 64): the rows of Cv as well, two per pair of registers x[u],
+// y[u] (rows_lane), a lane per pair slot: the rotation of a slot, then the
+// players move to the next lane.  x holds the p players and y the q players,
+// but in slot 0, whose q player stays, the other way round, so that x moves
+// down and y up.  They run while wavefront 0 has the pivots.  NR = 0: the
+// rotations are logged instead.
 template <int NB, int NR>
-QX_DEV void jacobi_rounds(const JacobiBuffers& jb, int m, int nrow, double tol, double min_s, double* x, int& f)
+QX_DEV void jacobi_rounds(const JacobiBuffers& jb, int m, int nrow, double tol, double min_s, double* x, double* y,
+                          int& f)
 {
     constexpr int kNU = kNT - 64, NW = kNT / 64 - 1, NK = NB > 3 ? 2 : 1;  // NK pivots per lane (half <= 64 NK)
     const int tid = qx_tid(), lane = tid & 63, wave = qx_wave(tid), ut = tid - 64;
     const int half = m / 2, nblk = half * (half + 1) / 2;
     double* blk = jb.blk;
+    const int k = lane & 31;             // pair slot of the lane's rows
     JacobiPivot pv[NK];                  // wavefront 0
     int bPR[NB], to01[NB], to23[NB];     // the others: their blocks and where each entry goes
     if (wave == 0) {
@@ -444,11 +450,11 @@ QX_DEV void jacobi_rounds(const JacobiBuffers& jb, int m, int nrow, double tol, 
 #pragma unroll
             for (int j = 0; j < NK; ++j) {
                 const double2 cs = pv[j].rotation(half, tol, min_s);
-                const int k = lane + 64 * j;
-                if (k < half) {
+                const int kp = lane + 64 * j;
+                if (kp < half) {
                     turn = turn || cs.y != 0.0;
-                    jb.rot[(f ^ 1) * half + k] = cs;
-                    if (!NR && r + 1 < m - 1) jb.log[(r + 1) * half + k] = cs;
+                    jb.rot[(f ^ 1) * half + kp] = cs;
+                    if (!NR && r + 1 < m - 1) jb.log[(r + 1) * half + kp] = cs;
                 }
             }
             turn = qx_any(turn);
@@ -462,26 +468,21 @@ QX_DEV void jacobi_rounds(const JacobiBuffers& jb, int m, int nrow, double tol, 
                 blk[to23[j] & 0xffff] = nn[j][2];
                 blk[(unsigned)to23[j] >> 16] = nn[j][3];
             }
-            if (NR && any) {
-                // pair slot, side and partner of the lane's player
-                int d = lane - r;
-                if (d < 0) d += m - 1;
-                bool qside = d > half - 1;
-                int k = qside ? m - 1 - d : d;
-                int partner = qside ? r + k : r - k;
-                if (partner < 0) partner += m - 1;
-                if (partner >= m - 1) partner -= m - 1;
-                if (lane == r) partner = m - 1;
-                if (lane >= m - 1) {
-                    qside = true;
-                    k = 0;
-                    partner = lane == m - 1 ? r : lane;
-                }
-                const double2 cs = rf[k];
-                const double s = qside ? cs.y : -cs.y;
+            if (NR) {
+                const double2 cs = rf[k < half ? k : 0];
+                const double sg = k == 0 ? -cs.y : cs.y;
 #pragma unroll
-                for (int u = 0; u < NR; ++u)
-                    if (wave - 1 + NW * u < nrow) x[u] = cs.x * x[u] + s * __shfl(x[u], partner, 64);
+                for (int u = 0; u < NR; ++u) {
+                    if (2 * (wave - 1 + NW * u) >= nrow) continue;
+                    double px = x[u], py = y[u];
+                    if (any) {
+                        px = cs.x * x[u] - sg * y[u];
+                        py = sg * x[u] + cs.x * y[u];
+                    }
+                    const double up = qx_lane_up(px, 0.0), down = qx_lane_down(py, 0.0);
+                    x[u] = k == 0 ? px : k == half - 1 ? py : up;
+                    y[u] = half == 1 ? py : k == 0 ? up : down;
+                }
             }
         }
         qx_lds_barrier();
@@ -625,18 +626,26 @@ QX_DEV void jacobi_replay_slots(const JacobiBuffers& jb, double* Cv, int m, int 
 // before its writes, one ends it.  Up to 64 columns the other wavefronts also
 // rotate Cv, held in registers; above that the rotations of a sweep are
 // logged and applied to Cv afterwards, without barriers.
-template <bool FAST, bool LDS>
+template <int NB, int NR>
 QX_DEV int jacobi(double* A, double* Cv, int m, int nrow, int lda, double tol, int maxsweep, double min_s,
                   const JacobiBuffers& jb)
 {
-    constexpr int NW = kNT / 64 - 1, NR = FAST ? (kFastM + NW - 1) / NW : (64 + NW - 1) / NW;
+    constexpr int NW = kNT / 64 - 1;
+    constexpr bool LDS = NB > 0, rows = NR > 0;
     const int half = m / 2, nblk = half * (half + 1) / 2;
     if (qx_uniform(offdiag_max(A, m, lda, jb.red) < tol)) return 0;
     const int tid = qx_tid(), lane = tid & 63, wave = qx_wave(tid);
-    const bool rows = FAST || (LDS && m <= 64);
     int sweep = 0, f = 0, g = 0;
     double* blk = LDS ? jb.blk : jb.gblk[0];
-    double x[NR];
+    double x[NR ? NR : 1], y[NR ? NR : 1];
+    // rows of Cv in registers (jacobi_rounds): row and columns of a lane
+    auto rows_lane = [&](int u, int& i, int& cx, int& cy) {
+        const int k = lane & 31;
+        i = 2 * (wave - 1 + NW * u) + (lane >> 5);
+        cx = k == 0 ? m - 1 : k;
+        cy = k == 0 ? 0 : m - 1 - k;
+        return wave > 0 && i < nrow && k < half;
+    };
     for (int b = tid; b < nblk; b += kNT) {
         int P, R;
         int2 p, r;
@@ -651,8 +660,10 @@ QX_DEV int jacobi(double* A, double* Cv, int m, int nrow, int lda, double tol, i
     if (rows) {
 #pragma unroll
         for (int u = 0; u < NR; ++u) {
-            const int i = wave - 1 + NW * u;
-            x[u] = wave > 0 && i < nrow && lane < m ? Cv[i * lda + lane] : 0.0;
+            int i, cx, cy;
+            const bool in = rows_lane(u, i, cx, cy);
+            x[u] = in ? Cv[i * lda + cx] : 0.0;
+            y[u] = in ? Cv[i * lda + cy] : 0.0;
         }
     }
     __syncthreads();
@@ -675,11 +686,8 @@ QX_DEV int jacobi(double* A, double* Cv, int m, int nrow, int lda, double tol, i
             for (int k = tid; k < half; k += kNT) jb.log[k] = jb.rot[f * half + k];
         if (tid == 0) jb.any[0] = jb.any[m - 1];
         __syncthreads();
-        if (FAST) jacobi_rounds<1, NR>(jb, m, nrow, tol, min_s, x, f);
-        else if (!LDS) jacobi_rounds_global(jb, m, tol, min_s, f, g);
-        else if (m <= 64) jacobi_rounds<2, NR>(jb, m, nrow, tol, min_s, x, f);
-        else if (nblk <= 3 * (kNT - 64)) jacobi_rounds<3, 0>(jb, m, nrow, tol, min_s, x, f);
-        else jacobi_rounds<6, 0>(jb, m, nrow, tol, min_s, x, f);
+        if constexpr (LDS) jacobi_rounds<NB, NR>(jb, m, nrow, tol, min_s, x, y, f);
+        else jacobi_rounds_global(jb, m, tol, min_s, f, g);
         if (!LDS) blk = jb.gblk[g];
         if (!rows) {
             __syncthreads();
@@ -718,12 +726,31 @@ QX_DEV int jacobi(double* A, double* Cv, int m, int nrow, int lda, double tol, i
     if (rows) {
 #pragma unroll
         for (int u = 0; u < NR; ++u) {
-            const int i = wave - 1 + NW * u;
-            if (wave > 0 && i < nrow && lane < m) Cv[i * lda + lane] = x[u];
+            int i, cx, cy;
+            if (rows_lane(u, i, cx, cy)) {
+                Cv[i * lda + cx] = x[u];
+                Cv[i * lda + cy] = y[u];
+            }
         }
     }
     __syncthreads();
     return sweep;
+}
+
+// jacobi() in the form for the system: rows of Cv in registers up to 64
+// columns, blocks per thread by the number of blocks, or the blocks in global
+// memory when they do not fit in LDS
+template <bool FAST>
+QX_DEV int jacobi_any(double* A, double* Cv, int m, int nrow, int lda, double tol, int maxsweep, double min_s,
+                      const JacobiBuffers& jb)
+{
+    constexpr int kNU = kNT - 64, kRows = 2 * (kNT / 64 - 1);  // rows of Cv per register pair
+    const int nblk = (m / 2) * (m / 2 + 1) / 2;
+    if (FAST) return jacobi<1, (kFastM + kRows - 1) / kRows>(A, Cv, m, nrow, lda, tol, maxsweep, min_s, jb);
+    if (!jb.lds) return jacobi<0, 0>(A, Cv, m, nrow, lda, tol, maxsweep, min_s, jb);
+    if (m <= 64) return jacobi<2, (64 + kRows - 1) / kRows>(A, Cv, m, nrow, lda, tol, maxsweep, min_s, jb);
+    if (nblk <= 3 * kNU) return jacobi<3, 0>(A, Cv, m, nrow, lda, tol, maxsweep, min_s, jb);
+    return jacobi<kMaxNB, 0>(A, Cv, m, nrow, lda, tol, maxsweep, min_s, jb);
 }
 
 constexpr double kCoarseSin = 0.02;  // |sin| of the rotations a coarse sweep applies
@@ -842,8 +869,7 @@ QX_DEV int eig_solve(double* A, double* Cv, int m, int nrow, int lda, double tol
                 min_s = kCoarseSin;
             }
         }
-        const int done = FAST || jb.lds ? jacobi<FAST, true>(A, Cv, m, nrow, lda, tol, sweeps, min_s, jb)
-                                        : jacobi<FAST, false>(A, Cv, m, nrow, lda, tol, sweeps, min_s, jb);
+        const int done = jacobi_any<FAST>(A, Cv, m, nrow, lda, tol, sweeps, min_s, jb);
         if (sweeps != 1) return done;
         QX_PH_ADD(29, 1);
     }
@@ -1493,7 +1519,7 @@ QX_DEV void scc_body(int sys, const SysInfo& si, BatchRef B0, OptRef opt, SysSha
             double jtol = fmin(1e-6, 1e-3 * errp);
             if (jtol < opt.jacobi_tol) jtol = opt.jacobi_tol;
             const int nblk = (m / 2) * (m / 2 + 1) / 2;
-            const bool blk_lds = FAST || (4 * nblk <= bf.nlds && nblk <= 6 * (kNT - 64));
+            const bool blk_lds = FAST || (4 * nblk <= bf.nlds && nblk <= kMaxNB * (kNT - 64));
             const JacobiBuffers jb{FAST ? Ft : bf.lds, {Ft, bf.E}, (double2*)P, (double2*)ss.rot, ss.any, ss.red, blk_lds};
             const int nsweep = eig_solve<EIG, FAST>(A, Cc, m, n, lb, jtol, Ft, P, bf.E, jb);
             QX_PH(3);
