@@ -593,7 +593,7 @@ size_t lds_scc_bytes_range(const qcxms_batch* b, int s0, int s1, int lds_max_m, 
     for (int s = s0; s < s1; ++s) {
         const SysInfo& si = b->info[s];
         const size_t m = (size_t)((si.nao + 1) & ~1);
-        const size_t pot = qx::pot_lds(si.nat, si.ndim), broy = (kBroydenLds + 1) * (kBroydenLds + 1);
+        const size_t pot = qx::pot_lds(si.nat), broy = (kBroydenLds + 1) * (kBroydenLds + 1);
         if (m <= (size_t)lds_max_m) {
             const size_t mm = m * (m + 1);
             lm = std::max(lm, m);

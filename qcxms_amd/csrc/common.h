@@ -159,6 +159,18 @@ QX_DEV double wave_reduce(double v)
 #endif
 }
 
+// sum over the four lanes of a quad, on each of them
+QX_DEV double quad_sum(double v)
+{
+#ifdef __HIP_DEVICE_COMPILE__
+    v += qx_dpp<0xb1>(v);
+    return v + qx_dpp<0x4e>(v);
+#else
+    v += __shfl_xor(v, 1, 64);
+    return v + __shfl_xor(v, 2, 64);
+#endif
+}
+
 QX_DEV double wave_sum(double v) { return wave_reduce<QxAdd>(v); }
 QX_DEV double wave_max(double v) { return wave_reduce<QxMax>(v); }
 

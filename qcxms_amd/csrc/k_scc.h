@@ -918,15 +918,14 @@ QX_DEV double fermi_wave(int n, const double* e, double kt, double nalpha, doubl
                          int& iters)
 {
     const int l = threadIdx.x & 63;
+    const double ikt = 1.0 / kt;
     double lo = 1e300, hi = -1e300;
     for (int i = l; i < n; i += 64) {
         lo = fmin(lo, e[i]);
         hi = fmax(hi, e[i]);
     }
-    for (int o = 32; o > 0; o >>= 1) {
-        lo = fmin(lo, __shfl_xor(lo, o, 64));
-        hi = fmax(hi, __shfl_xor(hi, o, 64));
-    }
+    lo = -wave_max(-lo);
+    hi = wave_max(hi);
     lo = lo - 50.0 * kt - 1.0;
     hi = hi + 50.0 * kt + 1.0;
     double mu = (mu_io > lo && mu_io < hi) ? mu_io : 0.5 * (lo + hi);
@@ -935,12 +934,12 @@ QX_DEV double fermi_wave(int n, const double* e, double kt, double nalpha, doubl
         ++iters;
         double s = 0.0, ds = 0.0;
         for (int i = l; i < n; i += 64) {
-            const double fi = 1.0 / (1.0 + exp((e[i] - mu) / kt));
+            const double fi = 1.0 / (1.0 + exp((e[i] - mu) * ikt));
             s += fi;
-            ds += fi * (1.0 - fi) / kt;
+            ds += fi * (1.0 - fi);
         }
         s = wave_sum(s);
-        ds = wave_sum(ds);
+        ds = wave_sum(ds) * ikt;
         const double diff = nalpha - s;
         if (fabs(diff) <= 1e-13 * fmax(nalpha, 1.0)) {
             if (ds > 0.0) mu += diff / ds;  // final Newton polish
@@ -955,7 +954,7 @@ QX_DEV double fermi_wave(int n, const double* e, double kt, double nalpha, doubl
     }
     double ts = 0.0;
     for (int i = l; i < n; i += 64) {
-        const double fi = 1.0 / (1.0 + exp((e[i] - mu) / kt));
+        const double fi = 1.0 / (1.0 + exp((e[i] - mu) * ikt));
         f[i] = fi;
         if (fi > 0.0 && fi < 1.0) ts += fi * log(fi) + (1.0 - fi) * log(1.0 - fi);
     }
@@ -989,16 +988,43 @@ struct SysShared {
     double eparts[6];  // es2, es3, aes, axc, d4, unused
 };
 
-// LDS doubles potentials() works in: inner D4 sums, multipole shares, outer
-// D4 sums
-inline __host__ __device__ int pot_lds(int nat, int ndim)
+// LDS doubles potentials() works in: inner D4 sums, multipole shares
+inline __host__ __device__ int pot_lds(int nat)
 {
-    const int nu = kNT - 64, nseg = ndim * 4 <= nu ? 4 : ndim * 2 <= nu ? 2 : 1;
-    return gfn2::kElem * QX_MAX_REF * nat + (nat <= 32 ? 20 : 40) * nat + nseg * ndim;
+    return gfn2::kElem * QX_MAX_REF * nat + (nat <= 32 ? 80 : 40) * nat;
 }
 
-// Potentials vs (per shell), vd (3 per atom), vq (6 per atom) and interaction
-// energies (ES2, ES3, AES, AXC, D4 two-body) at moments x = [qsh, dp, qp].
+// What a thread needs from the parameter tables in every call: of its D4
+// reference (threads 4 k .. 4 k + 3 of the first pass: reference k), its
+// shell's Coulomb row and its atom's on-site multipole kernels.
+struct PotTables {
+    double c, qref, zeff, gw, third, dk, qk;
+
+    QX_DEV void load(const SysInfo& si, BatchRef B, const SysShared& ss)
+    {
+        static_assert(kMaxRef <= kNT && QX_MAX_NSH <= kNT - 256, "one reference and one shell per thread");
+        const int tid = qx_tid();
+        c = qref = zeff = gw = third = dk = qk = 0.0;
+        if (tid < si.ndim) {
+            const int a = ss.refat[tid];
+            const ElemParams& e = g_tab.e[ss.sel[a]];
+            c = e.gam * gfn2::kD4Gc;
+            qref = e.refq[tid - ss.refoff[a]] + e.zeff;
+            zeff = e.zeff;
+            gw = B.gw[si.ref_off + tid];
+        }
+        const int a = kNT - 1 - tid;
+        if (a < si.nsh) third = g_tab.e[ss.sh[a].el].third[ss.sh[a].k];
+        if (tid < si.nat) {
+            dk = g_tab.e[ss.sel[tid]].dkernel;
+            qk = g_tab.e[ss.sel[tid]].qkernel;
+        }
+    }
+};
+
+// Potentials vs (per shell), vd (3 per atom), vq (6 per atom) and, with
+// energy set, interaction energies (ES2, ES3, AES, AXC, D4 two-body) at
+// moments x = [qsh, dp, qp].
 // The D4 response of reference k of atom i is
 //   y_k = gw_k sum_j disp_ij sum_(l of j) C6ref_kl gw_l z_l,
 // whose inner sum depends on i through its element and reference number only:
@@ -1006,69 +1032,100 @@ inline __host__ __device__ int pot_lds(int nat, int ndim)
 // terms per reference instead of ndim, and nat^2 values to read instead of
 // ndim^2.  The multipole terms read two damped kernels per atom pair (1/r^3
 // and 1/r^5) and take the directions from the coordinates.  First the
-// wavefronts 0 .. na - 1 sum the multipole terms of a share of the partners
-// each while the others form the inner D4 sums and the shell Coulomb
-// potential gamma q; then wavefront 0 adds the shares up (lane = atom) while
-// the others take the outer D4 sums, several threads per reference.  The AES
-// energy is x . v_aes / 2 (the multipole energy is a symmetric bilinear form
-// of the moments).  scr: LDS, pot_lds(nat, ndim) doubles.
+// wavefronts 0 .. 3 sum the multipole terms of a share of the partners each
+// (half-wavefronts up to 32 atoms) while the others form the inner D4 sums
+// and the shell Coulomb potential gamma q; then the shares are added up, a
+// thread per atom and term, and the outer D4 sums taken, four threads per
+// reference; then the atoms' terms are put together.  A call is bound by the
+// instructions on its longest wavefront, not by memory, so what is read from
+// memory is under way before it is needed and the tables' values are kept in
+// registers.  The AES energy is x . v_aes / 2 (the multipole energy is a
+// symmetric bilinear form of the moments).  scr: LDS, pot_lds(nat) doubles.
 // (26-atom C8H18+, 50 basis functions: 20-30 k cycles a call with one
 // multipole wavefront, ten kernel planes and the ndim^2 response matrix.)
-QX_DEV void potentials(const SysInfo& si, BatchRef B, SysShared& ss, const double* x, double* vs, double* vd,
-                       double* vq, double* scr)
+QX_DEV void potentials(const SysInfo& si, BatchRef B, SysShared& ss, const PotTables& pt, const double* x, double* vs,
+                       double* vd, double* vq, double* scr, bool energy)
 {
     const int tid = qx_tid(), lane = tid & 63, wave = qx_wave(tid);
     const int nat = si.nat, nsh = si.nsh, nd = si.ndim, nn = nat * nat;
     const double* qsh = x;
     const double* dp = x + nsh;
     const double* qp = x + nsh + 3 * nat;
+    constexpr int na = 4;          // multipole wavefronts
     const bool split = nat <= 32;  // two half-wavefronts of atoms
-    const int na = split ? 2 : 4;
+    const int nparts = split ? 2 * na : na;
     const int ner = qx_uniform(ss.eroff[gfn2::kElem]);
-    double* tt = scr;                  // ner x nat inner D4 sums
-    double* pa = tt + ner * nat;       // na x 10 x nat multipole shares
-    double* py = pa + na * 10 * nat;   // outer D4 sums of the threads of a reference
+    double* tt = scr;             // ner x nat inner D4 sums
+    double* pa = tt + ner * nat;  // nparts x 10 x nat multipole shares
     const double* pk = B.pairk + (size_t)si.pair_off / QX_PAIR_STRIDE * QX_PAIR_KERN;
+    // what the first pass of each wavefront reads from memory, on its way
+    // while the charges and D4 references are formed: kernels of the first
+    // NJ partners, or the C6 row of the first inner D4 sum and the start of
+    // the Coulomb row
+    constexpr int NJ = 4, NB = 8;
+    const int t0 = tid - 64 * na, nt = kNT - 64 * na;
+    const int ai = split ? (lane & 31) : lane;
+    const int part = split ? 2 * wave + (lane >> 5) : wave;
+    const int len = (nat + nparts - 1) / nparts, pj0 = part * len, pj1 = pj0 + len < nat ? pj0 + len : nat;
+    const double* G = B.gam + si.gam_off;
+    const int ga = kNT - 1 - tid;  // Coulomb row, from the last thread on
+    auto c6row = [&](int p) {
+        const int er = p / nat, j = p - er * nat;
+        int e = 0;
+        while (ss.eroff[e + 1] <= er) ++e;
+        return g_tab.c6ref[e][er - ss.eroff[e]][ss.sel[j]];
+    };
+    double h3[NJ], h5[NJ], c6[QX_MAX_REF], gr[NB];
+    auto kernels = [&](int jb) {
+#pragma unroll
+        for (int u = 0; u < NJ; ++u) {
+            const int j = jb + u < pj1 ? jb + u : ai;  // (i, i) is zero
+            h3[u] = pk[j * nat + ai];
+            h5[u] = pk[nn + j * nat + ai];
+        }
+    };
+    auto coulomb = [&](int b0) {
+#pragma unroll
+        for (int u = 0; u < NB; ++u) gr[u] = G[(b0 + u < nsh ? b0 + u : b0) * nsh + ga];
+    };
+    if (wave < na) {
+        if (ai < nat) kernels(pj0);
+    } else {
+        const double* c = c6row(t0 < ner * nat ? t0 : 0);
+#pragma unroll
+        for (int l = 0; l < QX_MAX_REF; ++l) c6[l] = c[l];
+        if (ga < nsh) coulomb(0);
+    }
+    qx_sched_fence();
     for (int a = tid; a < nat; a += kNT) {
         double q = 0.0;
         for (int s = ss.shoff[a]; s < ss.shoff[a + 1]; ++s) q += qsh[s];
         ss.qat[a] = q;
     }
     __syncthreads();
-    const double* gw = B.gw + si.ref_off;
-    for (int k = tid; k < nd; k += kNT) {
-        const int a = ss.refat[k];
-        const ElemParams& e = g_tab.e[ss.sel[a]];
-        const int r = k - ss.refoff[a];
+    if (tid < nd) {
         double z, dz;
-        d4_zeta_both(gfn2::kD4Ga, e.gam * gfn2::kD4Gc, e.refq[r] + e.zeff, ss.qat[a] + e.zeff, z, dz);
-        const double g = gw[k];
-        ss.zr[k] = z * g;
-        ss.dzr[k] = dz * g;
+        d4_zeta_both(gfn2::kD4Ga, pt.c, pt.qref, ss.qat[ss.refat[tid]] + pt.zeff, z, dz);
+        ss.zr[tid] = z * pt.gw;
+        ss.dzr[tid] = dz * pt.gw;
     }
     __syncthreads();
     double eaes = 0.0, eaxc = 0.0, es2 = 0.0, es3 = 0.0, ed4 = 0.0;
     if (wave < na) {
-        const int i = split ? (lane & 31) : lane;
-        const int part = split ? 2 * wave + (lane >> 5) : wave;  // of four
-        const int len = (nat + 3) / 4, j0 = part * len, j1 = j0 + len < nat ? j0 + len : nat;
+        const int i = ai;
         double v0 = 0.0, d0 = 0.0, d1 = 0.0, d2 = 0.0;
         double w0 = 0.0, w1 = 0.0, w2 = 0.0, w3 = 0.0, w4 = 0.0, w5 = 0.0;
         if (i < nat) {
             const double x0 = ss.sx[3 * i], x1 = ss.sx[3 * i + 1], x2 = ss.sx[3 * i + 2];
-            constexpr int NJ = 8;
-            for (int jb = j0; jb < j1; jb += NJ) {
-                double h3[NJ], h5[NJ];
-#pragma unroll
-                for (int u = 0; u < NJ; ++u) {
-                    const int j = jb + u < j1 ? jb + u : i;  // (i, i) is zero
-                    h3[u] = pk[j * nat + i];
-                    h5[u] = pk[nn + j * nat + i];
+            for (int jb = pj0; jb < pj1; jb += NJ) {
+                if (jb > pj0) {
+                    kernels(jb);
+                    qx_sched_fence();
                 }
-                qx_sched_fence();
 #pragma unroll
                 for (int u = 0; u < NJ; ++u) {
-                    const int j = jb + u < j1 ? jb + u : i;
+                    if (jb + u >= pj1) continue;
+                    const int j = jb + u;
                     const double rv0 = x0 - ss.sx[3 * j], rv1 = x1 - ss.sx[3 * j + 1], rv2 = x2 - ss.sx[3 * j + 2];
                     const double r2 = rv0 * rv0 + rv1 * rv1 + rv2 * rv2;
                     const double g0 = h3[u] * rv0, g1 = h3[u] * rv1, g2 = h3[u] * rv2;
@@ -1091,70 +1148,88 @@ QX_DEV void potentials(const SysInfo& si, BatchRef B, SysShared& ss, const doubl
                     w5 += qj * g8;
                 }
             }
-        }
-        double pv[10] = {v0, d0, d1, d2, w0, w1, w2, w3, w4, w5};
+            double* o = pa + part * 10 * nat + i;
+            const double pv[10] = {v0, d0, d1, d2, w0, w1, w2, w3, w4, w5};
 #pragma unroll
-        for (int k = 0; k < 10; ++k) {
-            if (split) pv[k] += __shfl_xor(pv[k], 32, 64);
-            if (i < nat && lane < (split ? 32 : 64)) pa[(wave * 10 + k) * nat + i] = pv[k];
+            for (int k = 0; k < 10; ++k) o[k * nat] = pv[k];
         }
     } else {
-        const int t0 = tid - 64 * na, nt = kNT - 64 * na;
         for (int p = t0; p < ner * nat; p += nt) {
-            const int er = p / nat, j = p - er * nat, ej = ss.sel[j];
-            int e = 0;
-            while (ss.eroff[e + 1] <= er) ++e;
-            const double* c6 = g_tab.c6ref[e][er - ss.eroff[e]][ej];
-            const int l0 = ss.refoff[j], nl = ss.refoff[j + 1] - l0;
-            double c[QX_MAX_REF], s = 0.0;
+            if (p > t0) {
+                const double* c = c6row(p);
 #pragma unroll
-            for (int l = 0; l < QX_MAX_REF; ++l) c[l] = c6[l];
+                for (int l = 0; l < QX_MAX_REF; ++l) c6[l] = c[l];
+            }
+            const int j = p % nat, l0 = ss.refoff[j], nl = ss.refoff[j + 1] - l0;
+            double s = 0.0;
 #pragma unroll
             for (int l = 0; l < QX_MAX_REF; ++l)
-                if (l < nl) s += c[l] * ss.zr[l0 + l];
+                if (l < nl) s += c6[l] * ss.zr[l0 + l];
             tt[p] = s;
         }
-        // shell Coulomb rows, from the threads at the other end
-        const double* G = B.gam + si.gam_off;
-        for (int a = nt - 1 - t0; a < nsh; a += nt) {
+        if (ga < nsh) {
             double v = 0.0;
-            constexpr int NB = 12;
             for (int b0 = 0; b0 < nsh; b0 += NB) {
                 double g[NB];
 #pragma unroll
-                for (int u = 0; u < NB; ++u) g[u] = G[(b0 + u < nsh ? b0 + u : b0) * nsh + a];
+                for (int u = 0; u < NB; ++u) g[u] = gr[u];
+                if (b0 + NB < nsh) coulomb(b0 + NB);
                 qx_sched_fence();
 #pragma unroll
                 for (int u = 0; u < NB; ++u)
                     if (b0 + u < nsh) v += g[u] * qsh[b0 + u];
             }
-            const double q = qsh[a];
-            const double g3 = g_tab.e[ss.sh[a].el].third[ss.sh[a].k];
+            const double q = qsh[ga];
             es2 += 0.5 * q * v;
-            es3 += g3 * q * q * q / 3.0;
-            vs[a] = v + g3 * q * q;
+            es3 += pt.third * q * q * q / 3.0;
+            vs[ga] = v + pt.third * q * q;
         }
     }
     __syncthreads();
-    const int nu = kNT - 64, nseg = nd * 4 <= nu ? 4 : nd * 2 <= nu ? 2 : 1;
+    // the multipole shares of one atom and term, into the first share
+    for (int p = tid; p < 10 * nat; p += kNT) {
+        double v = pa[p];
+        for (int w = 1; w < nparts; ++w) v += pa[w * 10 * nat + p];
+        pa[p] = v;
+    }
+    // the outer D4 sums: the four threads of a reference take a share of the
+    // atoms each; -dz_k y_k replaces dz_k
+    const int slen = (nat + 3) / 4;
+    for (int p = kNT - 1 - tid; p < ((4 * nd + 63) & ~63); p += kNT) {  // whole wavefronts
+        const int k = p < 4 * nd ? p >> 2 : nd - 1, seg = p & 3, i = ss.refat[k];
+        const double* t = tt + (ss.eroff[ss.sel[i]] + k - ss.refoff[i]) * nat;
+        const double* dsp = pk + 2 * nn + i;
+        const int j0 = seg * slen, j1 = p >= 4 * nd ? j0 : j0 + slen < nat ? j0 + slen : nat;
+        double y = 0.0;
+        constexpr int ND = 8;
+        for (int jb = j0; jb < j1; jb += ND) {
+            double ds[ND];
+#pragma unroll
+            for (int u = 0; u < ND; ++u) ds[u] = dsp[(jb + u < j1 ? jb + u : jb) * nat];
+            qx_sched_fence();
+#pragma unroll
+            for (int u = 0; u < ND; ++u)
+                if (jb + u < j1) y += ds[u] * t[jb + u];
+        }
+        y = quad_sum(y);
+        if (seg == 0 && p < 4 * nd) {
+            ed4 += -0.5 * ss.zr[k] * y;
+            ss.dzr[k] = -ss.dzr[k] * y;
+        }
+    }
+    __syncthreads();
     if (wave == 0) {
         const int i = lane;
         if (i < nat) {
-            double pv[10];
-#pragma unroll
-            for (int k = 0; k < 10; ++k) {
-                pv[k] = 0.0;
-                for (int w = 0; w < na; ++w) pv[k] += pa[(w * 10 + k) * nat + i];
-            }
-            const double v0 = pv[0], d0 = pv[1], d1 = pv[2], d2 = pv[3];
-            const double w0 = pv[4], w1 = 2.0 * pv[5], w2 = pv[6], w3 = 2.0 * pv[7], w4 = 2.0 * pv[8], w5 = pv[9];
-            const ElemParams& ei = g_tab.e[ss.sel[i]];
+            const double v0 = pa[i], d0 = pa[nat + i], d1 = pa[2 * nat + i], d2 = pa[3 * nat + i];
+            const double w0 = pa[4 * nat + i], w1 = 2.0 * pa[5 * nat + i], w2 = pa[6 * nat + i],
+                         w3 = 2.0 * pa[7 * nat + i], w4 = 2.0 * pa[8 * nat + i], w5 = pa[9 * nat + i];
             const double qi = ss.qat[i];
             const double mi0 = dp[3 * i], mi1 = dp[3 * i + 1], mi2 = dp[3 * i + 2];
             const double* ti = qp + 6 * i;
             eaes = 0.5 * (qi * v0 + mi0 * d0 + mi1 * d1 + mi2 * d2 + ti[0] * w0 + ti[1] * w1 + ti[2] * w2 +
                           ti[3] * w3 + ti[4] * w4 + ti[5] * w5);
-            const double dk = ei.dkernel, qk = ei.qkernel;
+            const double dk = pt.dk, qk = pt.qk;
             eaxc = dk * (mi0 * mi0 + mi1 * mi1 + mi2 * mi2) +
                    qk * (ti[0] * ti[0] + ti[2] * ti[2] + ti[5] * ti[5] +
                          2.0 * (ti[1] * ti[1] + ti[3] * ti[3] + ti[4] * ti[4]));
@@ -1167,46 +1242,23 @@ QX_DEV void potentials(const SysInfo& si, BatchRef B, SysShared& ss, const doubl
             vq[6 * i + 3] = w3 + 4.0 * qk * ti[3];
             vq[6 * i + 4] = w4 + 4.0 * qk * ti[4];
             vq[6 * i + 5] = w5 + 2.0 * qk * ti[5];
-            ss.vat[i] = v0;
         }
     } else {
-        const int len = (nat + nseg - 1) / nseg;
-        for (int p = tid - 64; p < nseg * nd; p += nu) {
-            const int seg = p / nd, k = p - seg * nd;
-            const int i = ss.refat[k];
-            const double* t = tt + (ss.eroff[ss.sel[i]] + k - ss.refoff[i]) * nat;
-            const double* dsp = pk + 2 * nn + i;
-            const int j1 = (seg + 1) * len < nat ? (seg + 1) * len : nat;
-            double y = 0.0;
-            constexpr int NJ = 8;
-            for (int j0 = seg * len; j0 < j1; j0 += NJ) {
-                double ds[NJ];
+        for (int a = tid - 64; a < nsh; a += kNT - 64) {
+            const int at = ss.sh[a].at, k0 = ss.refoff[at], nk = ss.refoff[at + 1] - k0;
+            double vdisp = 0.0;
 #pragma unroll
-                for (int u = 0; u < NJ; ++u) ds[u] = dsp[(j0 + u < j1 ? j0 + u : j0) * nat];
-                qx_sched_fence();
-#pragma unroll
-                for (int u = 0; u < NJ; ++u)
-                    if (j0 + u < j1) y += ds[u] * t[j0 + u];
-            }
-            py[p] = y;
-            ed4 += -0.5 * ss.zr[k] * y;
+            for (int k = 0; k < QX_MAX_REF; ++k)
+                if (k < nk) vdisp += ss.dzr[k0 + k];
+            vs[a] += pa[at] + vdisp;
         }
     }
-    __syncthreads();
-    for (int a = tid; a < nsh; a += kNT) {
-        const int at = ss.sh[a].at;
-        double vdisp = 0.0;
-        for (int k = ss.refoff[at]; k < ss.refoff[at + 1]; ++k) {
-            double y = py[k];
-            for (int s = 1; s < nseg; ++s) y += py[s * nd + k];
-            vdisp += -ss.dzr[k] * y;
-        }
-        vs[a] += ss.vat[at] + vdisp;
+    if (energy) {
+        double e5[5] = {es2, es3, eaes, eaxc, ed4};
+        block_sums<5>(e5, ss.red);
+        if (tid == 0)
+            for (int k = 0; k < 5; ++k) ss.eparts[k] = e5[k];
     }
-    double e5[5] = {es2, es3, eaes, eaxc, ed4};
-    block_sums<5>(e5, ss.red);
-    if (tid == 0)
-        for (int k = 0; k < 5; ++k) ss.eparts[k] = e5[k];
     __syncthreads();
 }
 
@@ -1440,6 +1492,8 @@ QX_DEV void scc_body(int sys, const SysInfo& si, BatchRef B0, OptRef opt, SysSha
     __syncthreads();
     QX_PH(11);
 
+    PotTables pt;
+    pt.load(si, qx_fresh(B0), ss);
     int hcount = 0;
     if (opt.keep > 0 && warm >= 1) {
         const double* hcnt = B0.hist + si.hist_off + 2 * (size_t)opt.mem * nx + 2 * (size_t)opt.mem * opt.mem +
@@ -1452,7 +1506,7 @@ QX_DEV void scc_body(int sys, const SysInfo& si, BatchRef B0, OptRef opt, SysSha
     // each iteration takes the potentials twice, at the input and at the
     // output moments (one copy of their code)
     for (bool out = false;; out = !out) {
-        potentials(si, qx_fresh(B0), ss, out ? xout : xin, vs, vd, vq, bf.pot);
+        potentials(si, qx_fresh(B0), ss, pt, out ? xout : xin, vs, vd, vq, bf.pot, out);
         if (!out) {
             QX_PH(0);
             {
@@ -1690,7 +1744,7 @@ QX_DEV void scc_system(BatchRef B, OptRef opt, int sys, SccLds& L, double* dyn)
         // a fifth matrix after the row sums when the launch's LDS holds it
         double* E = EIG && 5 * mm + kRs * m <= opt.lds_doubles ? dyn + 4 * mm + kRs * m : nullptr;
         // A and F are free at the potentials, P and the row sums are not
-        double* pot = dyn + (pot_lds(si.nat, si.ndim) <= 2 * mm ? mm : 4 * mm + kRs * m);
+        double* pot = dyn + (pot_lds(si.nat) <= 2 * mm ? mm : 4 * mm + kRs * m);
         SccBuffers bf{dyn + mm, dyn, dyn + 2 * mm, dyn + 3 * mm, dyn + 4 * mm, m + 1, E, dyn + mm,
                       opt.lds_doubles - mm, pot};
         scc_body<true, EIG>(sys, si, B, opt, L.ss, bf, L);
