@@ -48,6 +48,7 @@ std::mutex g_mu;
 bool g_ready = false;
 int g_device = -1;
 hipStream_t g_stream = nullptr;
+size_t g_setup_dyn_max = 0;  // dynamic LDS of the setup kernel
 size_t g_scc_dyn_max = 0;  // dynamic LDS the SCC kernels may take (set at init)
 unsigned char* g_scratch_dev = nullptr;  // device address of scratch on g_device
 std::mutex g_scratch_mu;                 // one allocation-free call at a time
@@ -247,9 +248,10 @@ int ensure_init(int device)
                                (int)g_scc_dyn_max));
     HIPCHK(hipFuncSetAttribute((const void*)qx::k_scc<true>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                (int)g_scc_dyn_max));
+    HIPCHK(hipFuncGetAttributes(&fa, (const void*)qx::k_setup));
+    g_setup_dyn_max = (size_t)lds_block - fa.sharedSizeBytes - kLdsReserve;
     HIPCHK(hipFuncSetAttribute((const void*)qx::k_setup, hipFuncAttributeMaxDynamicSharedMemorySize,
-                               (QX_LDS_MAXM * QX_LDS_MAXM + QX_LDS_MAXM * (QX_LDS_MAXM | 1)) *
-                                   (int)sizeof(double)));
+                               (int)g_setup_dyn_max));
     HIPCHK(hipFuncSetAttribute((const void*)qx::k_grad, hipFuncAttributeMaxDynamicSharedMemorySize, 0));
     HIPCHK(hipFuncSetAttribute((const void*)qx::k_md_fused<false>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                (int)g_scc_dyn_max));
@@ -574,11 +576,16 @@ int collect_times()
     return QCXMS_OK;
 }
 
-size_t lds_setup_bytes(const qcxms_batch* b)
+// the triangles of the overlap's factorisation, of the largest system whose
+// triangles fit (cap: the launch's limit)
+size_t lds_setup_bytes(const qcxms_batch* b, size_t cap)
 {
-    // Cholesky factor and the columns of its inverse
-    const size_t ls = std::min(b->max_ld, QX_LDS_MAXM);
-    return sizeof(double) * (ls * ls + ls * (ls | 1));
+    size_t need = 0;
+    for (const SysInfo& si : b->info) {
+        const size_t t = sizeof(double) * (size_t)si.nao * (si.nao + 2);
+        if (t <= cap) need = std::max(need, t);
+    }
+    return need;
 }
 // Dynamic LDS of an SCC launch.  Systems with their matrices in LDS: four
 // m x m working matrices and the AO row sums, a fifth matrix for the MFMA
@@ -696,9 +703,10 @@ int enqueue_scc_plan(qcxms_batch* b)
 int enqueue_egrad(qcxms_batch* b, bool with_grad)
 {
     int st;
-    const size_t l1 = lds_setup_bytes(b), l2 = lds_scc_bytes(b);
+    const size_t l1 = lds_setup_bytes(b, g_setup_dyn_max), l2 = lds_scc_bytes(b);
     if ((st = timed(b, b->t_setup, [&] {
-             hipLaunchKernelGGL(qx::k_setup, dim3(b->nsys), dim3(QX_BLOCK), l1, b->stream, b->d, 1);
+             hipLaunchKernelGGL(qx::k_setup, dim3(b->nsys), dim3(QX_BLOCK), l1, b->stream, b->d, 1,
+                                (int)(l1 / sizeof(double)));
          })))
         return st;
     int plan_st = QCXMS_OK;
@@ -1607,7 +1615,7 @@ int md_enqueue(qcxms_md* md)
 int md_enqueue_fused(qcxms_md* md, int nsteps)
 {
     qcxms_batch* b = md->b;
-    const size_t lds = std::max(lds_setup_bytes(b), lds_scc_bytes(b));
+    const size_t lds = std::max(lds_setup_bytes(b, g_scc_dyn_max), lds_scc_bytes(b));
     return timed(b, b->t_fused, [&] {
         hipLaunchKernelGGL(b->opts.eig_mfma ? qx::k_md_fused<true> : qx::k_md_fused<false>, dim3(md->ntraj),
                            dim3(QX_SCC_BLOCK), lds, b->stream,

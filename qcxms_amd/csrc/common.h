@@ -16,7 +16,6 @@
 #define QX_MAX_NSH 128
 #define QX_MAX_NAO 256
 #define QX_MAX_REF 7
-#define QX_LDS_MAXM 64  // Jacobi matrices up to this order live in LDS
 #define QX_PAIR_STRIDE 16  // doubles per ordered atom pair in the gradient pair buffer
 #define QX_PAIR_KERN 3     // kernel planes per ordered atom pair
 

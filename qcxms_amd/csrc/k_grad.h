@@ -303,10 +303,10 @@ QX_DEV void grad_system(BatchRef B, int sys, GradLds& Lg)
         double sr = 0.0;  // radial factor times 1/r
         // repulsion
         if (r <= gfn2::kRepCutoff) {
-            const double kexp = (ea.z <= 2 && eb.z <= 2) ? gfn2::kRepKexpLight : gfn2::kRepKexp;
-            const double sa = sqrt(ea.rep_alpha * eb.rep_alpha);
-            const double e = ea.rep_zeff * eb.rep_zeff / r * exp(-sa * pow(r, kexp));
-            sr += e * (-1.0 / r - sa * kexp * pow(r, kexp - 1.0)) / r;
+            const bool light = ea.z <= 2 && eb.z <= 2;  // exponent 1, else 3/2
+            const double sa = sqrt(ea.rep_alpha * eb.rep_alpha), rr = light ? 1.0 : sqrt(r);
+            const double e = ea.rep_zeff * eb.rep_zeff / r * exp(-sa * (r * rr));
+            sr += e * (-1.0 / r - sa * (light ? 1.0 : 1.5) * rr) / r;
         }
         // ES2: -q_s q_t gamma^3 R
         for (int s = ss.shoff[a]; s < ss.shoff[a + 1]; ++s) {
@@ -396,7 +396,7 @@ QX_DEV void grad_system(BatchRef B, int sys, GradLds& Lg)
                 const double r3 = 1.0 / (uvw * rijk);
                 const double atm = (0.375 * tt + 1.0) * r3;
                 const double alp3 = gfn2::kD4Alp / 3.0;
-                const double x = pow(cijk / rijk, alp3);
+                const double x = d4_pow(cijk / rijk);
                 const double fd = 1.0 / (1.0 + 6.0 * x);
                 const double c6ac = pb[(size_t)(a * nat + c) * kPairStride + 10];
                 const double c6bc = pb[(size_t)(b * nat + c) * kPairStride + 10];

@@ -759,7 +759,10 @@ __global__ __launch_bounds__(QX_SCC_BLOCK) void k_md_fused(MdArgs args)
         __syncthreads();
         QX_FUSED_PH(24);
         if (!qx_uniform(fresh().M.active[sys])) break;
-        setup_system(fresh().B, sys, 1, L.s, dyn);
+        {
+            QX_ARG(MdArgs) a = fresh();
+            setup_system(a.B, sys, 1, L.s, dyn, a.opt.lds_doubles);
+        }
         __syncthreads();
         QX_FUSED_PH(25);
         {

@@ -7,6 +7,16 @@
 
 namespace qx {
 
+// x^(alp / 3) of the ATM damping, and the exponents of the repulsion are
+// r^1 (H-H) and r^(3/2): roots instead of the general power
+QX_DEV double d4_pow(double x)
+{
+    static_assert(gfn2::kD4Alp == 16.0 && gfn2::kRepKexp == 1.5 && gfn2::kRepKexpLight == 1.0,
+                  "powers written as roots");
+    const double x2 = x * x;
+    return x2 * x2 * x * cbrt(x);
+}
+
 QX_DEV double d4_zeta(double a, double c, double qref, double qmod)
 {
     if (qmod < 0.0) return exp(a);
@@ -142,6 +152,100 @@ QX_DEV void setup_shell_row(const ShellDesc& sa, const ShellDesc& sb, const Elem
     }
 }
 
+// Cholesky factor L of S and X = L^-T in LDS: S = U D^-1 U^T column by column
+// (column j of U is the column of S as the elimination reaches it), the
+// identity eliminated along with it, so that after the last column it is the
+// inverse of the unit factor.  Row i of a step has the same i + 1 entries in
+// every step (0 .. j of the inverse, j + 1 .. i of S), half a wavefront takes
+// a row, and there is one barrier per column.  Both triangles are packed by
+// rows; a: n (n + 2) doubles.
+// (26-atom C8H18+, 50 basis functions: 82 us as a right-looking Cholesky of two
+// barriers per column followed by one thread per column of the inverse; 132
+// basis functions in global memory: 1.5 ms.)
+QX_DEV void factor_lds(const double* S, double* Lg, double* Xg, int n, int ld, double* a)
+{
+    constexpr int NR = QX_BLOCK / 32;
+    const int tid = qx_tid(), q0 = tid & 31, r0 = tid >> 5;
+    double* e = a + n * (n + 1) / 2;
+    double* rd = e + n * (n + 1) / 2;  // 1 / L_jj
+    __syncthreads();
+    for (int i = r0; i < n; i += NR)
+        for (int q = q0; q <= i; q += 32) {
+            a[i * (i + 1) / 2 + q] = S[i * ld + q];
+            e[i * (i + 1) / 2 + q] = q == i ? 1.0 : 0.0;
+        }
+    __syncthreads();
+    for (int j = 0; j < n - 1; ++j) {
+        const double inv = 1.0 / a[j * (j + 1) / 2 + j];
+        const double* ej = e + j * (j + 1) / 2;
+        for (int i = j + 1 + r0; i < n; i += NR) {
+            double* ai = a + i * (i + 1) / 2;
+            double* ei = e + i * (i + 1) / 2;
+            const double l = ai[j] * inv;
+            for (int q = q0; q <= i; q += 32) {
+                if (q <= j) ei[q] -= l * ej[q];
+                else ai[q] -= l * a[q * (q + 1) / 2 + j];
+            }
+        }
+        __syncthreads();
+    }
+    for (int j = tid; j < n; j += QX_BLOCK) rd[j] = 1.0 / sqrt(a[j * (j + 1) / 2 + j]);
+    __syncthreads();
+    for (int i = r0; i < ld; i += NR)
+        for (int q = q0; q < ld; q += 32) {
+            Lg[i * ld + q] = (i < n && q <= i) ? a[i * (i + 1) / 2 + q] * rd[q] : 0.0;
+            // row q of X is column q of L^-1
+            Xg[i * ld + q] = (q < n && i <= q) ? e[q * (q + 1) / 2 + i] * rd[q] : 0.0;
+        }
+}
+
+// The same in global memory, for systems whose triangles do not fit in LDS.
+QX_DEV void factor_global(const double* S, double* A, double* Xg, int n, int ld)
+{
+    const int tid = qx_tid();
+    const size_t ms = (size_t)ld * ld;
+    __syncthreads();
+    for (size_t i = tid; i < ms; i += QX_BLOCK) A[i] = S[i];
+    __syncthreads();
+    for (int j = 0; j < n; ++j) {
+        // every thread takes the pivot's root itself; thread 0 stores it
+        // while the others update the trailing block (two barriers a column)
+        const double d = sqrt(A[(size_t)j * ld + j]);
+        for (int i = j + 1 + tid; i < n; i += QX_BLOCK) A[(size_t)i * ld + j] /= d;
+        __syncthreads();
+        if (tid == 0) A[(size_t)j * ld + j] = d;
+        // trailing lower triangle: row j + 1 + r by lane r, its columns
+        // j + 1 + c (c <= r) by the wavefronts in turn
+        const int m = n - j - 1;
+        for (int r = tid & 63; r < m; r += 64) {
+            const int i = j + 1 + r;
+            const double lij = A[(size_t)i * ld + j];
+            for (int c = tid >> 6; c <= r; c += QX_BLOCK / 64) {
+                const int k = j + 1 + c;
+                A[(size_t)i * ld + k] -= lij * A[(size_t)k * ld + j];
+            }
+        }
+        __syncthreads();
+    }
+    for (size_t p = tid; p < ms; p += QX_BLOCK) {
+        const int i = (int)(p / ld), k = (int)(p % ld);
+        if (!(k <= i && i < n)) A[p] = 0.0;
+        Xg[p] = 0.0;
+    }
+    __syncthreads();
+    // X = (L^-1)^T: column c of L^-1 by forward substitution (thread c),
+    // written as row c of X
+    for (int c = tid; c < n; c += QX_BLOCK) {
+        double* xr = Xg + (size_t)c * ld;  // X[c][i] = Linv[i][c]
+        for (int i = c; i < n; ++i) {
+            double v = (i == c) ? 1.0 : 0.0;
+#pragma unroll 8
+            for (int k = c; k < i; ++k) v -= A[(size_t)i * ld + k] * xr[k];
+            xr[i] = v / A[(size_t)i * ld + i];
+        }
+    }
+}
+
 // ---------------------------------------------------------------------------
 // LDS of one system's setup (the Cholesky factor uses the dynamic LDS)
 struct SetupLds {
@@ -156,7 +260,8 @@ struct SetupLds {
     double zg[QX_MAX_REF * QX_MAX_NAT];
 };
 
-QX_DEV void setup_system(BatchRef B, int sys, int with_chol, SetupLds& Ls, double* dyn)
+// dyn: ndyn doubles of LDS for the factorisation
+QX_DEV void setup_system(BatchRef B, int sys, int with_chol, SetupLds& Ls, double* dyn, int ndyn)
 {
     const SysInfo si = qx_info(B, sys);
     const int tid = qx_tid();
@@ -361,8 +466,8 @@ QX_DEV void setup_system(BatchRef B, int sys, int with_chol, SetupLds& Ls, doubl
                      dz = sx[3 * i + 2] - sx[3 * j + 2];
         const double r = sqrt(dx * dx + dy * dy + dz * dz);
         if (r > gfn2::kRepCutoff) continue;
-        const double kexp = (ei.z <= 2 && ej.z <= 2) ? gfn2::kRepKexpLight : gfn2::kRepKexp;
-        erep += ei.rep_zeff * ej.rep_zeff / r * exp(-sqrt(ei.rep_alpha * ej.rep_alpha) * pow(r, kexp));
+        erep += ei.rep_zeff * ej.rep_zeff / r *
+                exp(-sqrt(ei.rep_alpha * ej.rep_alpha) * (ei.z <= 2 && ej.z <= 2 ? r : r * sqrt(r)));
     }
     erep = block_sum(erep, red);
     // 8. ATM energy at zero charges: pair C6 into scratch, then triples
@@ -413,7 +518,7 @@ QX_DEV void setup_system(BatchRef B, int sys, int with_chol, SetupLds& Ls, doubl
                 const double uvw = u * v * w, rijk = sqrt(uvw), cijk = cij * cjk * cik;
                 const double aa = u + v - w, bb = u + w - v, cc = w + v - u;
                 const double atm = (0.375 * aa * bb * cc / uvw + 1.0) / (rijk * rijk * rijk);
-                const double x = pow(cijk / rijk, gfn2::kD4Alp / 3.0);
+                const double x = d4_pow(cijk / rijk);
                 const double fd = 1.0 / (1.0 + 6.0 * x);
                 const double c9 = gfn2::kD4S9 * sqrt(c60[i * nat + j] * c60[j * nat + k] * c60[i * nat + k]);
                 eatm += c9 * atm * fd;
@@ -435,76 +540,17 @@ QX_DEV void setup_system(BatchRef B, int sys, int with_chol, SetupLds& Ls, doubl
     }
     if (!with_chol) return;
     // 9. Cholesky S = L L^T and X = L^-T
-    double* A = (ld <= QX_LDS_MAXM) ? dyn : (B.L + si.mat_off);
-    double* Lg = B.L + si.mat_off;
-    double* Xg = B.X + si.mat_off;
-    __syncthreads();
-    for (size_t i = tid; i < ms; i += QX_BLOCK) A[i] = S[i];
-    __syncthreads();
-    for (int j = 0; j < n; ++j) {
-        // every thread takes the pivot's root itself; thread 0 stores it
-        // while the others update the trailing block (two barriers a column)
-        const double d = sqrt(A[(size_t)j * ld + j]);
-        for (int i = j + 1 + tid; i < n; i += QX_BLOCK) A[(size_t)i * ld + j] /= d;
-        __syncthreads();
-        if (tid == 0) A[(size_t)j * ld + j] = d;
-        // trailing lower triangle: row j + 1 + r by lane r, its columns
-        // j + 1 + c (c <= r) by the wavefronts in turn
-        const int m = n - j - 1;
-        for (int r = tid & 63; r < m; r += 64) {
-            const int i = j + 1 + r;
-            const double lij = A[(size_t)i * ld + j];
-            for (int c = tid >> 6; c <= r; c += QX_BLOCK / 64) {
-                const int k = j + 1 + c;
-                A[(size_t)i * ld + k] -= lij * A[(size_t)k * ld + j];
-            }
-        }
-        __syncthreads();
-    }
-    // zero the upper triangle, store L
-    for (size_t p = tid; p < ms; p += QX_BLOCK) {
-        const int i = (int)(p / ld), k = (int)(p % ld);
-        const double v = (k <= i && i < n) ? A[p] : 0.0;
-        A[p] = v;
-        Lg[p] = v;
-    }
-    __syncthreads();
-    // X = (L^-1)^T: column c of L^-1 by forward substitution (thread c),
-    // written as row c of X.  With the factor in LDS the columns are built in
-    // LDS too (rows of odd stride) and copied out once.
-    const bool lx = ld <= QX_LDS_MAXM;
-    const int xs = n | 1;
-    double* xl = dyn + (size_t)ld * ld;
-    if (!lx) {
-        for (size_t p = tid; p < ms; p += QX_BLOCK) Xg[p] = 0.0;
-        __syncthreads();
-    }
-    for (int c = tid; c < n; c += QX_BLOCK) {
-        double* xr = lx ? xl + (size_t)c * xs : Xg + (size_t)c * ld;  // X[c][i] = Linv[i][c]
-        for (int i = c; i < n; ++i) {
-            double v = (i == c) ? 1.0 : 0.0;
-#pragma unroll 8
-            for (int k = c; k < i; ++k) v -= A[(size_t)i * ld + k] * xr[k];
-            xr[i] = v / A[(size_t)i * ld + i];
-        }
-    }
-    if (lx) {
-        __syncthreads();
-        for (size_t p = tid; p < ms; p += QX_BLOCK) {
-            const int c = (int)(p / ld), i = (int)(p % ld);
-            Xg[p] = (c < n && i >= c && i < n) ? xl[(size_t)c * xs + i] : 0.0;
-        }
-    }
-    // X as stored: row c holds column c of L^-1, i.e. Xg = (L^-1)^T row-major
+    if (n * (n + 2) <= ndyn) factor_lds(S, B.L + si.mat_off, B.X + si.mat_off, n, ld, dyn);
+    else factor_global(S, B.L + si.mat_off, B.X + si.mat_off, n, ld);
 }
 
-__global__ __launch_bounds__(QX_BLOCK) void k_setup(BatchPtrs B, int with_chol)
+__global__ __launch_bounds__(QX_BLOCK) void k_setup(BatchPtrs B, int with_chol, int ndyn)
 {
     const int sys = blockIdx.x;
     if (B.active && !B.active[sys]) return;
     __shared__ SetupLds Ls;
     extern __shared__ double dyn[];
-    setup_system(qx_args(B), sys, with_chol, Ls, dyn);
+    setup_system(qx_args(B), sys, with_chol, Ls, dyn, ndyn);
 }
 
 }  // namespace qx
