@@ -277,7 +277,7 @@ struct Timer {
 struct qcxms_batch {
     int nsys = 0;
     std::vector<SysInfo> info;
-    std::vector<int> elem;
+    std::vector<int> elem, order;
     std::vector<int2> items;  // shell-pair work items of all systems
     int natoms = 0, nshells = 0, nrefs = 0, nxtot = 0;
     size_t mat_total = 0, gam_total = 0, hist_total = 0, pair_total = 0;
@@ -456,6 +456,13 @@ int allocate(qcxms_batch* b)
     if ((st = dalloc(b, &(ptr), (size_t)(n))) != 0) return st;
     ALLOC(b->d_info, b->nsys);
     ALLOC(b->d_elem, b->natoms);
+    int* d_order = nullptr;
+    ALLOC(d_order, b->nsys);
+    d.order = d_order;
+    b->order.resize(b->nsys);
+    for (int s = 0; s < b->nsys; ++s) b->order[s] = s;
+    std::stable_sort(b->order.begin(), b->order.end(),
+                     [&](int x, int y) { return b->info[x].nao > b->info[y].nao; });
     int2* d_items = nullptr;
     ALLOC(d_items, b->items.size());
     d.spitem = d_items;
@@ -526,6 +533,7 @@ int allocate(qcxms_batch* b)
     if (!b->items.empty())
         HIPCHK(hipMemcpyAsync(d_items, b->items.data(), sizeof(int2) * b->items.size(), hipMemcpyHostToDevice,
                               b->stream));
+    HIPCHK(hipMemcpyAsync(d_order, b->order.data(), sizeof(int) * b->nsys, hipMemcpyHostToDevice, b->stream));
     HIPCHK(hipMemcpyAsync(b->d_info, b->info.data(), sizeof(SysInfo) * b->nsys, hipMemcpyHostToDevice, b->stream));
     HIPCHK(hipMemcpyAsync(b->d_elem, b->elem.data(), sizeof(int) * b->natoms, hipMemcpyHostToDevice, b->stream));
     return QCXMS_OK;
@@ -632,7 +640,7 @@ SccOpts launch_opts(const qcxms_batch* b, size_t lds)
     SccOpts o = b->opts;
     o.lds_doubles = (int)(lds / sizeof(double));
     o.lds_max_m = qx::kFastM;
-    o.first_sys = 0;
+    o.first_sys = -1;
     return o;
 }
 
@@ -658,7 +666,7 @@ int enqueue_scc_plan(qcxms_batch* b)
         if (runs.empty() || runs.back().bin != k) runs.push_back({s, s + 1, k});
         else runs.back().s1 = s + 1;
     }
-    auto launch = [&](const Run& r, hipStream_t st) {
+    auto launch = [&](const Run& r, hipStream_t st, int first) {
         const TuneBin& t = r.bin >= 0 ? b->tune[r.bin] : b->tune_mixed;
         const int lmax = t.lds ? qx::kFastM : 0;
         const size_t lds = lds_scc_bytes_range(b, r.s0, r.s1, lmax, t.eig);
@@ -666,18 +674,18 @@ int enqueue_scc_plan(qcxms_batch* b)
         o.eig_mfma = t.eig;
         o.lds_doubles = (int)(lds / sizeof(double));
         o.lds_max_m = lmax;
-        o.first_sys = r.s0;
+        o.first_sys = first;
         hipLaunchKernelGGL(t.eig ? qx::k_scc<true> : qx::k_scc<false>, dim3(r.s1 - r.s0), dim3(QX_SCC_BLOCK),
                            lds, st, qx::SccArgs{b->d, o});
         return hipGetLastError();
     };
     if (runs.size() == 1) {
-        HIPCHK(launch(runs[0], b->stream));
+        HIPCHK(launch(runs[0], b->stream, -1));
         return QCXMS_OK;
     }
     if (b->tune_mixed.eig >= 0) {
         // systems of several bins in one launch with the mixed choice
-        HIPCHK(launch(Run{0, b->nsys, -1}, b->stream));
+        HIPCHK(launch(Run{0, b->nsys, -1}, b->stream, -1));
         return QCXMS_OK;
     }
     if (!b->fork) {
@@ -691,7 +699,7 @@ int enqueue_scc_plan(qcxms_batch* b)
     const int nside = std::min<int>((int)runs.size(), qcxms_batch::kSide);
     for (int k = 0; k < nside; ++k) HIPCHK(hipStreamWaitEvent(b->side[k], b->fork, 0));
     // largest systems first (the batch's order), dealt round-robin
-    for (size_t r = 0; r < runs.size(); ++r) HIPCHK(launch(runs[r], b->side[r % nside]));
+    for (size_t r = 0; r < runs.size(); ++r) HIPCHK(launch(runs[r], b->side[r % nside], runs[r].s0));
     for (int k = 0; k < nside; ++k) {
         HIPCHK(hipEventRecord(b->join[k], b->side[k]));
         HIPCHK(hipStreamWaitEvent(b->stream, b->join[k], 0));

@@ -219,13 +219,16 @@ struct SccOpts {
     int eig_mfma;     // 1: MFMA simultaneous-rotation eigen refinement before Jacobi
     int lds_max_m;    // systems of at most this (even) basis size keep their SCC matrices in
                       // LDS, the others in global memory (set per launch, <= qx::kFastM)
-    int first_sys;    // system of workgroup 0 (a launch over a range of the batch's systems)
+    int first_sys;    // system of workgroup 0 (a launch over a range of the batch's systems); -1: all
+                      // systems in the batch's launch order
 };
 
 // Device-resident batch state.  Every pointer is a flat array over all systems.
 struct BatchPtrs {
     int nsys;
     const SysInfo* info;
+    const int* order; // systems by decreasing basis size: workgroup k of a launch over all takes
+                      // order[k], so the longest run first and the short ones fill the end
     const int* elem;  // per atom: element slot
     double* xyz;      // 3 per atom
     double* grad;     // 3 per atom

@@ -522,7 +522,7 @@ QX_DEV void grad_system(BatchRef B, int sys, GradLds& Lg)
 
 __global__ __launch_bounds__(QX_BLOCK) void k_grad(BatchPtrs B)
 {
-    const int sys = blockIdx.x;
+    const int sys = B.order[blockIdx.x];
     if (B.active && !B.active[sys]) return;
     __shared__ GradLds Lg;
     if (B.dblk) grad_system<true>(qx_args(B), sys, Lg);

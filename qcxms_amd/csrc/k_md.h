@@ -728,7 +728,7 @@ __global__ __launch_bounds__(QX_SCC_BLOCK) void k_md_fused(MdArgs args)
 {
     static_assert(QX_SCC_BLOCK == QX_BLOCK, "the fused phases assume one block size");
     QX_ARG(MdArgs) a0 = qx_args(args);
-    const int sys = blockIdx.x;
+    const int sys = qx_uniform(a0.B.order[blockIdx.x]);
     __shared__ FusedLds L;
     extern __shared__ double dyn[];
 #ifdef QX_PHASE_TIMING

@@ -1765,7 +1765,7 @@ template <bool EIG>
 __global__ __launch_bounds__(kNT) void k_scc(SccArgs args)
 {
     QX_ARG(SccArgs) a = qx_args(args);
-    const int sys = a.opt.first_sys + blockIdx.x;
+    const int sys = qx_uniform(a.opt.first_sys < 0 ? a.B.order[blockIdx.x] : a.opt.first_sys + (int)blockIdx.x);
     if (a.B.active && !a.B.active[sys]) return;
     __shared__ SccLds L;
     extern __shared__ double dyn[];

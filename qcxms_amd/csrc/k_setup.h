@@ -546,7 +546,7 @@ QX_DEV void setup_system(BatchRef B, int sys, int with_chol, SetupLds& Ls, doubl
 
 __global__ __launch_bounds__(QX_BLOCK) void k_setup(BatchPtrs B, int with_chol, int ndyn)
 {
-    const int sys = blockIdx.x;
+    const int sys = B.order[blockIdx.x];
     if (B.active && !B.active[sys]) return;
     __shared__ SetupLds Ls;
     extern __shared__ double dyn[];
