@@ -93,7 +93,11 @@ typedef double qx_d4 __attribute__((ext_vector_type(4)));
 // the edge read the last row or column (their results are not stored); only
 // the last k step is masked.  The operands of the next four k steps are
 // loaded while the matrix cores work on the current four, so a strip waits
-// for memory once.
+// for memory once.  Up to 56 columns a product is bound by that wait and the
+// tail, above by the L1 traffic of the operands (16 lines per load of A).
+// (A product of the eigenvector refinement with every strip formed -> now, in
+// cycles: 88 columns 12.9 k -> 12.2 k, 98: 38 k -> 34 k, 132: 129 k -> 114 k,
+// where the matrix cores need 43 k for all and half of it for the symmetric.)
 QX_DEV void mfma_gemm(int M, int N, int K, const double* A, int ai, int ak, const double* Bm, int bk,
                       int bj, double* Cm, int ldc, const double* d, bool sym)
 {
@@ -529,32 +533,40 @@ QX_DEV void jacobi_rounds_global(const JacobiBuffers& jb, int m, double tol, dou
     }
 }
 
-// Columns of the nrow x m matrix Cv rotated by the logged sweep, any m: a
-// lane per pair slot (NS slots per lane) and NR rows per wavefront at a time
-// in registers, the players
-// moved between the lanes after every round, NR rows per wavefront at a time.
-template <int NS, int NR>
-QX_DEV void jacobi_replay_slots(const JacobiBuffers& jb, double* Cv, int m, int nrow, int lda)
+// Columns of the nrow x m matrix Cv rotated by the logged sweep, m <= 2 NL NS.
+// 64 / NL rows share a wavefront, NL lanes each; a lane holds NS consecutive
+// pair slots of its row in registers, the players as in jacobi_rounds (x the p and y
+// the q players, in slot 0 the other way round), so that in the move after a
+// round only one player of x and one of y change the lane and the others the
+// register.  NR such sets of rows at a time.  Without LDS traffic or barriers a
+// round is bound by the instructions issued.
+// (Cycles a round with one row per wavefront and slots 64 apart -> now: 132
+// rows and columns 6.0 k -> 2.9 k, where the second set had used 2 lanes of 64;
+// 98: 1.75 k -> 1.50 k.)
+template <int NL, int NS, int NR>
+QX_DEV void jacobi_replay(const JacobiBuffers& jb, double* Cv, int m, int nrow, int lda)
 {
-    constexpr int NW = kNT / 64;
+    constexpr int NG = 64 / NL, NW = kNT / 64;
     const int tid = qx_tid(), lane = tid & 63, wave = qx_wave(tid), half = m / 2;
-    for (int i0 = 0; i0 < nrow; i0 += NW * NR) {
-        double p[NR][NS], q[NR][NS];
+    const int s0 = (lane & (NL - 1)) * NS;
+    const bool first = s0 == 0;
+    for (int i0 = 0; i0 < nrow; i0 += NG * NW * NR) {
+        double x[NR][NS], y[NR][NS];
 #pragma unroll
         for (int u = 0; u < NR; ++u) {
-            const int i = i0 + wave + NW * u < nrow ? i0 + wave + NW * u : nrow - 1;
+            const int row = i0 + NG * (wave + NW * u) + lane / NL, i = row < nrow ? row : nrow - 1;
 #pragma unroll
             for (int t = 0; t < NS; ++t) {
-                const int k = lane + 64 * t < half ? lane + 64 * t : half - 1;
-                p[u][t] = Cv[i * lda + k];
-                q[u][t] = Cv[i * lda + m - 1 - k];
+                const int k = s0 + t < half ? s0 + t : half - 1;
+                x[u][t] = Cv[i * lda + (k == 0 ? m - 1 : k)];
+                y[u][t] = Cv[i * lda + (k == 0 ? 0 : m - 1 - k)];
             }
         }
         double2 cs[NS];
         auto fetch = [&](int r) {
 #pragma unroll
             for (int t = 0; t < NS; ++t) {
-                const int k = lane + 64 * t < half ? lane + 64 * t : half - 1;
+                const int k = s0 + t < half ? s0 + t : half - 1;
                 cs[t] = jb.log[r * half + k];
             }
         };
@@ -563,45 +575,41 @@ QX_DEV void jacobi_replay_slots(const JacobiBuffers& jb, double* Cv, int m, int 
             double2 cr[NS];
 #pragma unroll
             for (int t = 0; t < NS; ++t) cr[t] = cs[t];
+            if (first) cr[0].y = -cr[0].y;
             if (r + 1 < m - 1) fetch(r + 1);
-            if (qx_uniform(jb.any[r])) {
-#pragma unroll
-                for (int u = 0; u < NR; ++u)
-#pragma unroll
-                    for (int t = 0; t < NS; ++t) {
-                        const double x = p[u][t], y = q[u][t];
-                        p[u][t] = cr[t].x * x - cr[t].y * y;
-                        q[u][t] = cr[t].y * x + cr[t].x * y;
-                    }
-            }
-            // p players one slot down, q players one up (rr_move)
+            const bool any = qx_uniform(jb.any[r]);
 #pragma unroll
             for (int u = 0; u < NR; ++u) {
-                double np[NS], nq[NS];
+                if (i0 + NG * (wave + NW * u) >= nrow) continue;
+                double px[NS], py[NS];
 #pragma unroll
                 for (int t = 0; t < NS; ++t) {
-                    const int k = lane + 64 * t;
-                    const double down = qx_lane_up(p[u][t], t + 1 < NS ? qx_bcast(p[u][t + 1 < NS ? t + 1 : t], 0) : 0.0);
-                    np[t] = k == half - 1 ? q[u][t] : down;
-                    const double y = k == 0 ? p[u][t] : q[u][t];  // p of slot 0 turns round to q of slot 1
-                    nq[t] = qx_lane_down(y, t > 0 ? qx_bcast(q[u][t > 0 ? t - 1 : 0], 63) : q[u][0]);
+                    px[t] = x[u][t];
+                    py[t] = y[u][t];
+                    if (any) {
+                        px[t] = cr[t].x * x[u][t] - cr[t].y * y[u][t];
+                        py[t] = cr[t].y * x[u][t] + cr[t].x * y[u][t];
+                    }
                 }
+                const double xin = qx_lane_up(px[0], 0.0), yin = qx_lane_down(py[NS - 1], 0.0);
 #pragma unroll
                 for (int t = 0; t < NS; ++t) {
-                    p[u][t] = np[t];
-                    q[u][t] = nq[t];
+                    const double down = t + 1 < NS ? px[t + 1 < NS ? t + 1 : t] : xin;
+                    const double up = t > 0 ? py[t > 0 ? t - 1 : 0] : yin;
+                    x[u][t] = s0 + t == half - 1 ? py[t] : t == 0 && first ? px[0] : down;
+                    y[u][t] = t == 0 && first ? px[1] : up;
                 }
             }
         }
 #pragma unroll
         for (int u = 0; u < NR; ++u) {
-            const int i = i0 + wave + NW * u;
+            const int i = i0 + NG * (wave + NW * u) + lane / NL;
 #pragma unroll
             for (int t = 0; t < NS; ++t) {
-                const int k = lane + 64 * t;
+                const int k = s0 + t;
                 if (i < nrow && k < half) {
-                    Cv[i * lda + k] = p[u][t];
-                    Cv[i * lda + m - 1 - k] = q[u][t];
+                    Cv[i * lda + (k == 0 ? m - 1 : k)] = x[u][t];
+                    Cv[i * lda + (k == 0 ? 0 : m - 1 - k)] = y[u][t];
                 }
             }
         }
@@ -689,10 +697,18 @@ QX_DEV int jacobi(double* A, double* Cv, int m, int nrow, int lda, double tol, i
         if constexpr (LDS) jacobi_rounds<NB, NR>(jb, m, nrow, tol, min_s, x, y, f);
         else jacobi_rounds_global(jb, m, tol, min_s, f, g);
         if (!LDS) blk = jb.gblk[g];
-        if (!rows) {
+        if constexpr (!rows) {
             __syncthreads();
-            if (m <= 128) jacobi_replay_slots<1, 6>(jb, Cv, m, nrow, lda);
-            else jacobi_replay_slots<2, 6>(jb, Cv, m, nrow, lda);
+            // sizes of the instantiation (jacobi_any): up to 102, 132, 256; the
+            // split that gives the longest wavefront the fewest rotations
+            if constexpr (NB == 3) {
+                if (m <= 96) jacobi_replay<16, 3, 3>(jb, Cv, m, nrow, lda);
+                else jacobi_replay<8, 7, 2>(jb, Cv, m, nrow, lda);
+            } else if constexpr (NB == kMaxNB) {
+                jacobi_replay<16, 5, 5>(jb, Cv, m, nrow, lda);
+            } else {
+                jacobi_replay<16, 8, 2>(jb, Cv, m, nrow, lda);
+            }
         }
         if (sweep < maxsweep) {
             double mx = 0.0;
@@ -1042,7 +1058,8 @@ struct PotTables {
 // registers.  The AES energy is x . v_aes / 2 (the multipole energy is a
 // symmetric bilinear form of the moments).  scr: LDS, pot_lds(nat) doubles.
 // (26-atom C8H18+, 50 basis functions: 20-30 k cycles a call with one
-// multipole wavefront, ten kernel planes and the ndim^2 response matrix.)
+// multipole wavefront, ten kernel planes and the ndim^2 response matrix, 15 k
+// now, 18 k with the energies.)
 QX_DEV void potentials(const SysInfo& si, BatchRef B, SysShared& ss, const PotTables& pt, const double* x, double* vs,
                        double* vd, double* vq, double* scr, bool energy)
 {
