@@ -96,7 +96,7 @@ typedef double qx_d4 __attribute__((ext_vector_type(4)));
 // for memory once.  Up to 56 columns a product is bound by that wait and the
 // tail, above by the L1 traffic of the operands (16 lines per load of A).
 // (A product of the eigenvector refinement with every strip formed -> now, in
-// cycles: 88 columns 12.9 k -> 12.2 k, 98: 38 k -> 34 k, 132: 129 k -> 114 k,
+// cycles: 58 columns 12.9 k -> 12.2 k, 88: 38 k -> 34 k, 132: 129 k -> 114 k,
 // where the matrix cores need 43 k for all and half of it for the symmetric.)
 QX_DEV void mfma_gemm(int M, int N, int K, const double* A, int ai, int ak, const double* Bm, int bk,
                       int bj, double* Cm, int ldc, const double* d, bool sym)
@@ -542,7 +542,7 @@ QX_DEV void jacobi_rounds_global(const JacobiBuffers& jb, int m, double tol, dou
 // round is bound by the instructions issued.
 // (Cycles a round with one row per wavefront and slots 64 apart -> now: 132
 // rows and columns 6.0 k -> 2.9 k, where the second set had used 2 lanes of 64;
-// 98: 1.75 k -> 1.50 k.)
+// 88: 1.75 k -> 1.50 k.)
 template <int NL, int NS, int NR>
 QX_DEV void jacobi_replay(const JacobiBuffers& jb, double* Cv, int m, int nrow, int lda)
 {
@@ -1623,8 +1623,8 @@ QX_DEV void scc_body(int sys, const SysInfo& si, BatchRef B0, OptRef opt, SysSha
             // up to three that share the loads of P, over one half of the rows.
             // Every matrix is read once per iteration, which bounds large
             // systems; so P is read by four wavefronts and not by all eight.
-            // (Cycles with a matrix or two per wavefront over all rows -> now: 88
-            // AOs 52 k -> 30 k, 98: 105 k -> 62 k, 132: 184 k -> 114 k.)
+            // (Cycles with a matrix or two per wavefront over all rows -> now: 58
+            // AOs 52 k -> 30 k, 88: 105 k -> 62 k, 132: 184 k -> 114 k.)
             const bool split = n >= kRs;  // A holds n x kRs
             {
                 static_assert(kNT / 64 == 8 && kRs <= 12, "three matrices by half the rows per wavefront");
