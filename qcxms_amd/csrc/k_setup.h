@@ -160,9 +160,8 @@ QX_DEV void setup_shell_row(const ShellDesc& sa, const ShellDesc& sb, const Elem
 // a row, and there is one barrier per column.  Both triangles are packed by
 // rows; a: n (n + 2) doubles.
 // (26-atom C8H18+, 50 basis functions: 82 us as a right-looking Cholesky of two
-// barriers per column followed by one thread per column of the inverse; 132
-// basis functions in global memory: 1.5 ms.  The whole setup of a C8H18+ step
-// takes 372 k cycles instead of 490 k with it.)
+// barriers per column followed by one thread per column of the inverse.  The
+// whole setup of a C8H18+ step takes 372 k cycles instead of 490 k with it.)
 QX_DEV void factor_lds(const double* S, double* Lg, double* Xg, int n, int ld, double* a)
 {
     constexpr int NR = QX_BLOCK / 32;
@@ -200,51 +199,58 @@ QX_DEV void factor_lds(const double* S, double* Lg, double* Xg, int n, int ld, d
         }
 }
 
-// The same in global memory, for systems whose triangles do not fit in LDS.
-QX_DEV void factor_global(const double* S, double* A, double* Xg, int n, int ld)
+// The same in global memory, for systems whose triangles do not fit in LDS:
+// every element goes through the same operations in the same order, so L and X
+// do not depend on where the triangles are.  They are kept by columns here
+// (element (i, q) at q * ld + i), a lane per row and the columns dealt to the
+// wavefronts, so that all accesses are contiguous or uniform; the loads of NC
+// columns are under way together, since a step is bound by their latency.
+// a, e: ld x ld scratch each; rd: n doubles of LDS.
+// (The whole setup of a 36-atom ring of 144 basis functions: 1.66 ms with a
+// right-looking Cholesky and one thread per column of the inverse, 1.35 ms now.)
+QX_DEV void factor_global(const double* S, double* Lg, double* Xg, int n, int ld, double* a, double* e, double* rd)
 {
-    const int tid = qx_tid();
-    const size_t ms = (size_t)ld * ld;
+    constexpr int NW = QX_BLOCK / 64, NC = 4;
+    const int tid = qx_tid(), lane = tid & 63, wave = qx_wave(tid);
     __syncthreads();
-    for (size_t i = tid; i < ms; i += QX_BLOCK) A[i] = S[i];
+    for (int q = wave; q < n; q += NW)
+        for (int i = q + lane; i < n; i += 64) {
+            a[q * ld + i] = S[i * ld + q];
+            e[q * ld + i] = q == i ? 1.0 : 0.0;
+        }
     __syncthreads();
-    for (int j = 0; j < n; ++j) {
-        // every thread takes the pivot's root itself; thread 0 stores it
-        // while the others update the trailing block (two barriers a column)
-        const double d = sqrt(A[(size_t)j * ld + j]);
-        for (int i = j + 1 + tid; i < n; i += QX_BLOCK) A[(size_t)i * ld + j] /= d;
-        __syncthreads();
-        if (tid == 0) A[(size_t)j * ld + j] = d;
-        // trailing lower triangle: row j + 1 + r by lane r, its columns
-        // j + 1 + c (c <= r) by the wavefronts in turn
-        const int m = n - j - 1;
-        for (int r = tid & 63; r < m; r += 64) {
-            const int i = j + 1 + r;
-            const double lij = A[(size_t)i * ld + j];
-            for (int c = tid >> 6; c <= r; c += QX_BLOCK / 64) {
-                const int k = j + 1 + c;
-                A[(size_t)i * ld + k] -= lij * A[(size_t)k * ld + j];
+    for (int j = 0; j < n - 1; ++j) {
+        const double inv = 1.0 / a[j * ld + j];
+        for (int i0 = j + 1; i0 < n; i0 += 64) {
+            const int i = i0 + lane, ir = i < n ? i : n - 1;
+            const double l = a[j * ld + ir] * inv;
+            // columns 0 .. j of the inverse, j + 1 .. of S down to the diagonal
+            const int qe = i0 + 64 < n ? i0 + 64 : n;
+            for (int q = wave; q < qe; q += NC * NW) {
+                double v[NC], x[NC];
+#pragma unroll
+                for (int u = 0; u < NC; ++u) {
+                    const int c = q + u * NW < qe ? q + u * NW : q;
+                    v[u] = (c <= j ? e : a)[c * ld + ir];
+                    x[u] = c <= j ? e[c * ld + j] : a[j * ld + c];
+                }
+                qx_sched_fence();
+#pragma unroll
+                for (int u = 0; u < NC; ++u) {
+                    const int c = q + u * NW;
+                    if (c < qe && i < n && (c <= j || c <= i)) (c <= j ? e : a)[c * ld + i] = v[u] - l * x[u];
+                }
             }
         }
         __syncthreads();
     }
-    for (size_t p = tid; p < ms; p += QX_BLOCK) {
-        const int i = (int)(p / ld), k = (int)(p % ld);
-        if (!(k <= i && i < n)) A[p] = 0.0;
-        Xg[p] = 0.0;
-    }
+    for (int j = tid; j < n; j += QX_BLOCK) rd[j] = 1.0 / sqrt(a[j * ld + j]);
     __syncthreads();
-    // X = (L^-1)^T: column c of L^-1 by forward substitution (thread c),
-    // written as row c of X
-    for (int c = tid; c < n; c += QX_BLOCK) {
-        double* xr = Xg + (size_t)c * ld;  // X[c][i] = Linv[i][c]
-        for (int i = c; i < n; ++i) {
-            double v = (i == c) ? 1.0 : 0.0;
-#pragma unroll 8
-            for (int k = c; k < i; ++k) v -= A[(size_t)i * ld + k] * xr[k];
-            xr[i] = v / A[(size_t)i * ld + i];
+    for (int i = wave; i < ld; i += NW)
+        for (int q = lane; q < ld; q += 64) {
+            Lg[i * ld + q] = (i < n && q <= i) ? a[q * ld + i] * rd[q] : 0.0;
+            Xg[i * ld + q] = (q < n && i <= q) ? e[i * ld + q] * rd[q] : 0.0;
         }
-    }
 }
 
 // ---------------------------------------------------------------------------
@@ -540,9 +546,10 @@ QX_DEV void setup_system(BatchRef B, int sys, int with_chol, SetupLds& Ls, doubl
         B.eparts[10 * sys + 7] = erep;
     }
     if (!with_chol) return;
-    // 9. Cholesky S = L L^T and X = L^-T
+    // 9. Cholesky S = L L^T and X = L^-T (the SCC's scratch is free)
+    static_assert(QX_MAX_REF * QX_MAX_NAT >= QX_MAX_NAO, "the pivots take the place of zg");
     if (n * (n + 2) <= ndyn) factor_lds(S, B.L + si.mat_off, B.X + si.mat_off, n, ld, dyn);
-    else factor_global(S, B.L + si.mat_off, B.X + si.mat_off, n, ld);
+    else factor_global(S, B.L + si.mat_off, B.X + si.mat_off, n, ld, B.T + si.mat_off, B.C + si.mat_off, zg);
 }
 
 __global__ __launch_bounds__(QX_BLOCK) void k_setup(BatchPtrs B, int with_chol, int ndyn)

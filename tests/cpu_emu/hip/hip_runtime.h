@@ -250,6 +250,11 @@ inline d4 mfma_f64_16x16x4(double a, double b, d4 c, int, int, int)
 
 inline void* dyn_lds() { return g_dyn; }
 
+// Called before a launch with the kernel, its shape and pointers to its
+// arguments, when set: false leaves the launch out.
+inline bool (*g_launch_hook)(const void* kernel, unsigned grid, unsigned block, size_t shmem,
+                             const void* const* args) = nullptr;
+
 extern "C" char __start_qx_emu_lds[], __stop_qx_emu_lds[];
 inline void poison_static_lds() { std::memset(__start_qx_emu_lds, 0xff, __stop_qx_emu_lds - __start_qx_emu_lds); }
 
@@ -264,6 +269,10 @@ void launch(void (*k)(P...), dim3 grid, dim3 block, size_t shmem, A... args)
     if (shmem > kMaxLds) {
         std::fprintf(stderr, "cpu emulation: %zu bytes of dynamic LDS exceed 160 KiB\n", shmem);
         std::abort();
+    }
+    if (g_launch_hook) {
+        const void* ptrs[] = {(const void*)&args..., nullptr};
+        if (!g_launch_hook((const void*)k, grid.x, block.x, shmem, ptrs)) return;
     }
     gridDim = grid;
     blockDim = block;
