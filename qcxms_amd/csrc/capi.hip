@@ -239,9 +239,11 @@ int ensure_init(int device)
     const size_t base_dyn = (4 * qx::kFastM * (qx::kFastM + 1) + qx::kRs * qx::kFastM) * sizeof(double);
     if ((size_t)lds_block < lds_static + base_dyn) return fail("the device's LDS per workgroup is too small");
     g_scc_dyn_max = (size_t)lds_block - lds_static;
-    // the optional fifth matrix (MFMA eigen refinement) only where the
-    // workgroup keeps 8 KiB of its LDS free: workgroups of up to 153 KB are
-    // what the MI355X runs have exercised (m <= 50)
+    // the optional fifth matrix (MFMA eigen refinement) and the triangles of
+    // the setup only where the workgroup keeps 8 KiB of its LDS free:
+    // workgroups of up to 153 KB are what the MI355X runs have exercised
+    // (fifth matrix up to 50 basis functions; triangles up to 133 in k_setup
+    // and 117 in the persistent kernel, whose static LDS is larger)
     constexpr size_t kLdsReserve = 8192;
     g_eig_dyn_max = g_scc_dyn_max > kLdsReserve ? g_scc_dyn_max - kLdsReserve : 0;
     HIPCHK(hipFuncSetAttribute((const void*)qx::k_scc<false>, hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -807,13 +809,13 @@ int enqueue_md_step(qcxms_md* md)
     int st;
     if ((st = timed(b, b->t_md_pre, [&] {
              hipLaunchKernelGGL(qx::k_md_pre, dim3(md->ntraj), dim3(64), 0, b->stream,
-                                qx::MdArgs{b->d, md->m, md->p, b->opts, 1});
+                                qx::MdArgs{b->d, md->m, md->p, b->opts, 1, 0});
          })))
         return st;
     if ((st = enqueue_egrad(b, true))) return st;
     return timed(b, b->t_md_post, [&] {
         hipLaunchKernelGGL(qx::k_md_post, dim3(md->ntraj), dim3(QX_BLOCK), 0, b->stream,
-                           qx::MdArgs{b->d, md->m, md->p, b->opts, 1});
+                           qx::MdArgs{b->d, md->m, md->p, b->opts, 1, 0});
     });
 }
 
@@ -1623,11 +1625,12 @@ int md_enqueue(qcxms_md* md)
 int md_enqueue_fused(qcxms_md* md, int nsteps)
 {
     qcxms_batch* b = md->b;
-    const size_t lds = std::max(lds_setup_bytes(b, g_scc_dyn_max), lds_scc_bytes(b));
+    // the setup's triangles with the same reserve as the fifth matrix
+    const size_t l1 = lds_setup_bytes(b, g_eig_dyn_max), l2 = lds_scc_bytes(b);
     return timed(b, b->t_fused, [&] {
         hipLaunchKernelGGL(b->opts.eig_mfma ? qx::k_md_fused<true> : qx::k_md_fused<false>, dim3(md->ntraj),
-                           dim3(QX_SCC_BLOCK), lds, b->stream,
-                           qx::MdArgs{b->d, md->m, md->p, launch_opts(b, lds), nsteps});
+                           dim3(QX_SCC_BLOCK), std::max(l1, l2), b->stream,
+                           qx::MdArgs{b->d, md->m, md->p, launch_opts(b, l2), nsteps, (int)(l1 / sizeof(double))});
     });
 }
 

@@ -687,13 +687,15 @@ QX_DEV void md_post_system(BatchRef B, MdRef M, MdParamRef p, int sys, MdLds& Lm
     }
 }
 
-// Arguments of the MD step kernels (opt, nsteps: the persistent one)
+// Arguments of the MD step kernels (opt, nsteps, setup_doubles: the persistent
+// one; setup_doubles: dynamic LDS of its setup, opt.lds_doubles that of its SCC,
+// which a launch of k_scc would have too)
 struct MdArgs {
     BatchPtrs B;
     MdPtrs M;
     MdParams p;
     SccOpts opt;
-    int nsteps;
+    int nsteps, setup_doubles;
 };
 
 __global__ __launch_bounds__(64) void k_md_pre(MdArgs args)
@@ -761,7 +763,7 @@ __global__ __launch_bounds__(QX_SCC_BLOCK) void k_md_fused(MdArgs args)
         if (!qx_uniform(fresh().M.active[sys])) break;
         {
             QX_ARG(MdArgs) a = fresh();
-            setup_system(a.B, sys, 1, L.s, dyn, a.opt.lds_doubles);
+            setup_system(a.B, sys, 1, L.s, dyn, a.setup_doubles);
         }
         __syncthreads();
         QX_FUSED_PH(25);

@@ -45,3 +45,29 @@ def test_factorisation_does_not_depend_on_where_the_triangles_are(nao):
         for a in (l, x):
             assert np.all(a[n:] == 0.0) and np.all(a[:, n:] == 0.0)
     assert m[0].tobytes() == m[1].tobytes()
+
+
+def launch(naos):
+    mols = [molecule(n)[0] for n in naos]
+    off = np.cumsum([0] + [len(m) for m in mols]).astype(np.int32)
+    raw = eb.part("launch", np.array([len(mols)], np.int32), off, np.concatenate(mols).astype(np.int32))
+    return np.frombuffer(raw, np.int64)
+
+
+@pytest.mark.timeout(900)
+def test_persistent_launch_keeps_its_lds_reserve():
+    """Whatever the basis size, the persistent MD kernel's workgroup leaves
+    8 KiB of the LDS free, as the SCC and setup kernels do."""
+    for nao in (2 + 6 * 8, 56, 58, 111, 113, 115, 116, 117, 118, 119, 120, 121, 122, 132, 134):
+        shmem, _, _, _, free = launch([nao])
+        assert shmem <= free, nao
+
+
+@pytest.mark.timeout(900)
+@pytest.mark.parametrize("naos", [(50, 56), (52,), (52, 117), (52, 119), (54, 121), (58, 134)])
+def test_scc_of_a_persistent_launch_has_the_lds_of_the_scc_kernel(naos):
+    """The LDS that the SCC may use (which decides about the fifth matrix of
+    the eigenvector refinement, so about the solver's path) is that of the
+    SCC kernel of a step, whatever the setup of another trajectory takes."""
+    shmem, doubles, step_shmem, step_doubles, _ = launch(naos)
+    assert doubles == step_doubles and 8 * doubles == step_shmem <= shmem
