@@ -1,5 +1,6 @@
 // Driver of the CPU-emulated build that runs single parts of the library: the
-// setup of one system, and the launch sizes of a trajectory ensemble.
+// setup of one system, the launch sizes of a trajectory ensemble, the
+// eigensolver and the solution for the Broyden weights.
 //   parts_emu setup in out
 //     in : int32 nat, num[nat]; double xyz[3 nat]
 //     out: int32 n, ld; then twice (triangles of the factorisation in LDS, in
@@ -9,6 +10,14 @@
 //     out: int64 shmem, lds_doubles of the persistent launch, of the SCC
 //          launch of a step, free: LDS bytes that a workgroup may take beside
 //          the static ones with the reserve kept
+//   parts_emu eig in out
+//     in : int32 m, nrow, form (0 blocks in global memory, 1 in LDS, 2 matrices
+//          of up to 56 columns in LDS), refine, maxsweep (0: eig_solve, else
+//          jacobi_any); double tol, min_s, A [m * m], C [nrow * m]
+//     out: int32 full sweeps; double A, C
+//   parts_emu broyden in out
+//     in : int32 n, st (0: in LDS); double B [n * n], g [n]
+//     out: double x [n]
 #include "_build/src/capi.hip"
 
 #include <cstdlib>
@@ -103,10 +112,79 @@ static void run_launch(FILE* in, FILE* out)
     wr(out, &lds, 1);
 }
 
+struct EigArgs {
+    int m, nrow, lda, lds, maxsweep;
+    double tol, min_s;
+    double *A, *C, *Y, *Z, *T;  // m x m each (C: nrow x m), leading dimension lda
+    int* done;
+};
+
+template <bool EIG, bool FAST>
+static void k_eig(EigArgs a)
+{
+    __shared__ __align__(16) double rot[2 * QX_MAX_NAO];
+    __shared__ int any[QX_MAX_NAO];
+    __shared__ double red[8 * (qx::kNT / 64)];
+    double* dyn = (double*)qx_emu::dyn_lds();
+    const qx::JacobiBuffers jb{FAST ? a.Y : dyn, {a.Y, a.T}, (double2*)a.Z, (double2*)rot, any, red, a.lds != 0};
+    const int n = a.maxsweep ? qx::jacobi_any<FAST>(a.A, a.C, a.m, a.nrow, a.lda, a.tol, a.maxsweep, a.min_s, jb)
+                             : qx::eig_solve<EIG, FAST>(a.A, a.C, a.m, a.nrow, a.lda, a.tol, a.Y, a.Z, a.T, jb);
+    if (threadIdx.x == 0) *a.done = n;
+}
+
+// the matrices' storage as the SCC has it: leading dimension m + 1 (LDS) or
+// the next multiple of 16 (global memory), the blocks exactly in the LDS
+static void run_eig(FILE* in, FILE* out)
+{
+    int32_t h[5];
+    rd(in, h, 5);
+    const int m = h[0], nrow = h[1], form = h[2], refine = h[3];
+    double t[2];
+    rd(in, t, 2);
+    const int lda = form == 2 ? m + 1 : (m + 15) & ~15, rows = form == 2 ? m : lda;
+    std::vector<double> mat[5];
+    for (auto& v : mat) v.assign((size_t)rows * lda, NAN);
+    for (int i = 0; i < m; ++i) rd(in, &mat[0][(size_t)i * lda], m);
+    for (int i = 0; i < nrow; ++i) rd(in, &mat[1][(size_t)i * lda], m);
+    int done = -1;
+    const EigArgs a{m, nrow, lda, form != 0, h[4], t[0], t[1], mat[0].data(), mat[1].data(), mat[2].data(),
+                    mat[3].data(), mat[4].data(), &done};
+    const size_t blk = form == 1 ? sizeof(double) * (size_t)m * (m + 2) / 2 : 0;
+    void (*k)(EigArgs) = form == 2 ? (refine ? k_eig<true, true> : k_eig<false, true>)
+                                   : (refine ? k_eig<true, false> : k_eig<false, false>);
+    hipLaunchKernelGGL(k, dim3(1), dim3(qx::kNT), blk, nullptr, a);
+    const int32_t d = done;
+    wr(out, &d, 1);
+    for (int i = 0; i < m; ++i) wr(out, &mat[0][(size_t)i * lda], m);
+    for (int i = 0; i < nrow; ++i) wr(out, &mat[1][(size_t)i * lda], m);
+}
+
+static void k_broyden(int n, int st, const double* B, const double* g, double* bt, double* x)
+{
+    __shared__ double gm[128];
+    double* t = bt ? bt : (double*)qx_emu::dyn_lds();
+    for (int p = threadIdx.x; p < (n + 1) * n; p += qx::kNT) t[p / n * st + p % n] = p / n == n ? g[p % n] : B[p];
+    __syncthreads();
+    qx::broyden_solve(t, st, gm, n);
+    for (int i = threadIdx.x; i < n; i += qx::kNT) x[i] = gm[i];
+}
+
+static void run_broyden(FILE* in, FILE* out)
+{
+    int32_t h[2];
+    rd(in, h, 2);
+    const int n = h[0], st = h[1] ? h[1] : (n | 1);
+    const auto B = rdv<double>(in, (size_t)n * n), g = rdv<double>(in, n);
+    std::vector<double> bt((size_t)(n + 1) * st, NAN), x(n);
+    hipLaunchKernelGGL(k_broyden, dim3(1), dim3(qx::kNT), h[1] ? 0 : sizeof(double) * bt.size(), nullptr, n, st,
+                       B.data(), g.data(), h[1] ? bt.data() : nullptr, x.data());
+    wr(out, x.data(), n);
+}
+
 int main(int argc, char** argv)
 {
     if (argc != 4) {
-        std::fprintf(stderr, "usage: %s setup|launch input output\n", argv[0]);
+        std::fprintf(stderr, "usage: %s setup|launch|eig|broyden input output\n", argv[0]);
         return 2;
     }
     FILE* in = std::fopen(argv[2], "rb");
@@ -115,6 +193,8 @@ int main(int argc, char** argv)
     const std::string part = argv[1];
     if (part == "setup") run_setup(in, out);
     else if (part == "launch") run_launch(in, out);
+    else if (part == "eig") run_eig(in, out);
+    else if (part == "broyden") run_broyden(in, out);
     else return 2;
     std::fclose(in);
     return std::fclose(out) ? 2 : 0;

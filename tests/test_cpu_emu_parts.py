@@ -71,3 +71,95 @@ def test_scc_of_a_persistent_launch_has_the_lds_of_the_scc_kernel(naos):
     SCC kernel of a step, whatever the setup of another trajectory takes."""
     shmem, doubles, step_shmem, step_doubles, _ = launch(naos)
     assert doubles == step_doubles and 8 * doubles == step_shmem <= shmem
+
+
+def eig(a, form, refine=0, maxsweep=0, tol=1e-11, min_s=0.0):
+    """The eigensolver on the n x n matrix a, padded to an even order by a
+    zero row and column; C starts as the identity, so that it ends as V."""
+    n = len(a)
+    m = (n + 1) & ~1
+    am, c = np.zeros((m, m)), np.zeros((n, m))
+    am[:n, :n] = a
+    c[:, :n] = np.eye(n)
+    raw = eb.part("eig", np.array([m, n, form, refine, maxsweep], np.int32), np.array([tol, min_s]), am, c)
+    out = np.frombuffer(raw, np.float64, offset=4)
+    return int(np.frombuffer(raw, np.int32, 1)[0]), out[:m * m].reshape(m, m), out[m * m:].reshape(n, m)
+
+
+def check_rotated(a, out, v, sweeps):
+    """V orthogonal and A_out = V^T A V: every row takes m - 1 rotations a
+    sweep, each within 4 eps of the norm (2 here), over at most 15 sweeps and
+    256 columns 4e-12."""
+    n = len(a)
+    one = np.zeros(len(out))
+    one[:n] = 1.0
+    assert np.abs(v.T @ v - np.diag(one)).max() < 4e-12, sweeps
+    assert np.abs(v.T @ a @ v - out).max() < 4e-12, sweeps
+
+
+def dense(n):
+    r = np.random.default_rng(n).standard_normal((n, n))
+    return np.diag(np.linspace(-1.0, 1.0, n)) + 0.25 * (r + r.T) / np.sqrt(n)
+
+
+def offdiag(a):
+    return np.abs(a - np.diag(np.diag(a))).max()
+
+
+@pytest.mark.timeout(900)
+@pytest.mark.parametrize("n,form", [(2, 2), (3, 2), (21, 2), (21, 1), (66, 1), (66, 0)])
+def test_jacobi_to_convergence(n, form):
+    """Every form of the sweeps: rows of C in registers (up to 64 columns) or
+    rotated by the logged sweep, blocks in LDS or in global memory."""
+    a = dense(n)
+    sweeps, out, v = eig(a, form)
+    assert 0 < sweeps <= 15 and offdiag(out) < 1e-11
+    check_rotated(a, out, v, sweeps)
+    assert np.array_equal(out, out.T)
+
+
+@pytest.mark.timeout(900)
+@pytest.mark.parametrize("n,form,min_s", [(55, 2, 0.02), (56, 2, 0.0), (57, 1, 0.0), (64, 1, 0.02), (96, 1, 0.0),
+                                          (97, 1, 0.02), (102, 1, 0.0), (104, 1, 0.02), (132, 1, 0.0),
+                                          (134, 0, 0.02), (256, 0, 0.0)])
+def test_two_jacobi_sweeps_at_the_limits_of_their_forms(n, form, min_s):
+    """Two sweeps at the largest orders of the matrices in LDS, the rows in
+    registers, the splits of the rotation replay and the blocks in LDS, and
+    beyond; all rotations or (a coarse sweep) the large ones."""
+    a = dense(n)
+    sweeps, out, v = eig(a, form, maxsweep=2, min_s=min_s)
+    assert sweeps == 2 and np.array_equal(out, out.T)
+    # a sweep that rotates every pair does not increase the sum of squares
+    assert np.sum(np.tril(out, -1) ** 2) < 0.5 * np.sum(np.tril(a, -1) ** 2)
+    check_rotated(a, out, v, sweeps)
+
+
+@pytest.mark.timeout(900)
+@pytest.mark.parametrize("n,form,strong", [(50, 2, 3), (57, 1, 0), (66, 1, 3), (134, 0, 3)])
+def test_eigenvector_refinement(n, form, strong):
+    """The simultaneous rotations, from small couplings (no Jacobi sweep) and
+    with near-degenerate, strongly coupled pairs (coarse sweeps first); the
+    fifth matrix shares its storage with the blocks in global memory."""
+    r = np.random.default_rng(n + strong).standard_normal((n, n))
+    a = np.diag(np.linspace(-1.0, 1.0, n)) + 2e-5 * (r + r.T)
+    for k in range(strong):
+        i, j = 5 * k, 5 * k + 1
+        a[i, j] = a[j, i] = 0.05
+    sweeps, out, v = eig(a, form, refine=1)
+    assert sweeps == 0 and offdiag(out) < 1e-11
+    check_rotated(a, out, v, sweeps)
+
+
+@pytest.mark.timeout(900)
+@pytest.mark.parametrize("n,st", [(1, 0), (2, 0), (40, 0), (41, 100), (64, 0), (65, 100), (100, 100)])
+def test_broyden_weights(n, st):
+    """The solution for the weights of n secant pairs, the matrix in LDS or in
+    global memory, against numpy: n eps times the condition (< 1e3) times 10."""
+    rng = np.random.default_rng(n)
+    g = rng.standard_normal((n, 3 * n))
+    b = np.eye(n) + g @ g.T / (3 * n)
+    assert np.linalg.cond(b) < 1e3
+    rhs = rng.standard_normal(n)
+    x = np.frombuffer(eb.part("broyden", np.array([n, st], np.int32), b, rhs), np.float64)
+    ref = np.linalg.solve(b, rhs)
+    assert np.abs(x - ref).max() < 1.2e-13 * n * np.abs(ref).max() * 10
