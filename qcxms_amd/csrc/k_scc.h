@@ -317,7 +317,14 @@ QX_DEV double2 pivot_rotation(double app, double aqq, double apq, double tol, do
     return make_double2(turn ? cs.x : 1.0, turn ? cs.y : 0.0);
 }
 
-constexpr int kMaxNB = 5;  // blocks per thread the rounds take (132 basis functions)
+// Blocks per thread that the rounds with the blocks in LDS take (up to 132
+// basis functions); above, the rounds work on global memory.  The LDS would
+// hold the blocks of 172 functions, but a thread keeps its blocks in registers
+// between the barriers.  (Six blocks: 136 functions 60.9 -> 36.1 ms and 144:
+// 75.3 -> 39.5 ms, single rings of carbon, but 132: 33.3 -> 33.7 ms; as a
+// further instantiation 104 to 132 functions take 0.5 % longer and the kernel
+// spills 112 instead of 57 vector registers.)
+constexpr int kMaxNB = 5;
 
 // Working storage of the Jacobi sweeps
 struct JacobiBuffers {
