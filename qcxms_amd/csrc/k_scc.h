@@ -29,23 +29,24 @@ constexpr int kFastM = 56;
 constexpr int kRs = 11;  // row sums per AO: S, D (3), Q (6), H0
 
 // Opt-in per-phase cycle counters of the SCC kernel (build with
-// -DQX_PHASE_TIMING); compiled out otherwise.
+// -DQX_PHASE_TIMING); compiled out otherwise.  Rows are systems of the batch,
+// whatever workgroup runs them.
 #ifdef QX_PHASE_TIMING
 constexpr int kPhaseSys = 1024, kPhaseSlots = 32;
 __device__ unsigned long long g_phase[kPhaseSys * kPhaseSlots];
 #define QX_PH_INIT unsigned long long ph_t = clock64();
-#define QX_PH(k)                                                                   \
+#define QX_PH(sys, k)                                                              \
     do {                                                                           \
         __syncthreads();                                                           \
-        if (threadIdx.x == 0 && blockIdx.x < kPhaseSys) {                          \
+        if (threadIdx.x == 0 && (sys) < kPhaseSys) {                               \
             const unsigned long long t_ = clock64();                               \
-            g_phase[blockIdx.x * kPhaseSlots + (k)] += t_ - ph_t;                  \
+            g_phase[(sys) * kPhaseSlots + (k)] += t_ - ph_t;                       \
             ph_t = t_;                                                             \
         }                                                                          \
     } while (0)
-#define QX_PH_ADD(k, v)                                                            \
+#define QX_PH_ADD(sys, k, v)                                                       \
     do {                                                                           \
-        if (threadIdx.x == 0 && blockIdx.x < kPhaseSys) g_phase[blockIdx.x * kPhaseSlots + (k)] += (v); \
+        if (threadIdx.x == 0 && (sys) < kPhaseSys) g_phase[(sys) * kPhaseSlots + (k)] += (v); \
     } while (0)
 #define QX_PT_INIT(tv) unsigned long long tv = clock64(), tv##_acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
 #define QX_PT(k, tv)                                                               \
@@ -72,11 +73,11 @@ __device__ unsigned long long g_phase[kPhaseSys * kPhaseSlots];
     do {                   \
     } while (0)
 #define QX_PH_INIT
-#define QX_PH(k) \
-    do {         \
+#define QX_PH(sys, k) \
+    do {              \
     } while (0)
-#define QX_PH_ADD(k, v) \
-    do {                \
+#define QX_PH_ADD(sys, k, v) \
+    do {                     \
     } while (0)
 #endif
 
@@ -335,6 +336,7 @@ struct JacobiBuffers {
     int* any;         // per round of a sweep: whether it rotates anything (LDS, m entries)
     double* red;
     bool lds;         // the blocks fit in LDS
+    int sys;          // system (phase counters)
 };
 
 // The pivot of a lane in the next round: its two slots and their blocks
@@ -894,7 +896,7 @@ QX_DEV int eig_solve(double* A, double* Cv, int m, int nrow, int lda, double tol
         }
         const int done = jacobi_any<FAST>(A, Cv, m, nrow, lda, tol, sweeps, min_s, jb);
         if (sweeps != 1) return done;
-        QX_PH_ADD(29, 1);
+        QX_PH_ADD(jb.sys, 29, 1);
     }
 }
 
@@ -1514,7 +1516,7 @@ QX_DEV void scc_body(int sys, const SysInfo& si, BatchRef B0, OptRef opt, SysSha
         if (tid == 0) L.s_e[1] = -1e300;
     }
     __syncthreads();
-    QX_PH(11);
+    QX_PH(sys, 11);
 
     PotTables pt;
     pt.load(si, qx_fresh(B0), ss);
@@ -1532,7 +1534,7 @@ QX_DEV void scc_body(int sys, const SysInfo& si, BatchRef B0, OptRef opt, SysSha
     for (bool out = false;; out = !out) {
         potentials(si, qx_fresh(B0), ss, pt, out ? xout : xin, vs, vd, vq, bf.pot, out);
         if (!out) {
-            QX_PH(0);
+            QX_PH(sys, 0);
             {
                 // G^T (row nu holds G_{mu nu} over mu), then F = H0 - (G + G^T) / 2
                 BatchRef B = qx_fresh(B0);
@@ -1581,7 +1583,7 @@ QX_DEV void scc_body(int sys, const SysInfo& si, BatchRef B0, OptRef opt, SysSha
                 }
                 __syncthreads();
             }
-            QX_PH(1);
+            QX_PH(sys, 1);
             // A = C^T F C (F C staged in the density buffer)
             for (int s = 0; s < 2; ++s) {
                 mfma_gemm(n, n, n, s ? Cc : Ft, s ? 1 : lb, s ? lb : 1, s ? P : Cc, lb, 1, s ? A : P, lb, nullptr,
@@ -1593,16 +1595,16 @@ QX_DEV void scc_body(int sys, const SysInfo& si, BatchRef B0, OptRef opt, SysSha
                     }
                 __syncthreads();
             }
-            QX_PH(2);
+            QX_PH(sys, 2);
             double jtol = fmin(1e-6, 1e-3 * errp);
             if (jtol < opt.jacobi_tol) jtol = opt.jacobi_tol;
             const int nblk = (m / 2) * (m / 2 + 1) / 2;
             const bool blk_lds = FAST || (4 * nblk <= bf.nlds && nblk <= kMaxNB * (kNT - 64));
-            const JacobiBuffers jb{FAST ? Ft : bf.lds, {Ft, bf.E}, (double2*)P, (double2*)ss.rot, ss.any, ss.red, blk_lds};
+            const JacobiBuffers jb{FAST ? Ft : bf.lds, {Ft, bf.E}, (double2*)P, (double2*)ss.rot, ss.any, ss.red, blk_lds, sys};
             const int nsweep = eig_solve<EIG, FAST>(A, Cc, m, n, lb, jtol, Ft, P, bf.E, jb);
-            QX_PH(3);
-            QX_PH_ADD(12, nsweep);
-            QX_PH_ADD(15, nsweep == 0);
+            QX_PH(sys, 3);
+            QX_PH_ADD(sys, 12, nsweep);
+            QX_PH_ADD(sys, 15, nsweep == 0);
             (void)nsweep;
             const int tid = qx_tid();
             for (int i = tid; i < n; i += kNT) eps[i] = A[i * lb + i];
@@ -1615,16 +1617,16 @@ QX_DEV void scc_body(int sys, const SysInfo& si, BatchRef B0, OptRef opt, SysSha
                     L.s_e[0] = t;
                     L.s_e[1] = mu;
                 }
-                QX_PH_ADD(14, fit);
+                QX_PH_ADD(sys, 14, fit);
                 (void)fit;
                 for (int i = tid; i < n; i += 64) f2[i] = 2.0 * L.focc[i];
             }
             __syncthreads();
             ts = L.s_e[0];
-            QX_PH(4);
+            QX_PH(sys, 4);
             mfma_gemm(n, n, n, Cc, lb, 1, Cc, 1, lb, P, lb, f2, true);
             __syncthreads();
-            QX_PH(5);
+            QX_PH(sys, 5);
             // row sums of P o M for M = S, D (3), Q (6), H0 as coalesced column
             // sweeps over all AOs (lanes): a wavefront takes every fourth matrix,
             // up to three that share the loads of P, over one half of the rows.
@@ -1695,10 +1697,10 @@ QX_DEV void scc_body(int sys, const SysInfo& si, BatchRef B0, OptRef opt, SysSha
                 else xout[nsh + 3 * nat + 6 * a + (c - 3)] = -v;
             }
             __syncthreads();
-            QX_PH(6);
+            QX_PH(sys, 6);
             continue;
         }
-        QX_PH(7);
+        QX_PH(sys, 7);
         double red2[2] = {0.0, 0.0};
         for (int mu = qx_tid(); mu < n; mu += kNT) red2[0] += rs[mu * kRs + 10];
         for (int i = qx_tid(); i < nx; i += kNT) {
@@ -1717,12 +1719,12 @@ QX_DEV void scc_body(int sys, const SysInfo& si, BatchRef B0, OptRef opt, SysSha
             break;
         }
         if (it == opt.maxiter) break;
-        QX_PH(8);
+        QX_PH(sys, 8);
         broyden_step(si, qx_fresh(B0).hist + si.hist_off, opt, bf, xin, xout, ss.gm, ss.red, it, hcount);
-        QX_PH(9);
+        QX_PH(sys, 9);
         ++it;
     }
-    QX_PH_ADD(13, it);
+    QX_PH_ADD(sys, 13, it);
     BatchRef B = qx_fresh(B0);
     const int tid = qx_tid();
     if (opt.keep > 0 && tid == 0) {
@@ -1752,7 +1754,7 @@ QX_DEV void scc_body(int sys, const SysInfo& si, BatchRef B0, OptRef opt, SysSha
     // W = C diag(2 f e) C^T ; U = L^T C for the next warm start
     mfma_gemm(n, n, n, Cc, lb, 1, Cc, 1, lb, B.W + si.mat_off, ld, f2, true);
     mfma_gemm(n, n, n, B.L + si.mat_off, 1, ld, Cc, lb, 1, B.U + si.mat_off, ld, nullptr, false);
-    QX_PH(10);
+    QX_PH(sys, 10);
     if (tid == 0) {
         double* ep = B.eparts + 10 * sys;
         ep[0] = eband;

@@ -319,6 +319,7 @@ inline void run_or_record(std::function<void()> f)
 #define __shfl_xor(v, m, w) qx_emu::shfl_xor((v), (m), (w))
 #define __shfl(v, l, w) qx_emu::shfl((v), (l), (w))
 #define __builtin_amdgcn_mfma_f64_16x16x4f64 qx_emu::mfma_f64_16x16x4
+#define clock64() ((unsigned long long)std::chrono::steady_clock::now().time_since_epoch().count())
 #define __ffsll(x) __builtin_ffsll(x)
 #define __builtin_amdgcn_readlane(v, l) qx_emu::readlane((v), (l))
 #define __double_as_longlong(d) qx_emu::double_as_longlong(d)
@@ -336,6 +337,7 @@ inline hipError_t hipGetDeviceCount(int* n)
     return hipSuccess;
 }
 inline hipError_t hipSetDevice(int) { return hipSuccess; }
+inline hipError_t hipDeviceSynchronize() { return hipSuccess; }
 inline hipError_t hipGetLastError() { return hipSuccess; }
 inline const char* hipGetErrorString(hipError_t) { return "error in the CPU emulation"; }
 inline hipError_t hipFuncSetAttribute(const void*, hipFuncAttribute, int v)

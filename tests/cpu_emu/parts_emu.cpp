@@ -18,6 +18,10 @@
 //   parts_emu broyden in out
 //     in : int32 n, st (0: in LDS); double B [n * n], g [n]
 //     out: double x [n]
+//   phase_emu phase in out
+//     in : int32 nsys, max_nao of the first of two launches; offsets[nsys + 1],
+//          num[natoms]; double xyz[3 natoms]
+//     out: per system int32 SCC iterations, the phase counters' iterations
 #include "_build/src/capi.hip"
 
 #include <cstdlib>
@@ -181,10 +185,37 @@ static void run_broyden(FILE* in, FILE* out)
     wr(out, x.data(), n);
 }
 
+#ifdef QX_PHASE_TIMING
+static void run_phase(FILE* in, FILE* out)
+{
+    int32_t h[2];
+    rd(in, h, 2);
+    const int nsys = h[0];
+    const auto off = rdv<int32_t>(in, nsys + 1), num = rdv<int32_t>(in, off[nsys]);
+    const auto xyz = rdv<double>(in, 3 * (size_t)off[nsys]);
+    const std::vector<int32_t> charge(nsys, 0);
+    const std::vector<double> et(nsys, 300.0);
+    const int32_t bins[2] = {h[1], 256}, eig[2] = {0, 0}, lds[2] = {1, 1};
+    std::vector<double> e(nsys), g(3 * (size_t)off[nsys]), q(off[nsys]);
+    std::vector<int32_t> st(nsys);
+    if (qcxms_set_tuning(h[1] < 256 ? 2 : 1, bins, eig, lds, -1, 0) != QCXMS_OK) std::exit(3);
+    qcxms_batch* b = qcxms_batch_create(nsys, off.data(), num.data(), charge.data(), QCXMS_GFN2_XTB);
+    if (!b || qcxms_batch_egrad(b, xyz.data(), et.data(), e.data(), g.data(), q.data(), st.data()) != QCXMS_OK)
+        std::exit(3);
+    std::vector<unsigned long long> row((size_t)nsys * qx::kPhaseSlots);
+    std::memcpy(row.data(), qx::g_phase, sizeof(row[0]) * row.size());
+    for (int s = 0; s < nsys; ++s) {
+        const int32_t n[2] = {b->d.iters[s], (int32_t)row[(size_t)s * qx::kPhaseSlots + 13]};
+        wr(out, n, 2);
+    }
+    qcxms_batch_destroy(b);
+}
+#endif
+
 int main(int argc, char** argv)
 {
     if (argc != 4) {
-        std::fprintf(stderr, "usage: %s setup|launch|eig|broyden input output\n", argv[0]);
+        std::fprintf(stderr, "usage: %s setup|launch|eig|broyden|phase input output\n", argv[0]);
         return 2;
     }
     FILE* in = std::fopen(argv[2], "rb");
@@ -195,6 +226,9 @@ int main(int argc, char** argv)
     else if (part == "launch") run_launch(in, out);
     else if (part == "eig") run_eig(in, out);
     else if (part == "broyden") run_broyden(in, out);
+#ifdef QX_PHASE_TIMING
+    else if (part == "phase") run_phase(in, out);
+#endif
     else return 2;
     std::fclose(in);
     return std::fclose(out) ? 2 : 0;

@@ -105,19 +105,21 @@ def md_run(trajs, nsteps, fused, use_graph=1, timeout=1800, env=None):
 
 
 EMU_PARTS = os.path.join(EMU_DIR, "_build", "parts_emu")
+EMU_PHASE = os.path.join(EMU_DIR, "_build", "phase_emu")
 
 
 def part(name, *arrays, timeout=800):
     """One part of the library in the emulation (parts_emu.cpp): the arrays
     are its input file; returns the bytes of its output file."""
-    subprocess.run(["make", "-s", "-C", EMU_DIR, "parts"], check=True)
+    target = "phase" if name == "phase" else "parts"
+    subprocess.run(["make", "-s", "-C", EMU_DIR, target], check=True)
     with tempfile.TemporaryDirectory() as d:
         fin, fout = os.path.join(d, "in.bin"), os.path.join(d, "out.bin")
         with open(fin, "wb") as f:
             for a in arrays:
                 np.ascontiguousarray(a).tofile(f)
         env = dict(os.environ, ASAN_OPTIONS="detect_leaks=0:abort_on_error=1")
-        p = subprocess.run([EMU_PARTS, name, fin, fout], capture_output=True, text=True, timeout=timeout, env=env)
+        p = subprocess.run([EMU_PHASE if target == "phase" else EMU_PARTS, name, fin, fout], capture_output=True, text=True, timeout=timeout, env=env)
         if p.returncode != 0:
             raise RuntimeError(f"emulated part failed ({p.returncode}):\n{p.stderr[-6000:]}")
         with open(fout, "rb") as f:

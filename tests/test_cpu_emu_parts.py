@@ -163,3 +163,18 @@ def test_broyden_weights(n, st):
     x = np.frombuffer(eb.part("broyden", np.array([n, st], np.int32), b, rhs), np.float64)
     ref = np.linalg.solve(b, rhs)
     assert np.abs(x - ref).max() < 1.2e-13 * n * np.abs(ref).max() * 10
+
+
+@pytest.mark.timeout(900)
+@pytest.mark.parametrize("first", [256, 4])
+def test_phase_counters_belong_to_their_system(first):
+    """Row s of the phase counters (builds with QX_PHASE_TIMING) is system s
+    of the batch, in a launch that takes the systems by size and in one launch
+    per run of systems of one bin."""
+    mols = [(np.array([1, 1], np.int32), np.array([[0.0, 0.0, 0.0], [0.0, 0.0, 1.5]])), molecule(6)]
+    off = np.cumsum([0] + [len(n) for n, _ in mols]).astype(np.int32)
+    raw = eb.part("phase", np.array([len(mols), first], np.int32), off,
+                  np.concatenate([n for n, _ in mols]).astype(np.int32), np.concatenate([x for _, x in mols]))
+    iters, counted = np.frombuffer(raw, np.int32).reshape(-1, 2).T
+    assert iters[0] != iters[1]
+    assert np.array_equal(iters, counted)
