@@ -560,10 +560,13 @@ QX_DEV void jacobi_replay(const JacobiBuffers& jb, double* Cv, int m, int nrow, 
     const int s0 = (lane & (NL - 1)) * NS;
     const bool first = s0 == 0;
     for (int i0 = 0; i0 < nrow; i0 += NG * NW * NR) {
+        // lanes without a row read the wavefront's first one
+        const int own = i0 + NG * wave;
+        if (own >= nrow) break;
         double x[NR][NS], y[NR][NS];
 #pragma unroll
         for (int u = 0; u < NR; ++u) {
-            const int row = i0 + NG * (wave + NW * u) + lane / NL, i = row < nrow ? row : nrow - 1;
+            const int row = i0 + NG * (wave + NW * u) + lane / NL, i = row < nrow ? row : own;
 #pragma unroll
             for (int t = 0; t < NS; ++t) {
                 const int k = s0 + t < half ? s0 + t : half - 1;

@@ -222,7 +222,7 @@ QX_DEV void factor_global(const double* S, double* Lg, double* Xg, int n, int ld
     for (int j = 0; j < n - 1; ++j) {
         const double inv = 1.0 / a[j * ld + j];
         for (int i0 = j + 1; i0 < n; i0 += 64) {
-            const int i = i0 + lane, ir = i < n ? i : n - 1;
+            const int i = i0 + lane, ir = i < n ? i : j;  // (row j is not written)
             const double l = a[j * ld + ir] * inv;
             // columns 0 .. j of the inverse, j + 1 .. of S down to the diagonal
             const int qe = i0 + 64 < n ? i0 + 64 : n;

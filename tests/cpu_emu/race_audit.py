@@ -54,6 +54,7 @@ def summarize(logdir):
 def main():
     ap = argparse.ArgumentParser()
     ap.add_argument("--out", default=os.path.join(HERE, "_build", "race_audit"))
+    ap.add_argument("--only", default="", help="cases whose name starts with this")
     args = ap.parse_args()
     subprocess.run(["make", "-s", "-C", HERE, "tsan"], check=True)
     eb.EMU_BIN = os.path.join(HERE, "_build", "egrad_emu_tsan")
@@ -70,13 +71,16 @@ def main():
     small = np.diag(np.linspace(-1.0, 1.0, 58)) + 2e-5
     small[3, 4] = small[4, 3] = 0.05
     spd = np.eye(66) + np.ones((66, 66)) / 66
-    cases.append(("setup", "part", lambda: eb.part("setup", np.array([len(num)], np.int32), num.astype(np.int32), xyz)))
+    cases.append(("setup", "part", lambda num=num, xyz=xyz: eb.part(
+        "setup", np.array([len(num)], np.int32), num.astype(np.int32), xyz)))
     cases += [(f"jacobi {n} form {form}", "part", lambda n=n, form=form: parts.eig(parts.dense(n), form, maxsweep=1))
               for n, form in ((33, 2), (58, 1), (66, 1), (104, 1), (66, 0))]
     cases += [(f"refinement form {form}", "part", lambda form=form: parts.eig(small, form, refine=1)) for form in (1, 0)]
     cases += [(f"broyden {st}", "part", lambda st=st: eb.part("broyden", np.array([66, st], np.int32), spd, np.ones(66)))
               for st in (0, 100)]
     for name, kind, arg in cases:
+        if not name.startswith(args.only):
+            continue
         d = os.path.join(args.out, name.replace(" ", "_"))
         os.makedirs(d, exist_ok=True)
         for f in glob.glob(os.path.join(d, "tsan.*")):
