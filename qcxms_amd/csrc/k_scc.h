@@ -48,30 +48,7 @@ __device__ unsigned long long g_phase[kPhaseSys * kPhaseSlots];
     do {                                                                           \
         if (threadIdx.x == 0 && (sys) < kPhaseSys) g_phase[(sys) * kPhaseSlots + (k)] += (v); \
     } while (0)
-#define QX_PT_INIT(tv) unsigned long long tv = clock64(), tv##_acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-#define QX_PT(k, tv)                                                               \
-    do {                                                                           \
-        const unsigned long long t_ = clock64();                                   \
-        tv##_acc[(k) & 7] += t_ - tv;                                              \
-        tv = t_;                                                                   \
-    } while (0)
-#define QX_PT_COUNT(tv, k) (tv##_acc[(k)&7] += 1)
-#define QX_PT_FLUSH(tv)                                                            \
-    do {                                                                           \
-        if (threadIdx.x == 0 && blockIdx.x < kPhaseSys)                            \
-            for (int k_ = 0; k_ < 8; ++k_) g_phase[blockIdx.x * kPhaseSlots + 16 + k_] += tv##_acc[k_]; \
-    } while (0)
 #else
-#define QX_PT_INIT(tv)
-#define QX_PT(k, tv) \
-    do {             \
-    } while (0)
-#define QX_PT_FLUSH(tv) \
-    do {                \
-    } while (0)
-#define QX_PT_COUNT(tv, k) \
-    do {                   \
-    } while (0)
 #define QX_PH_INIT
 #define QX_PH(sys, k) \
     do {              \
@@ -999,7 +976,7 @@ struct SysShared {
     int eroff[gfn2::kElem + 1];            // D4 references of the elements present: [off[e], off[e+1])
     double sx[3 * QX_MAX_NAT];
     double mrad[QX_MAX_NAT];
-    double qat[QX_MAX_NAT], vat[QX_MAX_NAT];
+    double qat[QX_MAX_NAT];
     // D4 references inside potentials(); between its calls the same LDS holds
     // the Jacobi rotations, its round flags and the Broyden weights
     union {

@@ -22,13 +22,6 @@ QX_DEV double d4_zeta(double a, double c, double qref, double qmod)
     if (qmod < 0.0) return exp(a);
     return exp(a * (1.0 - exp(c * (1.0 - qref / qmod))));
 }
-QX_DEV double d4_dzeta(double a, double c, double qref, double qmod)
-{
-    if (qmod < 0.0) return 0.0;
-    const double e = exp(c * (1.0 - qref / qmod));
-    return -a * c * e * exp(a * (1.0 - e)) * qref / (qmod * qmod);
-}
-
 // both at once
 QX_DEV void d4_zeta_both(double a, double c, double qref, double qmod, double& z, double& dz)
 {
