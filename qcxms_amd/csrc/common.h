@@ -227,8 +227,10 @@ struct SccOpts {
 struct BatchPtrs {
     int nsys;
     const SysInfo* info;
-    const int* order; // systems by decreasing basis size: workgroup k of a launch over all takes
-                      // order[k], so the longest run first and the short ones fill the end
+    const int* order; // systems by decreasing basis size: workgroup k of a setup, SCC, gradient or
+                      // persistent MD launch over all takes order[k], so the longest run first
+                      // and the short ones fill the end (launches over a range and k_dblocks
+                      // keep the batch's order)
                       // (6 MD steps of 512 chains of 2 .. 11 heavy atoms: 28.9 -> 21.5 ms)
     const int* elem;  // per atom: element slot
     double* xyz;      // 3 per atom

@@ -298,8 +298,8 @@ QX_DEV double2 pivot_rotation(double app, double aqq, double apq, double tol, do
 // Blocks per thread that the rounds with the blocks in LDS take (up to 132
 // basis functions); above, the rounds work on global memory.  The LDS would
 // hold the blocks of 172 functions, but a thread keeps its blocks in registers
-// between the barriers.  (Six blocks: 136 functions 60.9 -> 36.1 ms and 144:
-// 75.3 -> 39.5 ms, single rings of carbon, but 132: 33.3 -> 33.7 ms; as a
+// between the barriers.  (Six blocks: 136 functions 57.9 -> 36.1 ms and 144:
+// 72.6 -> 39.5 ms, single rings of carbon, but 132: 33.3 -> 33.7 ms; as a
 // further instantiation 104 to 132 functions take 0.5 % longer and the kernel
 // spills 112 instead of 57 vector registers.)
 constexpr int kMaxNB = 5;
@@ -524,8 +524,10 @@ QX_DEV void jacobi_rounds_global(const JacobiBuffers& jb, int m, double tol, dou
 // pair slots of its row in registers, the players as in jacobi_rounds (x the p and y
 // the q players, in slot 0 the other way round), so that in the move after a
 // round only one player of x and one of y change the lane and the others the
-// register.  NR such sets of rows at a time.  Without LDS traffic or barriers a
-// round is bound by the instructions issued.
+// register.  NR such sets of rows at a time.  Without barriers, and with one LDS
+// read (whether the round rotates anything), a round is bound by the
+// instructions issued.  More than one pair (m > 2: smaller systems have their
+// rows in registers).
 // (Cycles a round with one row per wavefront and slots 64 apart -> now: 132
 // rows and columns 6.0 k -> 2.9 k, where the second set had used 2 lanes of 64;
 // 88: 1.75 k -> 1.50 k.)
@@ -1000,8 +1002,8 @@ inline __host__ __device__ int pot_lds(int nat)
 }
 
 // What a thread needs from the parameter tables in every call: of its D4
-// reference (threads 4 k .. 4 k + 3 of the first pass: reference k), its
-// shell's Coulomb row and its atom's on-site multipole kernels.
+// reference (thread k: reference k), its shell's Coulomb row (from the last
+// thread on) and its atom's on-site multipole kernels.
 struct PotTables {
     double c, qref, zeff, gw, third, dk, qk;
 

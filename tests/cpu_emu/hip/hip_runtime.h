@@ -351,9 +351,8 @@ inline hipError_t hipDeviceGetAttribute(int* v, hipDeviceAttribute_t, int)
     return hipSuccess;
 }
 // Static LDS per kernel: the emulation keeps every kernel's __shared__
-// objects in one section, so it reports the MI355X build's figure for the
-// largest kernels (46,480 bytes for the SCC and persistent MD kernels),
-// rounded up.
+// objects in one section, so it reports a figure above the MI355X build's for
+// the largest kernels (43,616 bytes for the persistent MD kernel).
 struct hipFuncAttributes {
     size_t sharedSizeBytes;
 };
