@@ -14,9 +14,14 @@
 // library that the Python package and the C ABI load.
 #pragma once
 
+#include <linux/futex.h>
+#include <sched.h>
+#include <sys/syscall.h>
+#include <unistd.h>
+
+#include <atomic>
 #include <chrono>
 #include <cmath>
-#include <condition_variable>
 #include <cstdint>
 #include <cstdio>
 #include <cstdlib>
@@ -81,6 +86,7 @@ namespace qx_emu {
 constexpr int kMaxThreads = 1024;
 constexpr size_t kMaxLds = 160 * 1024;
 constexpr int kTimeoutSeconds = 300;
+constexpr int kYields = 1000;
 
 // Barrier whose participant count can shrink while it is in use.  A block
 // barrier also checks that every thread of one barrier generation arrives
@@ -90,9 +96,8 @@ constexpr int kTimeoutSeconds = 300;
 // anywhere) and which can desynchronise the waves or hang them.
 struct Barrier {
     std::mutex m;
-    std::condition_variable cv;
+    std::atomic<unsigned> gen{0};
     int expected = 0, arrived = 0;
-    unsigned long gen = 0;
     const char* site_file = nullptr;
     int site_line = 0;
     unsigned site_thread = 0;
@@ -102,44 +107,60 @@ struct Barrier {
         expected = n;
         arrived = 0;
     }
+    // the waiting threads give way to those that have yet to arrive (waking a
+    // block of sleeping threads takes longer than most rounds), and sleep on
+    // the generation (a futex) when that takes long
     void wait(const char* what, const char* file = nullptr, int line = 0)
     {
-        std::unique_lock<std::mutex> l(m);
-        const unsigned long g = gen;
-        if (file) {
-            if (arrived == 0) {
-                site_file = file;
-                site_line = line;
-                site_thread = threadIdx.x;
-            } else if (line != site_line || std::strcmp(file, site_file) != 0) {
-                std::fprintf(stderr,
-                             "cpu emulation: divergent %s barrier (block %u): thread %u at %s:%d, "
-                             "thread %u at %s:%d\n",
-                             what, blockIdx.x, site_thread, site_file, site_line, threadIdx.x, file, line);
-                std::abort();
+        unsigned g;
+        {
+            std::lock_guard<std::mutex> l(m);
+            g = gen.load(std::memory_order_relaxed);
+            if (file) {
+                if (arrived == 0) {
+                    site_file = file;
+                    site_line = line;
+                    site_thread = threadIdx.x;
+                } else if (line != site_line || std::strcmp(file, site_file) != 0) {
+                    std::fprintf(stderr,
+                                 "cpu emulation: divergent %s barrier (block %u): thread %u at %s:%d, "
+                                 "thread %u at %s:%d\n",
+                                 what, blockIdx.x, site_thread, site_file, site_line, threadIdx.x, file, line);
+                    std::abort();
+                }
+            }
+            if (++arrived == expected) {
+                finish();
+                return;
             }
         }
-        if (++arrived == expected) {
-            arrived = 0;
-            ++gen;
-            cv.notify_all();
-            return;
+        for (int k = 0; k < kYields; ++k) {
+            if (gen.load(std::memory_order_acquire) != g) return;
+            sched_yield();
         }
-        if (!cv.wait_for(l, std::chrono::seconds(kTimeoutSeconds), [&] { return gen != g; })) {
-            std::fprintf(stderr, "cpu emulation: %s barrier not reached by all threads (block %u thread %u, %d of %d)\n",
-                         what, blockIdx.x, threadIdx.x, arrived, expected);
-            std::abort();
+        const auto end = std::chrono::steady_clock::now() + std::chrono::seconds(kTimeoutSeconds);
+        while (gen.load(std::memory_order_acquire) == g) {
+            const timespec t{kTimeoutSeconds, 0};
+            syscall(SYS_futex, &gen, FUTEX_WAIT_PRIVATE, g, &t, nullptr, 0);
+            if (gen.load(std::memory_order_acquire) == g && std::chrono::steady_clock::now() > end) {
+                std::fprintf(stderr,
+                             "cpu emulation: %s barrier not reached by all threads (block %u thread %u, %d of %d)\n",
+                             what, blockIdx.x, threadIdx.x, arrived, expected);
+                std::abort();
+            }
         }
     }
     void drop()
     {
         std::lock_guard<std::mutex> l(m);
         --expected;
-        if (arrived > 0 && arrived == expected) {
-            arrived = 0;
-            ++gen;
-            cv.notify_all();
-        }
+        if (arrived > 0 && arrived == expected) finish();
+    }
+    void finish()
+    {
+        arrived = 0;
+        gen.fetch_add(1, std::memory_order_acq_rel);
+        syscall(SYS_futex, &gen, FUTEX_WAKE_PRIVATE, INT32_MAX, nullptr, nullptr, 0);
     }
 };
 
