@@ -1,10 +1,12 @@
 """Single parts of the kernels and the launch sizes in the CPU emulation
 (tests/cpu_emu/parts_emu.cpp: bounds-checked, LDS filled with NaN bytes), at
-the sizes where they change their path."""
+the sizes where they change their path, and whole systems above 64 basis
+functions."""
 import numpy as np
 import pytest
 
 import emu_bind as eb
+import oracle_bind as ob
 from qcxms_amd import workloads as W
 
 
@@ -178,3 +180,19 @@ def test_phase_counters_belong_to_their_system(first):
     iters, counted = np.frombuffer(raw, np.int32).reshape(-1, 2).T
     assert iters[0] != iters[1]
     assert np.array_equal(iters, counted)
+
+
+@pytest.mark.timeout(900)
+def test_emulated_large_systems_match_the_oracle():
+    """Systems of 66, 104 and 134 basis functions in one launch with the
+    eigenvector refinement, at the bars of the GPU parity tests."""
+    eb.build()
+    mols = [molecule(n) for n in (66, 104, 134)]
+    systems, coords = [(num, 1) for num, _ in mols], [xyz for _, xyz in mols]
+    rc, e, g, q, st, err = eb.egrad_batch(systems, coords, 5000.0, tuning=[(256, 1, 1)])
+    assert rc == 0 and np.all(st == 0), err
+    re, rg, rq, rst = ob.gfn2_egrad_batch(systems, coords, 5000.0, opts=ob.default_opts(econv=1e-12, pconv=1e-10))
+    assert np.all(rst == 0)
+    assert np.abs(e - re).max() <= 1e-8
+    assert max(np.abs(a - b).max() for a, b in zip(g, rg)) <= 1e-6
+    assert max(np.abs(a - b).max() for a, b in zip(q, rq)) <= 1e-6
